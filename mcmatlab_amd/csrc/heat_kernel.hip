@@ -10,12 +10,12 @@
 //   y sweep   substeps 2a + 2b: the -dt/2 L_y correction and the y solve;
 //   z sweep   substeps 3a + 3b: the -dt/2 L_z correction, the z solve, the
 //             Arrhenius damage update and the per-medium maximum temperature.
-// FP64 (default), lines of up to 512 voxels: each line is solved by one
-// wavefront (partition method + parallel cyclic reduction across the 64
-// lanes); the x sweep reads its lines directly (contiguous), the y and z
-// sweeps stage tiles of lines through LDS.  FP32 (the reference's arithmetic)
-// and longer lines: one lane per line running the Thomas recurrence over
-// blocks of loaded elements.
+// FP64 (default), lines of up to 512 voxels: the sweeps solve for increments
+// (below) by a partition method with parallel cyclic reduction between the
+// chunks of a line; along x a wavefront holds contiguous voxels, along y and z
+// a workgroup holds 16 neighbouring lines in registers.  FP32 (the reference's
+// arithmetic) and longer lines: one lane per line running the Thomas
+// recurrence over blocks of loaded elements.
 // The explicit (forward Euler) scheme is one kernel per step.
 //
 // Arithmetic follows the reference's expressions (built without FMA
@@ -117,12 +117,22 @@ __device__ inline RT cc(const HeatArgs<RT>& a, int m, int n, int d) {
   return a.c[m + n * a.nM + d * a.nM * a.nM];
 }
 
+// Running maxima per medium.  The keys in LDS start from the global running
+// maxima, so a voxel that does not raise its medium's maximum touches no
+// atomic (a stale start is harmless: the keys only grow), and a workgroup
+// writes back only what it raised.  Starting every workgroup from -inf cost
+// one LDS atomic per lane and one same-address global atomic per workgroup,
+// medium and step.
 struct MaxRun {
   int m = -1;
   double v = -INFINITY;
+  __device__ static void raise(unsigned long long* s, int m, double v) {
+    const unsigned long long k = order_key(v);
+    if (k > *(volatile unsigned long long*)&s[m]) atomicMax(&s[m], k);
+  }
   __device__ void add(int mm, double t, unsigned long long* s) {
     if (mm != m) {
-      if (m >= 0) atomicMax(&s[m], order_key(v));
+      if (m >= 0) raise(s, m, v);
       m = mm;
       v = t;
     } else if (t > v) {
@@ -130,20 +140,15 @@ struct MaxRun {
     }
   }
   __device__ void flush(unsigned long long* s) {
-    if (m >= 0) atomicMax(&s[m], order_key(v));
+    if (m >= 0) raise(s, m, v);
     m = -1;
   }
 };
 
-__device__ inline void init_lds_max(unsigned long long* s, int nM) {
-  for (int k = threadIdx.x; k < nM; k += blockDim.x) s[k] = order_key(-INFINITY);
-  __syncthreads();
-}
 __device__ inline void fold_lds_max(unsigned long long* s, unsigned long long* g, int nM) {
   __syncthreads();
-  const unsigned long long none = order_key(-INFINITY);
   for (int k = threadIdx.x; k < nM; k += blockDim.x)
-    if (s[k] != none) atomicMax(&g[k], s[k]);
+    if (s[k] > g[k]) atomicMax(&g[k], s[k]);
 }
 
 enum : int { SWEEP_X = 0, SWEEP_Y = 1, SWEEP_Z = 2 };
@@ -151,7 +156,7 @@ constexpr int kLdsCoef = 1536;  // coefficient tables up to 22 media live in LDS
 
 template <typename RT>
 __device__ inline RT coef(const RT* c, int nM, int m, int nb, int d) {
-  return c[m + nb * nM + d * nM * nM];
+  return c[d * nM * nM + (int)(__umul24((unsigned)nb, (unsigned)nM) + (unsigned)m)];
 }
 
 // Per-workgroup copies of the small per-medium tables.
@@ -171,7 +176,7 @@ __device__ inline const RT* stage_tables(const HeatArgs<RT>& a, HeatLds<RT>& s) 
   for (int k = threadIdx.x; k < a.nM; k += blockDim.x) {
     s.logA[k] = a.logA[k];
     s.E[k] = a.E[k];
-    s.maxKey[k] = order_key(-INFINITY);
+    s.maxKey[k] = a.maxKey[k];
   }
   __syncthreads();
   return nc <= kLdsCoef ? s.c : a.c;
@@ -191,6 +196,7 @@ __device__ inline const RT* stage_tables(const HeatArgs<RT>& a, HeatLds<RT>& s) 
 template <typename RT, int KIND, int U>
 __device__ void sweep_line(const HeatArgs<RT>& a, const RT* cT, const HeatLds<RT>& L, int i0, int st, int n, bool lf, int d, int s1,
                            int k1, int n1, int s2, int k2, int n2, MaxRun* run, unsigned long long* sMax) {
+  constexpr bool kIncrement = std::is_same<RT, double>::value;  // FP64 sweeps solve for increments (see below)
   const int nM = a.nM;
   const RT dt = a.dt;
   const bool sk = a.sinked;
@@ -241,17 +247,17 @@ __device__ void sweep_line(const HeatArgs<RT>& a, const RT* cT, const HeatLds<RT
         RT dTdt = 0;
         if (!fz) {
           dTdt = a.lightsOn ? (RT)Qv[u] : (RT)0;
-          if (k != 0) dTdt += (Tw[u] - Tw[u + 1]) * coef(cT, nM, m, Mw[u], 0) / 2;
-          if (k != n - 1) dTdt += (Tw[u + 2] - Tw[u + 1]) * coef(cT, nM, m, Mw[u + 2], 0) / 2;
+          if (k != 0) dTdt += (Tw[u] - Tw[u + 1]) * coef(cT, nM, m, Mw[u], 0) / (kIncrement ? 1 : 2);
+          if (k != n - 1) dTdt += (Tw[u + 2] - Tw[u + 1]) * coef(cT, nM, m, Mw[u + 2], 0) / (kIncrement ? 1 : 2);
           if (k1 != 0) dTdt += (Ta[u] - Tw[u + 1]) * coef(cT, nM, m, Ma[u], 1);
           if (k1 != n1 - 1) dTdt += (Tb[u] - Tw[u + 1]) * coef(cT, nM, m, Mb[u], 1);
           if (k2 != 0) dTdt += (Tc[u] - Tw[u + 1]) * coef(cT, nM, m, Mc[u], 2);
           if (k2 != n2 - 1) dTdt += (Td[u] - Tw[u + 1]) * coef(cT, nM, m, Md[u], 2);
         }
-        t = Tw[u + 1] + dt * dTdt;
+        t = kIncrement ? dt * dTdt : Tw[u + 1] + dt * dTdt;
       } else {
         t = R0[u];
-        if (!fz) {
+        if (!kIncrement && !fz) {
           RT dTdt = 0;
           if (k != 0) dTdt -= (Tw[u] - Tw[u + 1]) * coef(cT, nM, m, Mw[u], d) / 2;
           if (k != n - 1) dTdt -= (Tw[u + 2] - Tw[u + 1]) * coef(cT, nM, m, Mw[u + 2], d) / 2;
@@ -307,6 +313,10 @@ __device__ void sweep_line(const HeatArgs<RT>& a, const RT* cT, const HeatLds<RT
       }
       xnext = t;
       if (KIND == SWEEP_Z) {
+        if (kIncrement) {
+          t = T1v[u] + t;
+          a.T2[i] = t;
+        }
         if (a.calcDamage && L.E[m] != 0) a.Om[i] = Omv[u] + dt * (RT)exp(L.logA[m] - L.E[m] / (a.Rgas * ((t + T1v[u]) / 2 + a.czero)));
         run->add(m, (double)t, sMax);
       }
@@ -370,14 +380,21 @@ __global__ void __launch_bounds__(kHeatTPB) heat_sweep_z(HeatArgs<RT> a) {
 // 64 / W systems side by side), S consecutive rows per lane (row
 // r = lane * S + s, lane counted within the segment); unused rows are
 // a = c = 0, b = 1, d = 0.  The matrices of the heat step are strictly
-// diagonally dominant, so no pivoting is needed.  Partition method:
-//   1. each lane eliminates its interior rows 1..S-2, expressing them through
-//      its own first and last unknowns;
-//   2. the first unknown of each lane is eliminated as well, leaving one
-//      tridiagonal equation per lane in the lanes' last unknowns U;
-//   3. that W-row system is solved by parallel cyclic reduction, log2(W)
-//      steps of lane shuffles that never cross a segment's edge;
-//   4. each lane recovers its first and interior unknowns from U.
+// diagonally dominant, so no pivoting is needed.  With U the lanes' last
+// unknowns and UL the one of the lane before:
+//   1. each lane eliminates downwards and keeps three numbers per row,
+//      x[s] = p[s] - q[s] UL - g[s] x[s+1];
+//   2. its first unknown in terms of UL and U goes to the lane before, which
+//      leaves one tridiagonal equation per lane in U with a unit diagonal;
+//   3. that W-row system is solved by parallel cyclic reduction, at most
+//      log2(W) steps of lane moves that never cross a segment's edge.  The
+//      couplings are products of S off-diagonal/diagonal ratios and square at
+//      every step, so they fall fast: once all of a wavefront's are at most
+//      2^-30, one correction with the neighbours' right-hand sides leaves a
+//      relative error of 2^-60 and the steps end (time steps of up to 1.5
+//      times the explicit limit have ratios of about 0.1: no step at S = 13,
+//      one at S = 8, two at S = 4; larger time steps take more);
+//   4. each lane recovers its unknowns upwards from U and UL.
 // Same solution as the sequential Thomas recurrence up to rounding.
 __device__ inline double lane_shfl(double v, int src) { return __shfl(v, src < 0 ? 0 : (src > 63 ? 63 : src), 64); }
 __device__ inline int lane_shfl(int v, int src) { return __shfl(v, src < 0 ? 0 : (src > 63 ? 63 : src), 64); }
@@ -414,111 +431,110 @@ __device__ inline V seg_shift(V v, int h) {
   return lane_shfl(v, UP ? wl + h : wl - h);
 }
 
-// a / b for the positive, well-scaled pivots of the solver: hardware
-// reciprocal estimate refined by two Newton steps (a few ulp), instead of the
-// correctly rounded division sequence.
-__device__ inline double pdiv(double a, double b) {
+// 1 / b for the well-scaled pivots of the solver: hardware reciprocal estimate
+// refined by two Newton steps (a few ulp), instead of the correctly rounded
+// division sequence.
+__device__ inline double prcp(double b) {
   double r = __builtin_amdgcn_rcp(b);
   r = fma(fma(-b, r, 1.0), r, r);
   r = fma(fma(-b, r, 1.0), r, r);
-  return a * r;
+  return r;
 }
+
+// couplings below this are dropped after one correction step (line_solve)
+constexpr double kDecoupled = 0x1p-30;
 
 template <int S, int W = 64>
-__device__ inline void wave_tridiag(const double (&a)[S], const double (&b)[S], const double (&c)[S], const double (&d)[S],
-                                    double (&x)[S]) {
+__device__ inline void line_solve(const double (&a)[S], const double (&b)[S], const double (&c)[S], const double (&d)[S], double (&x)[S]) {
   // a line per W-lane segment of the wavefront; lane is the index within it
   static_assert(W == 16 || W == 32 || W == 64, "segments of 16, 32 or 64 lanes");
-  const int wl = __lane_id(), lane = wl & (W - 1);
-  double al[S], be[S], ga[S], de[S];
-  double A1 = a[0], B1 = b[0], C1 = c[0], D1 = d[0];
-  double A2 = a[S - 1], B2 = b[S - 1], C2 = c[S - 1], D2 = d[S - 1];
-  if constexpr (S >= 3) {
-    // forward elimination of the interior, first unknown kept symbolic
-    al[1] = a[1];
-    be[1] = b[1];
-    ga[1] = c[1];
-    de[1] = d[1];
-#pragma unroll
-    for (int s = 2; s <= S - 2; ++s) {
-      const double r = pdiv(a[s], be[s - 1]);
-      al[s] = -r * al[s - 1];
-      be[s] = b[s] - r * ga[s - 1];
-      ga[s] = c[s];
-      de[s] = d[s] - r * de[s - 1];
-    }
-    // backward elimination, last unknown kept symbolic
-#pragma unroll
-    for (int s = S - 3; s >= 1; --s) {
-      const double r = pdiv(ga[s], be[s + 1]);
-      al[s] -= r * al[s + 1];
-      ga[s] = -r * ga[s + 1];
-      de[s] -= r * de[s + 1];
-    }
-    const double r1 = pdiv(c[0], be[1]);
-    B1 = b[0] - r1 * al[1];
-    C1 = -r1 * ga[1];
-    D1 = d[0] - r1 * de[1];
-    const double r2 = pdiv(a[S - 1], be[S - 2]);
-    A2 = -r2 * al[S - 2];
-    B2 = b[S - 1] - r2 * ga[S - 2];
-    D2 = d[S - 1] - r2 * de[S - 2];
+  const int lane = __lane_id() & (W - 1);
+  // 1: x[s] = p[s] - q[s] UL - g[s] x[s+1]
+  double g[S], p[S], q[S];
+  {
+    const double r = prcp(b[0]);
+    g[0] = c[0] * r;
+    p[0] = d[0] * r;
+    q[0] = a[0] * r;
   }
-  // one equation per lane in U = last unknowns:  pa U[l-1] + pb U[l] + pc U[l+1] = pd
-  double pa, pb, pc, pd;
-  if constexpr (S == 1) {
-    pa = A1;
-    pb = B1;
-    pc = C1;
-    pd = D1;
-  } else {
-    // shuffles run in every lane (a lane reading from a lane that is
-    // inactive at the shuffle gets 0), then the edge lanes are masked
-    const bool hasNext = lane < W - 1;
-    const double sA = seg_shift<W, true>(A1, 1), sB = seg_shift<W, true>(B1, 1);
-    const double sC = seg_shift<W, true>(C1, 1), sD = seg_shift<W, true>(D1, 1);
-    const double nA = hasNext ? sA : 0.0, nB = hasNext ? sB : 1.0, nC = hasNext ? sC : 0.0, nD = hasNext ? sD : 0.0;
-    const double iB1 = pdiv(1.0, B1), inB = pdiv(1.0, nB);
-    pa = -A2 * A1 * iB1;
-    pb = B2 - A2 * C1 * iB1 - C2 * nA * inB;
-    pc = -C2 * nC * inB;
-    pd = D2 - A2 * D1 * iB1 - C2 * nD * inB;
+#pragma unroll
+  for (int s = 1; s < S; ++s) {
+    const double r = prcp(fma(-a[s], g[s - 1], b[s]));
+    g[s] = c[s] * r;
+    p[s] = fma(-a[s], p[s - 1], d[s]) * r;
+    q[s] = -a[s] * q[s - 1] * r;
   }
+  // 2: x[0] = P - Q UL + R U
+  double P = 0.0, Q = 0.0, R = 1.0;
+#pragma unroll
+  for (int s = S - 2; s >= 0; --s) {
+    P = fma(-g[s], P, p[s]);
+    Q = fma(-g[s], Q, q[s]);
+    R = -g[s] * R;
+  }
+  // shuffles run in every lane (a lane reading from a lane that is inactive
+  // at the shuffle gets 0), then lanes without the neighbour are masked; DPP
+  // moves deliver 0 there by themselves
+  double Pn = seg_shift<W, true>(P, 1), Qn = seg_shift<W, true>(Q, 1), Rn = seg_shift<W, true>(R, 1);
+  if (W != 16 && lane == W - 1) Pn = Qn = Rn = 0.0;
+  const double e = g[S - 1], ib = prcp(fma(-e, Qn, 1.0));
+  double pa = q[S - 1] * ib, pc = e * Rn * ib, pd = fma(-e, Pn, p[S - 1]) * ib;
+  // 3: U + pa U(lane - h) + pc U(lane + h) = pd
+  double U = pd;
 #pragma unroll
   for (int h = 1; h < W; h <<= 1) {
-    const bool lo = lane >= h, hi = lane + h < W;
-    const double sam = seg_shift<W, false>(pa, h), sbm = seg_shift<W, false>(pb, h);
-    const double scm = seg_shift<W, false>(pc, h), sdm = seg_shift<W, false>(pd, h);
-    const double sap = seg_shift<W, true>(pa, h), sbp = seg_shift<W, true>(pb, h);
-    const double scp = seg_shift<W, true>(pc, h), sdp = seg_shift<W, true>(pd, h);
-    const double am = lo ? sam : 0.0, bm = lo ? sbm : 1.0, cm = lo ? scm : 0.0, dm = lo ? sdm : 0.0;
-    const double ap = hi ? sap : 0.0, bp = hi ? sbp : 1.0, cp = hi ? scp : 0.0, dp = hi ? sdp : 0.0;
-    const double k1 = pdiv(pa, bm), k2 = pdiv(pc, bp);
-    pb = pb - k1 * cm - k2 * ap;
-    pd = pd - k1 * dm - k2 * dp;
-    pa = -k1 * am;
-    pc = -k2 * cp;
-  }
-  const double U = pdiv(pd, pb);
-  if constexpr (S == 1) {
-    x[0] = U;
-  } else {
-    const double sU = seg_shift<W, false>(U, 1);
-    const double Up = lane > 0 ? sU : 0.0;
-    const double first = pdiv(D1 - A1 * Up - C1 * U, B1);
-    x[0] = first;
-    x[S - 1] = U;
-    if constexpr (S >= 3) {
-#pragma unroll
-      for (int s = 1; s <= S - 2; ++s) x[s] = pdiv(de[s] - al[s] * first - ga[s] * U, be[s]);
+    double dm = seg_shift<W, false>(pd, h), dp = seg_shift<W, true>(pd, h);
+    if (W != 16) {
+      dm = lane >= h ? dm : 0.0;
+      dp = lane + h < W ? dp : 0.0;
     }
+    if (__all(fmax(fabs(pa), fabs(pc)) <= kDecoupled)) {
+      pd = fma(-pc, dp, fma(-pa, dm, pd));
+      break;
+    }
+    double am = seg_shift<W, false>(pa, h), cm = seg_shift<W, false>(pc, h);
+    double ap = seg_shift<W, true>(pa, h), cp = seg_shift<W, true>(pc, h);
+    if (W != 16) {
+      am = lane >= h ? am : 0.0;
+      cm = lane >= h ? cm : 0.0;
+      ap = lane + h < W ? ap : 0.0;
+      cp = lane + h < W ? cp : 0.0;
+    }
+    const double r = prcp(fma(-pc, ap, fma(-pa, cm, 1.0)));
+    pd = fma(-pc, dp, fma(-pa, dm, pd)) * r;
+    pa = -pa * am * r;
+    pc = -pc * cp * r;
   }
+  U = pd;
+  // 4
+  double UL = seg_shift<W, false>(U, 1);
+  if (W != 16 && lane == 0) UL = 0.0;
+  x[S - 1] = U;
+#pragma unroll
+  for (int s = S - 2; s >= 0; --s) x[s] = fma(-g[s], x[s + 1], fma(-q[s], UL, p[s]));
 }
 
-// substeps 1a + 1b in FP64 with one wavefront per (y, z) x-line: lane l holds
-// voxels x = l*S .. l*S+S-1, so every load of the wavefront is contiguous.
-// The right-hand side is the full 7-point explicit stencil (x half-weighted)
-// plus the source, in the expression order of the sequential kernel.
+// The FP64 sweeps work on increments: with u the temperature at the start of
+// the step, A_d = I - dt/2 L_d and L = L_x + L_y + L_z,
+//   A_x dx = dt (L u + Q),  A_y dy = dx,  A_z dz = dy,  T = u + dz
+// is the Douglas-Gunn step written for T1 - u, T2 - u and T3 - u instead of
+// the substeps' temperatures T1, T2, T3 (A_y (T2 - u) = T1 - dt/2 L_y u - A_y u
+// = T1 - u, and likewise along z).  The y and z sweeps then need neither u's
+// stencil nor u itself before the end, and rounding enters relative to the
+// increment.  Frozen voxels have increment 0.
+
+// Workgroup b of n, renumbered so that each of the 8 XCDs (which take
+// workgroups in turn) works on consecutive ones and finds its neighbours'
+// data in its own L2.
+__device__ inline int xcd_contiguous(int b, int n) {
+  const int q = n >> 3, r = n & 7, x = b & 7;
+  return x * q + min(x, r) + (b >> 3);
+}
+
+// substeps 1a + 1b in FP64, a (y, z) x-line per W lanes: lane l holds voxels
+// x = l*S .. l*S+S-1, so every load of the wavefront is contiguous.  Bound by
+// instruction issue (52 us at 200^3; 75 us with all six reduction steps and
+// workgroups dealt to the XCDs in turn).
 template <int S, int W, bool LDS_COEF>
 __global__ void __launch_bounds__(kHeatTPB) heat_sweep_x_wave(HeatArgs<double> a) {
   // the coefficient table in LDS when it fits (LDS_COEF), else read from
@@ -535,7 +551,7 @@ __global__ void __launch_bounds__(kHeatTPB) heat_sweep_x_wave(HeatArgs<double> a
   // a line per W-lane segment; a segment past the last line solves the
   // last line again and stores nothing
   const int wl = __lane_id(), lane = wl & (W - 1);
-  const int line = (blockIdx.x * (kHeatTPB / 64) + (threadIdx.x >> 6)) * (64 / W) + wl / W;
+  const int line = (xcd_contiguous(blockIdx.x, gridDim.x) * (kHeatTPB / 64) + (threadIdx.x >> 6)) * (64 / W) + wl / W;
   const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = nx * ny, nM = a.nM;
   const bool valid = line < ny * nz;
   const int y = (valid ? line : ny * nz - 1) % ny, z = (valid ? line : ny * nz - 1) / ny;
@@ -605,42 +621,34 @@ __global__ void __launch_bounds__(kHeatTPB) heat_sweep_x_wave(HeatArgs<double> a
   const double Tl = seg_shift<W, false>(T[S - 1], 1), Tr = seg_shift<W, true>(T[0], 1);
   const int Ml = seg_shift<W, false>(Mv[S - 1], 1), Mr = seg_shift<W, true>(Mv[0], 1);
   double ca[S], cb[S], cc_[S], cd[S], xs[S];
+  const double h = dt / 2;
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const int k = lane * S + s;
-    ca[s] = 0.0;
-    cb[s] = 1.0;
-    cc_[s] = 0.0;
-    cd[s] = 0.0;
-    if (k >= nx) continue;
     const int m = Mv[s];
     const double TL = s > 0 ? T[s - 1] : Tl, TR = s < S - 1 ? T[s + 1] : Tr;
     const int ML = s > 0 ? Mv[s - 1] : Ml, MR = s < S - 1 ? Mv[s + 1] : Mr;
-    const bool fz = lf || (sk && (k == 0 || k == nx - 1));
-    if (fz) {
-      cd[s] = T[s];
-      continue;
-    }
+    // Every lookup is done and unwanted ones dropped by selects (no branch).
+    // Neighbours outside the grid: along y and z the clamped addresses above
+    // read the voxel itself, whose difference is 0; along x the coefficient
+    // is made 0 (and the difference finite).
+    const bool on = k < nx && !lf && !(sk && (k == 0 || k == nx - 1));
+    const bool hasL = on && k > 0, hasR = on && k < nx - 1;
+    const double cL = coef(cT, nM, m, ML, 0), cR = coef(cT, nM, m, MR, 0);
+    const double cl = hasL ? cL : 0.0, cr = hasR ? cR : 0.0;
     double dTdt = a.lightsOn ? (double)Qv[s] : 0.0;
-    if (k != 0) dTdt += (TL - T[s]) * coef(cT, nM, m, ML, 0) / 2;
-    if (k != nx - 1) dTdt += (TR - T[s]) * coef(cT, nM, m, MR, 0) / 2;
-    if (y != 0) dTdt += (Tym[s] - T[s]) * coef(cT, nM, m, Mym[s], 1);
-    if (y != ny - 1) dTdt += (Typ[s] - T[s]) * coef(cT, nM, m, Myp[s], 1);
-    if (z != 0) dTdt += (Tzm[s] - T[s]) * coef(cT, nM, m, Mzm[s], 2);
-    if (z != nz - 1) dTdt += (Tzp[s] - T[s]) * coef(cT, nM, m, Mzp[s], 2);
-    cd[s] = T[s] + dt * dTdt;
-    if (k < nx - 1) {
-      const double q = dt / 2 * coef(cT, nM, m, MR, 0);
-      cb[s] += q;
-      cc_[s] = -q;
-    }
-    if (k > 0) {
-      const double q = dt / 2 * coef(cT, nM, m, ML, 0);
-      cb[s] += q;
-      ca[s] = -q;
-    }
+    dTdt = fma(hasL ? TL - T[s] : 0.0, cl, dTdt);
+    dTdt = fma(hasR ? TR - T[s] : 0.0, cr, dTdt);
+    dTdt = fma(Tym[s] - T[s], coef(cT, nM, m, Mym[s], 1), dTdt);
+    dTdt = fma(Typ[s] - T[s], coef(cT, nM, m, Myp[s], 1), dTdt);
+    dTdt = fma(Tzm[s] - T[s], coef(cT, nM, m, Mzm[s], 2), dTdt);
+    dTdt = fma(Tzp[s] - T[s], coef(cT, nM, m, Mzp[s], 2), dTdt);
+    cd[s] = on ? dt * dTdt : 0.0;
+    ca[s] = -h * cl;
+    cc_[s] = -h * cr;
+    cb[s] = fma(h, cl + cr, 1.0);
   }
-  wave_tridiag<S, W>(ca, cb, cc_, cd, xs);
+  line_solve<S, W>(ca, cb, cc_, cd, xs);
   double* __restrict__ T2 = a.T2;
   if (!valid) return;
   if (vec) {
@@ -655,225 +663,247 @@ __global__ void __launch_bounds__(kHeatTPB) heat_sweep_x_wave(HeatArgs<double> a
   }
 }
 
-// substeps 2a + 2b (KIND Y) and 3a + 3b with the Arrhenius update and the
-// per-medium maxima (KIND Z) in FP64, lines staged through LDS: a workgroup
-// takes TX consecutive x-lines at one z (Y) or y (Z), loads them row by row
-// (TX consecutive x per row, coalesced; all of a thread's loads issued before
-// its first LDS store) into LDS with each line contiguous, each wavefront
-// solves TX/4 lines from LDS with the wavefront solver (lane l holds voxels
-// l*S .. l*S+S-1), and the workgroup writes the rows back.  The right-hand
-// side is T1 of the previous substep minus dt/2 L_d T(step start) along the
-// line, in the expression order of the sequential kernel.
-template <int S, int W>
-struct YzTile {
-  static constexpr int NP = W * S;            // padded line length
-  static constexpr int LD = NP + 1;           // LDS pitch of a line (doubles)
-  // lines per workgroup: 16 (128-byte rows) up to 128 voxels a line; longer
-  // lines would need ~70 KB of LDS per workgroup at 16, leaving only two
-  // workgroups per CU, so they take 8
-  static constexpr int TX = NP <= 128 ? 16 : 8;
+// The same solve for lines along y or z by a whole workgroup: 16 neighbouring
+// lines (one cache line of doubles per row of voxels), NC chunks of S voxels
+// each, thread t holding chunk t / 16 of line t % 16 in registers.  Steps 2-4
+// exchange between chunks through LDS, two barriers when the couplings fall
+// below kDecoupled at once (S large enough) and one more per reduction step.
+// Bound by memory: at 200^3 the y sweep moves 136 MB in 24.9 us (5.5 TB/s; a
+// 64 MiB copy reaches 8.1).  Lines staged through LDS tiles, with u's stencil
+// in the y and z sweeps, took 60.9 (y) and 96.4 us (z); four lines per
+// wavefront without LDS 40.2 and 83.0 us (32-byte pieces of cache lines).
+template <int NC>
+struct LineLds {
+  double v[2][3][NC * 16];  // two buffers used in turn
+  int coupled[8];           // per reduction step: some coupling is above kDecoupled
 };
 
-// Coefficient tables of up to 8 media (3 * 8 * 8 entries) go to LDS in the
-// tile kernels, whose LDS is mostly taken by the lines.
-constexpr int kTileCoef = 192;
+template <int S, int NC>
+__device__ inline void block_line_solve(const double (&a)[S], const double (&b)[S], const double (&c)[S], const double (&d)[S], double (&x)[S],
+                                        LineLds<NC>& L) {
+  const int t = threadIdx.x, ch = t >> 4;
+  double g[S], p[S], q[S];
+  {
+    const double r = prcp(b[0]);
+    g[0] = c[0] * r;
+    p[0] = d[0] * r;
+    q[0] = a[0] * r;
+  }
+#pragma unroll
+  for (int s = 1; s < S; ++s) {
+    const double r = prcp(fma(-a[s], g[s - 1], b[s]));
+    g[s] = c[s] * r;
+    p[s] = fma(-a[s], p[s - 1], d[s]) * r;
+    q[s] = -a[s] * q[s - 1] * r;
+  }
+  double P = 0.0, Q = 0.0, R = 1.0;
+#pragma unroll
+  for (int s = S - 2; s >= 0; --s) {
+    P = fma(-g[s], P, p[s]);
+    Q = fma(-g[s], Q, q[s]);
+    R = -g[s] * R;
+  }
+  L.v[0][0][t] = P;
+  L.v[0][1][t] = Q;
+  L.v[0][2][t] = R;
+  if (t < 8) L.coupled[t] = 0;
+  __syncthreads();
+  // entry of chunk ch + h (0 outside the line)
+  auto at = [&](int buf, int k, int h) {
+    const bool in = ch + h >= 0 && ch + h < NC;
+    const double v = L.v[buf][k][in ? t + 16 * h : t];
+    return in ? v : 0.0;
+  };
+  const double Pn = at(0, 0, 1), Qn = at(0, 1, 1), Rn = at(0, 2, 1);
+  const double e = g[S - 1], ib = prcp(fma(-e, Qn, 1.0));
+  double pa = q[S - 1] * ib, pc = e * Rn * ib, pd = fma(-e, Pn, p[S - 1]) * ib;
+  double U = 0.0, UL = 0.0;
+  int buf = 1;
+  for (int h = 1, step = 0;; h <<= 1, ++step) {
+    L.v[buf][0][t] = pd;
+    L.v[buf][1][t] = pa;
+    L.v[buf][2][t] = pc;
+    if (!(fmax(fabs(pa), fabs(pc)) <= kDecoupled)) L.coupled[step] = 1;
+    __syncthreads();
+    const double dm = at(buf, 0, -h), dp = at(buf, 0, h);
+    if (h >= NC || !L.coupled[step]) {
+      U = fma(-pc, dp, fma(-pa, dm, pd));
+      UL = fma(-at(buf, 2, -1), at(buf, 0, h - 1), fma(-at(buf, 1, -1), at(buf, 0, -h - 1), at(buf, 0, -1)));
+      break;
+    }
+    const double am = at(buf, 1, -h), cm = at(buf, 2, -h), ap = at(buf, 1, h), cp = at(buf, 2, h);
+    const double r = prcp(fma(-pc, ap, fma(-pa, cm, 1.0)));
+    pd = fma(-pc, dp, fma(-pa, dm, pd)) * r;
+    pa = -pa * am * r;
+    pc = -pc * cp * r;
+    buf ^= 1;
+  }
+  x[S - 1] = U;
+#pragma unroll
+  for (int s = S - 2; s >= 0; --s) x[s] = fma(-g[s], x[s + 1], fma(-q[s], UL, p[s]));
+}
 
-template <int S, int W, int KIND, bool LDS_COEF>
-__global__ void __launch_bounds__(kHeatTPB) heat_sweep_yz_tile(HeatArgs<double> a) {
-  constexpr int TX = YzTile<S, W>::TX, NP = YzTile<S, W>::NP, LD = YzTile<S, W>::LD;
-  __shared__ double sT[TX * LD], sR[TX * LD];
-  __shared__ double sC[LDS_COEF ? kTileCoef : 1];
-  if (LDS_COEF)
-    for (int k = threadIdx.x; k < a.nM * a.nM * 3; k += blockDim.x) sC[k] = a.c[k];
-  const double* __restrict__ cT = LDS_COEF ? sC : a.c;  // LDS or global, never a generic pointer
-  __shared__ uint8_t sM[TX * NP];
-  __shared__ double sLogA[KIND == SWEEP_Z ? 256 : 1], sE[KIND == SWEEP_Z ? 256 : 1];
-  __shared__ unsigned long long sMax[KIND == SWEEP_Z ? 256 : 1];
-  const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = nx * ny, nM = a.nM;
-  const int nLine = KIND == SWEEP_Y ? ny : nz;
-  const int st = KIND == SWEEP_Y ? nx : nxy;
-  const int d = KIND == SWEEP_Y ? 1 : 2;
-  const int nOther = KIND == SWEEP_Y ? nz : ny;
-  const int ntx = (nx + TX - 1) / TX;
-  const int tx0 = (blockIdx.x % ntx) * TX, o = blockIdx.x / ntx;
-  const int base = KIND == SWEEP_Y ? tx0 + o * nxy : tx0 + o * nx;
-  const int cols = min(TX, nx - tx0);
+// per-axis coefficient tables of up to this many entries go to LDS in the y/z
+// kernels (22 media, like kLdsCoef)
+constexpr int kAxisCoef = 512;
+
+// What a thread of a y/z kernel works on: chunk `ch` (voxels k0 .. k0+S-1) of
+// the line at x and the other coordinate o.
+struct LinePos {
+  int x, o, k0, base;
+  bool valid;  // false: a copy of the last line, which stores nothing
+};
+template <int S, int NC, int AXIS>
+__device__ inline LinePos line_pos(int nx, int ny) {
+  LinePos L;
+  const int ntx = (nx + 15) >> 4, blk = xcd_contiguous(blockIdx.x, gridDim.x);
+  L.o = blk / ntx;
+  const int xw = ((blk - L.o * ntx) << 4) + (threadIdx.x & 15);
+  L.valid = xw < nx;
+  L.x = L.valid ? xw : nx - 1;
+  L.k0 = (threadIdx.x >> 4) * S;
+  L.base = L.x + L.o * (AXIS == 1 ? nx * ny : nx);
+  return L;
+}
+
+// Arrhenius updates collected per wavefront: the voxels whose medium can be
+// damaged are few and scattered over lanes, so a wavefront appends them to a
+// queue and evaluates 64 at a time with all its lanes.
+constexpr int kBurnQueue = 128;
+struct BurnQueue {
+  double th[kBurnQueue];  // mean temperature of the step [K]
+  int i[kBurnQueue], m[kBurnQueue];
+};
+__device__ inline void burn(const HeatArgs<double>& a, const BurnQueue& B, int e, const double* sLogA, const double* sE) {
+  const int m = B.m[e], i = B.i[e];
+  a.Om[i] += a.dt * exp(fma(-sE[m], prcp(a.Rgas * B.th[e]), sLogA[m]));
+}
+
+// substeps 2a + 2b (KIND Y) and 3a + 3b with the Arrhenius update and the
+// per-medium maxima (KIND Z) in FP64.  50 us for z at 200^3, half of it the
+// damage and maxima; exponentials evaluated where their voxels lie (13 rounds
+// with 3 of 16 lanes) cost 30 us more.
+template <int S, int NC, int KIND, bool LDS_COEF>
+__global__ void __launch_bounds__(NC * 16) heat_sweep_yz(HeatArgs<double> a) {
+  constexpr bool Z = KIND == SWEEP_Z;
+  constexpr int d = Z ? 2 : 1;
+  __shared__ LineLds<NC> lds;
+  __shared__ double sC[LDS_COEF ? kAxisCoef : 1];
+  __shared__ double sLogA[Z ? 256 : 1], sE[Z ? 256 : 1];
+  __shared__ unsigned long long sMax[Z ? 256 : 1];
+  __shared__ BurnQueue sBurn[Z ? NC / 4 : 1];
+  const int nx = a.nx, ny = a.ny, nz = a.nz, nM = a.nM;
+  const int n = Z ? nz : ny, nOther = Z ? ny : nz, st = Z ? nx * ny : nx;
+  const LinePos L = line_pos<S, NC, d>(nx, ny);
+  double* __restrict__ T2 = a.T2;
   const double* __restrict__ T1 = a.T1;
   const uint8_t* __restrict__ Mg = a.M;
-  if (KIND == SWEEP_Z)
+  double cd[S], T[Z ? S : 1];
+  int Mv[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int i = L.base + min(L.k0 + s, n - 1) * st;
+    cd[s] = T2[i];
+    Mv[s] = Mg[i];
+    if (Z) T[s] = T1[i];
+  }
+  const int Ml = Mg[L.base + min(max(L.k0 - 1, 0), n - 1) * st], Mr = Mg[L.base + min(L.k0 + S, n - 1) * st];
+  if (LDS_COEF)
+    for (int k = threadIdx.x; k < nM * nM; k += blockDim.x) sC[k] = a.c[k + d * nM * nM];
+  if (Z)
     for (int k = threadIdx.x; k < nM; k += blockDim.x) {
       sLogA[k] = a.logA[k];
       sE[k] = a.E[k];
-      sMax[k] = order_key(-INFINITY);
+      sMax[k] = a.maxKey[k];
     }
-  // all loads of a thread are issued before the first LDS store
-  constexpr int kIt = (TX * NP + kHeatTPB - 1) / kHeatTPB;
-  {
-    double vT[kIt], vR[kIt];
-    int vM[kIt];
-#pragma unroll
-    for (int q = 0; q < kIt; ++q) {
-      const int e = threadIdx.x + q * kHeatTPB;
-      const int c = e % TX, k = e / TX;
-      const bool ok = c < cols && k < nLine;
-      const int i = ok ? base + c + k * st : base;
-      vT[q] = T1[i];
-      vR[q] = a.T2[i];
-      vM[q] = Mg[i];
-    }
-#pragma unroll
-    for (int q = 0; q < kIt; ++q) {
-      const int e = threadIdx.x + q * kHeatTPB;
-      const int c = e % TX, k = e / TX;
-      if (c < cols && k < nLine) {
-        sT[c * LD + k] = vT[q];
-        sR[c * LD + k] = vR[q];
-        sM[c * NP + k] = (uint8_t)vM[q];
-      }
-    }
-  }
   __syncthreads();
-  // a line per W-lane segment: segment g of wavefront w solves lines
-  // w * 64 / W + g, + 4 * 64 / W, ...; a segment past the last line solves
-  // an empty system and stores nothing
-  const int wl = __lane_id(), lane = wl & (W - 1), wave = threadIdx.x >> 6;
-  const bool sk = a.sinked;
-  const double dt = a.dt;
-  for (int c0 = wave * (64 / W); c0 < cols; c0 += kHeatTPB / W) {
-    const bool valid = c0 + wl / W < cols;
-    const int c = valid ? c0 + wl / W : c0;
-    const int n = valid ? nLine : 0;
-    const int x = tx0 + c;
-    const bool lf = sk && (x == 0 || x == nx - 1 || o == 0 || o == nOther - 1);
-    double Tn[S], R0[S];
-    int Mv[S];
+  const double* __restrict__ cT = LDS_COEF ? sC : a.c + d * nM * nM;  // LDS or global, never a generic pointer
+  const bool sk = a.sinked, lf = sk && (L.x == 0 || L.x == nx - 1 || L.o == 0 || L.o == nOther - 1);
+  const double h = a.dt / 2;
+  double ca[S], cb[S], cc_[S], xs[S];
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int k = lane * S + s;
-      Tn[s] = k < n ? sT[c * LD + k] : 0.0;
-      R0[s] = k < n ? sR[c * LD + k] : 0.0;
-      Mv[s] = k < n ? (int)sM[c * NP + k] : 0;
-    }
-    const double Tl = seg_shift<W, false>(Tn[S - 1], 1), Tr = seg_shift<W, true>(Tn[0], 1);
-    const int Ml = seg_shift<W, false>(Mv[S - 1], 1), Mr = seg_shift<W, true>(Mv[0], 1);
-    double ca[S], cb[S], cc_[S], cd[S], xs[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int k = lane * S + s;
-      ca[s] = 0.0;
-      cb[s] = 1.0;
-      cc_[s] = 0.0;
-      cd[s] = 0.0;
-      if (k >= n) continue;
-      const int m = Mv[s];
-      const double TL = s > 0 ? Tn[s - 1] : Tl, TR = s < S - 1 ? Tn[s + 1] : Tr;
-      const int ML = s > 0 ? Mv[s - 1] : Ml, MR = s < S - 1 ? Mv[s + 1] : Mr;
-      const bool fz = lf || (sk && (k == 0 || k == n - 1));
-      double t = R0[s];
-      if (!fz) {
-        double dTdt = 0;
-        if (k != 0) dTdt -= (TL - Tn[s]) * coef(cT, nM, m, ML, d) / 2;
-        if (k != n - 1) dTdt -= (TR - Tn[s]) * coef(cT, nM, m, MR, d) / 2;
-        t = t + dt * dTdt;
-        if (k < n - 1) {
-          const double q = dt / 2 * coef(cT, nM, m, MR, d);
-          cb[s] += q;
-          cc_[s] = -q;
-        }
-        if (k > 0) {
-          const double q = dt / 2 * coef(cT, nM, m, ML, d);
-          cb[s] += q;
-          ca[s] = -q;
-        }
-      }
-      cd[s] = t;
-    }
-    wave_tridiag<S, W>(ca, cb, cc_, cd, xs);
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int k = lane * S + s;
-      if (k < n) sR[c * LD + k] = xs[s];
-    }
+  for (int s = 0; s < S; ++s) {
+    const int k = L.k0 + s;
+    const double cl = coef(cT, nM, Mv[s], s > 0 ? Mv[s - 1] : Ml, 0), cr = coef(cT, nM, Mv[s], s < S - 1 ? Mv[s + 1] : Mr, 0);
+    const bool on = k < n && !lf && !(sk && (k == 0 || k == n - 1));
+    ca[s] = on && k > 0 ? -h * cl : 0.0;
+    cc_[s] = on && k < n - 1 ? -h * cr : 0.0;
+    cb[s] = 1.0 - (ca[s] + cc_[s]);
+    cd[s] = k < n ? cd[s] : 0.0;
   }
-  __syncthreads();
+  block_line_solve<S, NC>(ca, cb, cc_, cd, xs, lds);
+  if (!Z) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (L.valid && L.k0 + s < n) T2[L.base + (L.k0 + s) * st] = xs[s];
+    return;
+  }
   MaxRun run;
-  double* __restrict__ T2 = a.T2;
-  double* __restrict__ Om = a.Om;
-  double vO[KIND == SWEEP_Z ? kIt : 1];
-  if (KIND == SWEEP_Z && a.calcDamage) {
+  BurnQueue& B = sBurn[threadIdx.x >> 6];
+  const int lane = __lane_id();
+  int queued = 0;  // wavefront-uniform
 #pragma unroll
-    for (int q = 0; q < kIt; ++q) {
-      const int e = threadIdx.x + q * kHeatTPB;
-      const int c = e % TX, k = e / TX;
-      const bool ok = c < cols && k < nLine;
-      vO[q] = Om[ok ? base + c + k * st : base];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < kIt; ++q) {
-    const int e = threadIdx.x + q * kHeatTPB;
-    const int c = e % TX, k = e / TX;
-    if (c >= cols || k >= nLine) continue;
-    const int i = base + c + k * st;
-    const double t = sR[c * LD + k];
-    T2[i] = t;
-    if (KIND == SWEEP_Z) {
-      const int m = sM[c * NP + k];
-      if (a.calcDamage && sE[m] != 0) Om[i] = vO[q] + dt * exp(sLogA[m] - sE[m] / (a.Rgas * ((t + sT[c * LD + k]) / 2 + a.czero)));
+  for (int s = 0; s < S; ++s) {
+    const int k = L.k0 + s, i = L.base + k * st, m = Mv[s];
+    const bool live = L.valid && k < n;
+    const double t = T[s] + xs[s];
+    if (live) {
+      T2[i] = t;
       run.add(m, t, sMax);
     }
+    const bool burns = live && a.calcDamage && sE[m] != 0;
+    const unsigned long long bal = __ballot(burns);
+    if (bal) {
+      if (burns) {
+        const int e = queued + __popcll(bal & ((1ull << lane) - 1ull));
+        B.th[e] = (t + T[s]) / 2 + a.czero;
+        B.i[e] = i;
+        B.m[e] = m;
+      }
+      queued += __popcll(bal);
+      if (queued >= 64) {
+        queued -= 64;
+        burn(a, B, queued + lane, sLogA, sE);
+      }
+    }
   }
-  if (KIND == SWEEP_Z) {
-    run.flush(sMax);
-    fold_lds_max(sMax, a.maxKey, nM);
-  }
+  if (lane < queued) burn(a, B, lane, sLogA, sE);
+  run.flush(sMax);
+  fold_lds_max(sMax, a.maxKey, nM);
 }
 
-// rows per lane of the wavefront x-solve for a line of n voxels (0: use the
-// sequential lane-per-line kernel)
-inline int wave_rows(int n) { return n <= 64 ? 1 : n <= 128 ? 2 : n <= 256 ? 4 : n <= 512 ? 8 : 0; }
+// whether the wavefront solvers take a line of n voxels (else the sequential
+// lane-per-line kernels)
+inline bool wave_line(int n) { return n <= 512; }
 
-// rows per lane S and lanes per line W of the forward wavefront solver for a
-// line of n <= 512 voxels.  Fewer lanes per line mean more rows per lane and
-// fewer cyclic-reduction steps, with 64 / W lines solved side by side in one
-// wavefront.  Measured per step (200 on + 200 off steps, layered skin):
-// y/z sweeps with W = 16 up to 128 voxels and W = 32 up to 256 took the DG-ADI
-// step at 128^3 from 0.097 to 0.064 ms and at 200^3 from 0.259 to 0.232 ms;
-// the x sweep, which also gathers four neighbouring lines, gains from W = 32
-// only up to 128 voxels (more rows per lane cost it occupancy: 154 VGPRs at
-// S = 8).
-struct WaveShape {
-  int S, W;
-};
-inline WaveShape wave_shape(int n, bool xAxis) {
-  if (n <= 32 || n > 256) return {wave_rows(n), 64};
-  if (xAxis) return n <= 128 ? WaveShape{n <= 64 ? 2 : 4, 32} : WaveShape{4, 64};
-  return n <= 128 ? WaveShape{n <= 64 ? 4 : 8, 16} : WaveShape{8, 32};
+// Calls f(integral_constant S, integral_constant W) with the rows per lane and
+// lanes per line of the x sweeps.
+template <class F>
+inline void with_x_shape(int n, F&& f) {
+  using std::integral_constant;
+  if (n <= 64) return f(integral_constant<int, 2>(), integral_constant<int, 32>());
+  if (n <= 128) return f(integral_constant<int, 4>(), integral_constant<int, 32>());
+  if (n <= 256) return f(integral_constant<int, 4>(), integral_constant<int, 64>());
+  return f(integral_constant<int, 8>(), integral_constant<int, 64>());
 }
 
-// calls f(integral_constant S, integral_constant W) for the shapes
-// wave_shape picks (X: the x sweep's, else the y/z sweeps')
-template <bool X, class F>
-inline void with_wave_shape(WaveShape ws, F&& f) {
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I4 = std::integral_constant<int, 4>;
-  using I8 = std::integral_constant<int, 8>;
-  using I16 = std::integral_constant<int, 16>;
-  using I32 = std::integral_constant<int, 32>;
-  using I64 = std::integral_constant<int, 64>;
-  const int key = ws.W * 16 + ws.S;
-  if (key == 64 * 16 + 1) return f(I1(), I64());
-  if (key == 64 * 16 + 8) return f(I8(), I64());
-  if constexpr (X) {
-    if (key == 64 * 16 + 4) return f(I4(), I64());
-    if (key == 32 * 16 + 2) return f(I2(), I32());
-    if (key == 32 * 16 + 4) return f(I4(), I32());
-  } else {
-    if (key == 32 * 16 + 8) return f(I8(), I32());
-    if (key == 16 * 16 + 4) return f(I4(), I16());
-    if (key == 16 * 16 + 8) return f(I8(), I16());
-  }
+// The same with the rows per thread and chunks per line of the y and z
+// sweeps: the fewest rows of the compiled ones that hold the line in 16
+// chunks (32 chunks beyond 256 voxels).
+template <class F>
+inline void with_yz_shape(int n, F&& f) {
+  using std::integral_constant;
+  using C16 = integral_constant<int, 16>;
+  using C32 = integral_constant<int, 32>;
+  if (n <= 32) return f(integral_constant<int, 2>(), C16());
+  if (n <= 64) return f(integral_constant<int, 4>(), C16());
+  if (n <= 96) return f(integral_constant<int, 6>(), C16());
+  if (n <= 128) return f(integral_constant<int, 8>(), C16());
+  if (n <= 160) return f(integral_constant<int, 10>(), C16());
+  if (n <= 208) return f(integral_constant<int, 13>(), C16());
+  if (n <= 256) return f(integral_constant<int, 16>(), C16());
+  if (n <= 416) return f(integral_constant<int, 13>(), C32());
+  return f(integral_constant<int, 16>(), C32());
 }
 
 // Forward Euler step (no reference counterpart; the 7-point right-hand side
@@ -1115,179 +1145,92 @@ __global__ void __launch_bounds__(kHeatTPB) heat_adj_solve(HeatArgs<double> a, c
   }
 }
 
-// A_d^T x = r along one line of n voxels held S per lane by a wavefront
-// (lane l: voxels l*S .. l*S+S-1; rv the right-hand side, Mv the media; lf:
-// the whole line is frozen).  The rows of A^T are (sub, diag, super) =
-// (c_(k-1), b_k, a_(k+1)) of A's rows; the neighbouring lane's edge
-// coefficients come by one shuffle each.
-template <int S, int W>
-__device__ inline void adj_line_solve(const HeatArgs<double>& a, const double* cT, int axis, int n, bool lf, const double (&rv)[S],
-                                      const int (&Mv)[S], double (&xs)[S]) {
-  const int wl = __lane_id(), lane = wl & (W - 1);  // lane within the line's W-lane segment
+// Rows of A_d^T on S consecutive voxels k0 .. k0+S-1 of a line of n voxels (lf:
+// the whole line is frozen; Ml, Mr: media of the voxels before and after).  The
+// rows of A^T are (sub, diag, super) = (c_(k-1), b_k, a_(k+1)) of A's rows,
+// which vanish where voxel k-1 (k+1) is frozen.
+template <int S>
+__device__ inline void adj_rows(const HeatArgs<double>& a, const double* cT, int n, int k0, bool lf, const int (&Mv)[S], int Ml, int Mr,
+                                double (&ta)[S], double (&tb)[S], double (&tc)[S]) {
   const double h = a.dt / 2;
-  double A[S], B[S], Cc[S];
-  const int Ml = seg_shift<W, false>(Mv[S - 1], 1), Mr = seg_shift<W, true>(Mv[0], 1);
-  // rows of A
+  const int nM = a.nM;
+  auto moves = [&](int k) { return k >= 0 && k < n && !lf && !(a.sinked && (k == 0 || k == n - 1)); };
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int k = lane * S + s;
-    A[s] = 0.0;
-    B[s] = 1.0;
-    Cc[s] = 0.0;
-    if (k >= n || lf || (a.sinked && (k == 0 || k == n - 1))) continue;
-    const int m = Mv[s];
+    const int k = k0 + s, m = Mv[s];
     const int ML = s > 0 ? Mv[s - 1] : Ml, MR = s < S - 1 ? Mv[s + 1] : Mr;
-    if (k > 0) {
-      const double q = h * coef(cT, a.nM, m, ML, axis);
-      B[s] += q;
-      A[s] = -q;
-    }
-    if (k < n - 1) {
-      const double q = h * coef(cT, a.nM, m, MR, axis);
-      B[s] += q;
-      Cc[s] = -q;
-    }
+    const double toL = coef(cT, nM, m, ML, 0), toR = coef(cT, nM, m, MR, 0), fromL = coef(cT, nM, ML, m, 0), fromR = coef(cT, nM, MR, m, 0);
+    const bool on = moves(k);
+    ta[s] = k < n && moves(k - 1) ? -h * fromL : 0.0;
+    tc[s] = k < n && moves(k + 1) ? -h * fromR : 0.0;
+    tb[s] = 1.0 + (on && k > 0 ? h * toL : 0.0) + (on && k < n - 1 ? h * toR : 0.0);
   }
-  // rows of A^T
-  const double cPrevLane = seg_shift<W, false>(Cc[S - 1], 1), aNextLane = seg_shift<W, true>(A[0], 1);
-  double ta[S], tb[S], tc[S];
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const int k = lane * S + s;
-    const bool ok = k < n;
-    ta[s] = ok && k > 0 ? (s > 0 ? Cc[s - 1] : cPrevLane) : 0.0;
-    tb[s] = ok ? B[s] : 1.0;
-    tc[s] = ok && k < n - 1 ? (s < S - 1 ? A[s + 1] : aNextLane) : 0.0;
-  }
-  wave_tridiag<S, W>(ta, tb, tc, rv, xs);
 }
 
-// A_d^T y = r with one wavefront per line (lines of up to 512 voxels),
-// loading the line directly (x lines; strided along y and z).
-template <int S, int W, int AXIS, bool LDS_COEF>
-__global__ void __launch_bounds__(kHeatTPB) heat_adj_solve_wave(HeatArgs<double> a, const double* __restrict__ r, double* y) {
-  __shared__ double sC[LDS_COEF ? kTileCoef : 1];
-  if (LDS_COEF) {
-    for (int k = threadIdx.x; k < a.nM * a.nM * 3; k += blockDim.x) sC[k] = a.c[k];
-    __syncthreads();
-  }
-  const double* __restrict__ cT = LDS_COEF ? sC : a.c;
-  const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = nx * ny;
-  // a line per W-lane segment; a segment past the last line solves the
-  // last line again and stores nothing
+// A_d^T y = r on x lines of up to 512 voxels, a line per W lanes.
+template <int S, int W, bool LDS_COEF>
+__global__ void __launch_bounds__(kHeatTPB) heat_adj_solve_x(HeatArgs<double> a, const double* __restrict__ r, double* __restrict__ y) {
+  __shared__ double sC[LDS_COEF ? kAxisCoef : 1];
+  const int nx = a.nx, ny = a.ny, nz = a.nz;
+  // a segment past the last line solves the last line again and stores nothing
   const int wl = __lane_id(), lane = wl & (W - 1);
-  const int seg = (blockIdx.x * (kHeatTPB / 64) + (threadIdx.x >> 6)) * (64 / W) + wl / W;
-  const int nLines = AXIS == 0 ? ny * nz : AXIS == 1 ? nx * nz : nxy;
-  const bool valid = seg < nLines;
-  const int line = valid ? seg : nLines - 1;
-  int i0, st, n;
-  bool lf;
-  if (AXIS == 0) {
-    const int yy = line % ny, zz = line / ny;
-    i0 = yy * nx + zz * nxy, st = 1, n = nx;
-    lf = a.sinked && (yy == 0 || yy == ny - 1 || zz == 0 || zz == nz - 1);
-  } else if (AXIS == 1) {
-    const int xx = line % nx, zz = line / nx;
-    i0 = xx + zz * nxy, st = nx, n = ny;
-    lf = a.sinked && (xx == 0 || xx == nx - 1 || zz == 0 || zz == nz - 1);
-  } else {
-    i0 = line, st = nxy, n = nz;
-    const int xx = line % nx, yy = line / nx;
-    lf = a.sinked && (xx == 0 || xx == nx - 1 || yy == 0 || yy == ny - 1);
-  }
-  double rv[S], xs[S];
+  const int seg = (xcd_contiguous(blockIdx.x, gridDim.x) * (kHeatTPB / 64) + (threadIdx.x >> 6)) * (64 / W) + wl / W;
+  const bool valid = seg < ny * nz;
+  const int line = valid ? seg : ny * nz - 1;
+  const int yy = line % ny, zz = line / ny, i0 = line * nx;
+  const bool lf = a.sinked && (yy == 0 || yy == ny - 1 || zz == 0 || zz == nz - 1);
+  double rv[S], xs[S], ta[S], tb[S], tc[S];
   int Mv[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int k = lane * S + s;
-    const int i = i0 + (k < n ? k : 0) * st;
-    rv[s] = k < n ? r[i] : 0.0;
+    const int k = lane * S + s, i = i0 + min(k, nx - 1);
+    const double v = r[i];
+    rv[s] = k < nx ? v : 0.0;
     Mv[s] = a.M[i];
   }
-  adj_line_solve<S, W>(a, cT, AXIS, n, lf, rv, Mv, xs);
+  if (LDS_COEF)
+    for (int k = threadIdx.x; k < a.nM * a.nM; k += blockDim.x) sC[k] = a.c[k];
+  __syncthreads();
+  const int Ml = seg_shift<W, false>(Mv[S - 1], 1), Mr = seg_shift<W, true>(Mv[0], 1);
+  adj_rows<S>(a, LDS_COEF ? sC : a.c, nx, lane * S, lf, Mv, Ml, Mr, ta, tb, tc);
+  line_solve<S, W>(ta, tb, tc, rv, xs);
   if (!valid) return;
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const int k = lane * S + s;
-    if (k < n) y[i0 + k * st] = xs[s];
+    if (k < nx) y[i0 + k] = xs[s];
   }
 }
 
-// A_d^T y = r along y (AXIS 1) or z (AXIS 2) with the lines staged through
-// LDS like the forward y/z sweeps: a workgroup takes TX consecutive x-lines
-// at one z (AXIS 1) or y (AXIS 2), loads them row by row (coalesced), each
-// wavefront solves TX/4 lines, and the rows are written back.
-template <int S, int W, int AXIS, bool LDS_COEF>
-__global__ void __launch_bounds__(kHeatTPB) heat_adj_solve_tile(HeatArgs<double> a, const double* __restrict__ r, double* y) {
-  constexpr int TX = YzTile<S, W>::TX, NP = YzTile<S, W>::NP, LD = YzTile<S, W>::LD;
-  __shared__ double sR[TX * LD];
-  __shared__ uint8_t sM[TX * NP];
-  __shared__ double sC[LDS_COEF ? kTileCoef : 1];
+// A_d^T y = r along y (AXIS 1) or z (AXIS 2), lines of up to 512 voxels laid
+// out over the workgroups like the forward y/z sweeps.
+template <int S, int NC, int AXIS, bool LDS_COEF>
+__global__ void __launch_bounds__(NC * 16) heat_adj_solve_yz(HeatArgs<double> a, const double* __restrict__ r, double* __restrict__ y) {
+  __shared__ LineLds<NC> lds;
+  __shared__ double sC[LDS_COEF ? kAxisCoef : 1];
+  const int nx = a.nx, ny = a.ny, nz = a.nz, nM = a.nM;
+  const int n = AXIS == 1 ? ny : nz, nOther = AXIS == 1 ? nz : ny, st = AXIS == 1 ? nx : nx * ny;
+  const LinePos L = line_pos<S, NC, AXIS>(nx, ny);
+  double rv[S], xs[S], ta[S], tb[S], tc[S];
+  int Mv[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int k = L.k0 + s, i = L.base + min(k, n - 1) * st;
+    const double v = r[i];
+    rv[s] = k < n ? v : 0.0;
+    Mv[s] = a.M[i];
+  }
+  const int Ml = a.M[L.base + min(max(L.k0 - 1, 0), n - 1) * st], Mr = a.M[L.base + min(L.k0 + S, n - 1) * st];
   if (LDS_COEF)
-    for (int k = threadIdx.x; k < a.nM * a.nM * 3; k += blockDim.x) sC[k] = a.c[k];
-  const double* __restrict__ cT = LDS_COEF ? sC : a.c;
-  const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = nx * ny;
-  const int nLine = AXIS == 1 ? ny : nz;
-  const int st = AXIS == 1 ? nx : nxy;
-  const int nOther = AXIS == 1 ? nz : ny;
-  const int ntx = (nx + TX - 1) / TX;
-  const int tx0 = (blockIdx.x % ntx) * TX, o = blockIdx.x / ntx;
-  const int base = AXIS == 1 ? tx0 + o * nxy : tx0 + o * nx;
-  const int cols = min(TX, nx - tx0);
-  constexpr int kIt = (TX * NP + kHeatTPB - 1) / kHeatTPB;
-  {
-    double vR[kIt];
-    int vM[kIt];
-#pragma unroll
-    for (int q = 0; q < kIt; ++q) {
-      const int e = threadIdx.x + q * kHeatTPB;
-      const int c = e % TX, k = e / TX;
-      const int i = c < cols && k < nLine ? base + c + k * st : base;
-      vR[q] = r[i];
-      vM[q] = a.M[i];
-    }
-#pragma unroll
-    for (int q = 0; q < kIt; ++q) {
-      const int e = threadIdx.x + q * kHeatTPB;
-      const int c = e % TX, k = e / TX;
-      if (c < cols && k < nLine) {
-        sR[c * LD + k] = vR[q];
-        sM[c * NP + k] = (uint8_t)vM[q];
-      }
-    }
-  }
+    for (int k = threadIdx.x; k < nM * nM; k += blockDim.x) sC[k] = a.c[k + AXIS * nM * nM];
   __syncthreads();
-  // a line per W-lane segment; a segment past the last line solves an
-  // empty system and stores nothing
-  const int wl = __lane_id(), lane = wl & (W - 1), wave = threadIdx.x >> 6;
-  for (int c0 = wave * (64 / W); c0 < cols; c0 += kHeatTPB / W) {
-    const bool valid = c0 + wl / W < cols;
-    const int c = valid ? c0 + wl / W : c0;
-    const int n = valid ? nLine : 0;
-    const int x = tx0 + c;
-    const bool lf = a.sinked && (x == 0 || x == nx - 1 || o == 0 || o == nOther - 1);
-    double rv[S], xs[S];
-    int Mv[S];
+  const bool lf = a.sinked && (L.x == 0 || L.x == nx - 1 || L.o == 0 || L.o == nOther - 1);
+  adj_rows<S>(a, LDS_COEF ? sC : a.c + AXIS * nM * nM, n, L.k0, lf, Mv, Ml, Mr, ta, tb, tc);
+  block_line_solve<S, NC>(ta, tb, tc, rv, xs, lds);
+  if (!L.valid) return;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int k = lane * S + s;
-      rv[s] = k < n ? sR[c * LD + k] : 0.0;
-      Mv[s] = k < n ? (int)sM[c * NP + k] : 0;
-    }
-    adj_line_solve<S, W>(a, cT, AXIS, n, lf, rv, Mv, xs);
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int k = lane * S + s;
-      if (k < n) sR[c * LD + k] = xs[s];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < kIt; ++q) {
-    const int e = threadIdx.x + q * kHeatTPB;
-    const int c = e % TX, k = e / TX;
-    if (c < cols && k < nLine) y[base + c + k * st] = sR[c * LD + k];
-  }
+  for (int s = 0; s < S; ++s)
+    if (L.k0 + s < n) y[L.base + (L.k0 + s) * st] = xs[s];
 }
 
 __device__ inline bool heat_frozen(const HeatArgs<double>& a, int x, int y, int z) { return frozen(a, x, y, z); }
@@ -1298,7 +1241,7 @@ __global__ void __launch_bounds__(kHeatTPB) heat_adj_combine(HeatArgs<double> a,
                                                             const double* __restrict__ mu3, const double* __restrict__ x0,
                                                             const double* __restrict__ x1, const uint8_t* __restrict__ target,
                                                             double* lamOut, double* dQ, int lightsOn) {
-  __shared__ double sC[LDS_COEF ? kTileCoef : 1];
+  __shared__ double sC[LDS_COEF ? kLdsCoef : 1];
   if (LDS_COEF) {
     for (int k = threadIdx.x; k < a.nM * a.nM * 3; k += blockDim.x) sC[k] = a.c[k];
     __syncthreads();
@@ -1680,9 +1623,9 @@ void launch_lane_sweep(mcm_heat_plan* P, const HeatArgs<RT>& a, unsigned g) {
 template <typename RT>
 void launch_sweep_x(mcm_heat_plan* P, const HeatArgs<RT>& a, unsigned gx) {
   if constexpr (std::is_same<RT, double>::value) {
-    if (wave_rows(P->nx)) {
+    if (wave_line(P->nx)) {
       const bool lc = P->nM * P->nM * 3 <= kLdsCoef;
-      with_wave_shape<true>(wave_shape(P->nx, true), [&](auto sTag, auto wTag) {
+      with_x_shape(P->nx, [&](auto sTag, auto wTag) {
         constexpr int SS = decltype(sTag)::value, WW = decltype(wTag)::value;
         const int64_t lines = (int64_t)P->ny * P->nz, perBlock = kHeatTPB / WW;
         const unsigned gw = (unsigned)((lines + perBlock - 1) / perBlock);
@@ -1698,27 +1641,22 @@ void launch_sweep_x(mcm_heat_plan* P, const HeatArgs<RT>& a, unsigned gx) {
 
 // y and z sweeps: the wavefront solver for FP64 lines of up to 512 voxels,
 // else the sequential lane-per-line kernels.
-template <int S, int W, int KIND>
-void launch_yz_tile(mcm_heat_plan* P, const HeatArgs<double>& a) {
-  constexpr int TX = YzTile<S, W>::TX;
-  const unsigned g = (unsigned)(((P->nx + TX - 1) / TX) * (KIND == SWEEP_Y ? P->nz : P->ny));
-  if (P->nM * P->nM * 3 <= kTileCoef) hipLaunchKernelGGL((heat_sweep_yz_tile<S, W, KIND, true>), dim3(g), dim3(kHeatTPB), 0, P->stream, a);
-  else hipLaunchKernelGGL((heat_sweep_yz_tile<S, W, KIND, false>), dim3(g), dim3(kHeatTPB), 0, P->stream, a);
-}
-
 template <int KIND>
 void launch_yz_wave(mcm_heat_plan* P, const HeatArgs<double>& a, int n) {
-  with_wave_shape<false>(wave_shape(n, false), [&](auto sTag, auto wTag) {
-    launch_yz_tile<decltype(sTag)::value, decltype(wTag)::value, KIND>(P, a);
+  with_yz_shape(n, [&](auto sTag, auto cTag) {
+    constexpr int S = decltype(sTag)::value, NC = decltype(cTag)::value;
+    const unsigned g = (unsigned)(((P->nx + 15) / 16) * (KIND == SWEEP_Y ? P->nz : P->ny));
+    if (P->nM * P->nM <= kAxisCoef) hipLaunchKernelGGL((heat_sweep_yz<S, NC, KIND, true>), dim3(g), dim3(NC * 16), 0, P->stream, a);
+    else hipLaunchKernelGGL((heat_sweep_yz<S, NC, KIND, false>), dim3(g), dim3(NC * 16), 0, P->stream, a);
   });
 }
 
 template <typename RT>
 void launch_sweep_yz(mcm_heat_plan* P, const HeatArgs<RT>& a, unsigned gy, unsigned gz) {
   if constexpr (std::is_same<RT, double>::value) {
-    if (wave_rows(P->ny)) launch_yz_wave<SWEEP_Y>(P, a, P->ny);
+    if (wave_line(P->ny)) launch_yz_wave<SWEEP_Y>(P, a, P->ny);
     else launch_lane_sweep<RT, 1>(P, a, gy);
-    if (wave_rows(P->nz)) launch_yz_wave<SWEEP_Z>(P, a, P->nz);
+    if (wave_line(P->nz)) launch_yz_wave<SWEEP_Z>(P, a, P->nz);
     else launch_lane_sweep<RT, 2>(P, a, gz);
     return;
   }
@@ -1914,26 +1852,23 @@ template <int AXIS>
 void adj_solve(mcm_heat_plan* P, const HeatArgs<double>& a, const double* r, double* y, double* beta, unsigned gLane) {
   const int n = AXIS == 0 ? P->nx : AXIS == 1 ? P->ny : P->nz;
   const int64_t lines = AXIS == 0 ? (int64_t)P->ny * P->nz : AXIS == 1 ? (int64_t)P->nx * P->nz : (int64_t)P->nx * P->ny;
-  const bool lc = P->nM * P->nM * 3 <= kTileCoef;
-  if (!wave_rows(n)) {
+  if (!wave_line(n)) {
     hipLaunchKernelGGL(heat_adj_solve<AXIS>, dim3(gLane), dim3(kHeatTPB), 0, P->stream, a, r, y, beta);
     return;
   }
   if constexpr (AXIS != 0) {
-    // y and z lines through LDS tiles, in the shapes of the forward sweeps
-    with_wave_shape<false>(wave_shape(n, false), [&](auto sTag, auto wTag) {
-      constexpr int S = decltype(sTag)::value, W = decltype(wTag)::value;
-      constexpr int TX = YzTile<S, W>::TX;
-      const unsigned g = (unsigned)(((P->nx + TX - 1) / TX) * (AXIS == 1 ? P->nz : P->ny));
-      if (lc) hipLaunchKernelGGL((heat_adj_solve_tile<S, W, AXIS == 1 ? 1 : 2, true>), dim3(g), dim3(kHeatTPB), 0, P->stream, a, r, y);
-      else hipLaunchKernelGGL((heat_adj_solve_tile<S, W, AXIS == 1 ? 1 : 2, false>), dim3(g), dim3(kHeatTPB), 0, P->stream, a, r, y);
+    with_yz_shape(n, [&](auto sTag, auto cTag) {
+      constexpr int S = decltype(sTag)::value, NC = decltype(cTag)::value;
+      const unsigned g = (unsigned)(((P->nx + 15) / 16) * (AXIS == 1 ? P->nz : P->ny));
+      if (P->nM * P->nM <= kAxisCoef) hipLaunchKernelGGL((heat_adj_solve_yz<S, NC, AXIS, true>), dim3(g), dim3(NC * 16), 0, P->stream, a, r, y);
+      else hipLaunchKernelGGL((heat_adj_solve_yz<S, NC, AXIS, false>), dim3(g), dim3(NC * 16), 0, P->stream, a, r, y);
     });
   } else {
-    with_wave_shape<true>(wave_shape(n, true), [&](auto sTag, auto wTag) {
+    with_x_shape(n, [&](auto sTag, auto wTag) {
       constexpr int S = decltype(sTag)::value, W = decltype(wTag)::value;
       const unsigned gw = (unsigned)((lines + kHeatTPB / W - 1) / (kHeatTPB / W));
-      if (lc) hipLaunchKernelGGL((heat_adj_solve_wave<S, W, AXIS, true>), dim3(gw), dim3(kHeatTPB), 0, P->stream, a, r, y);
-      else hipLaunchKernelGGL((heat_adj_solve_wave<S, W, AXIS, false>), dim3(gw), dim3(kHeatTPB), 0, P->stream, a, r, y);
+      if (P->nM * P->nM <= kAxisCoef) hipLaunchKernelGGL((heat_adj_solve_x<S, W, true>), dim3(gw), dim3(kHeatTPB), 0, P->stream, a, r, y);
+      else hipLaunchKernelGGL((heat_adj_solve_x<S, W, false>), dim3(gw), dim3(kHeatTPB), 0, P->stream, a, r, y);
     });
   }
 }
@@ -2303,7 +2238,7 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
       adj_solve<1>(P, a, (const double*)mu3.p, (double*)mu2.p, B, gy);
       adj_solve<0>(P, a, (const double*)mu2.p, (double*)mu1.p, B, gx);
       const dim3 gc((unsigned)((P->nx * P->ny + tpb - 1) / tpb), (unsigned)P->nz);
-      if (P->nM * P->nM * 3 <= kTileCoef)
+      if (P->nM * P->nM * 3 <= kLdsCoef)
         hipLaunchKernelGGL(heat_adj_combine<true>, gc, dim3(tpb), 0, s, a, (const double*)mu1.p, (const double*)mu2.p,
                            (const double*)mu3.p, x0, x1, (const uint8_t*)dMask.p, (double*)lamN.p, (double*)dQ.p, lights[(size_t)n]);
       else
