@@ -120,28 +120,22 @@ __device__ inline RT cc(const HeatArgs<RT>& a, int m, int n, int d) {
 // Running maxima per medium.  The keys in LDS start from the global running
 // maxima, so a voxel that does not raise its medium's maximum touches no
 // atomic (a stale start is harmless: the keys only grow), and a workgroup
-// writes back only what it raised.  Starting every workgroup from -inf cost
+// writes back only what it raised.  Like the reference's comparison
+// (maxT < T), a NaN raises nothing.  Starting every workgroup from -inf cost
 // one LDS atomic per lane and one same-address global atomic per workgroup,
 // medium and step.
 struct MaxRun {
   int m = -1;
-  double v = -INFINITY;
-  __device__ static void raise(unsigned long long* s, int m, double v) {
-    const unsigned long long k = order_key(v);
-    if (k > *(volatile unsigned long long*)&s[m]) atomicMax(&s[m], k);
-  }
+  double v = 0;  // the maximum of medium m as far as this lane knows
   __device__ void add(int mm, double t, unsigned long long* s) {
     if (mm != m) {
-      if (m >= 0) raise(s, m, v);
       m = mm;
-      v = t;
-    } else if (t > v) {
+      v = key_value(__hip_atomic_load(&s[m], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+    }
+    if (t > v) {
+      atomicMax(&s[m], order_key(t));
       v = t;
     }
-  }
-  __device__ void flush(unsigned long long* s) {
-    if (m >= 0) raise(s, m, v);
-    m = -1;
   }
 };
 
@@ -367,7 +361,6 @@ __global__ void __launch_bounds__(kHeatTPB) heat_sweep_z(HeatArgs<RT> a) {
     const bool lf = a.sinked && (x == 0 || x == a.nx - 1 || y == 0 || y == a.ny - 1);
     MaxRun run;
     sweep_line<RT, SWEEP_Z, kSweepU>(a, cT, L, line, a.nx * a.ny, a.nz, lf, 2, 0, 0, 1, 0, 0, 1, &run, L.maxKey);
-    run.flush(L.maxKey);
   }
   fold_lds_max(L.maxKey, a.maxKey, a.nM);
 }
@@ -868,7 +861,6 @@ __global__ void __launch_bounds__(NC * 16) heat_sweep_yz(HeatArgs<double> a) {
     }
   }
   if (lane < queued) burn(a, B, lane, sLogA, sE);
-  run.flush(sMax);
   fold_lds_max(sMax, a.maxKey, nM);
 }
 
@@ -906,102 +898,119 @@ inline void with_yz_shape(int n, F&& f) {
   return f(integral_constant<int, 16>(), C32());
 }
 
+// v of the lane before (after) in the wavefront; lane 0 (63) gets 0
+template <typename V>
+__device__ inline V lane_before(V v) {
+  return __shfl_up(v, 1, 64);
+}
+template <typename V>
+__device__ inline V lane_after(V v) {
+  return __shfl_down(v, 1, 64);
+}
+
 // Forward Euler step (no reference counterpart; the 7-point right-hand side
 // of substep 1a with all three axes fully weighted, the damage update and
-// the per-medium maxima of the DG-ADI step).  A workgroup owns a
-// kTileX x kTileY column tile and a run of kZRun z planes (chosen per plan by
-// timing, see tune_explicit), marching up in z:
-// each plane of T and M (with its x/y halo) is staged through LDS once, so
-// every voxel is loaded from memory once and its four in-plane neighbours
-// come from LDS; the z neighbours are carried in registers.
-constexpr int kTileX = 64, kTileY = 4;
-
-template <typename RT, bool LDS_COEF>
-__global__ void __launch_bounds__(kTileX * kTileY) heat_explicit_tile(HeatArgs<RT> a, int kZRun) {
+// the per-medium maxima of the DG-ADI step).  A thread owns a column and
+// marches up a run of zRun z planes (chosen per plan by timing, see
+// tune_explicit); the threads of a workgroup own consecutive voxels of the
+// plane, whatever the row length.  The z neighbours are carried in registers,
+// the x neighbours come from the neighbouring lanes (the wavefront's first and
+// last lane load theirs), the y neighbours are loaded, and all loads of a plane
+// are issued one plane ahead of their use (the voxel above two ahead).
+//
+// 225x190x171, lights on and off: 39 us a step (3.4 to 4 TB/s of compulsory
+// bytes), bound by instruction issue together with the memory's latency;
+// staging each plane through LDS behind two barriers took 53 us (45 of them
+// once maxima no longer went through global atomics).  Two planes ahead, or
+// register roles rotated instead of copied, need 4 wavefronts' registers
+// instead of 5 and were slower on large grids.  Addresses are a plane's base in
+// scalar registers plus a 32-bit byte offset in the plane (OFF = uint32_t;
+// planes of 2^28 voxels or more use 64-bit offsets); a coefficient's address is
+// one multiply-add.
+template <typename RT, bool LDS_COEF, typename OFF>
+__global__ void __launch_bounds__(kHeatTPB) heat_explicit_march(HeatArgs<RT> a, int zRun) {
   __shared__ HeatLds<RT> L;
-  __shared__ RT sT[kTileY + 2][kTileX + 2];
-  __shared__ uint8_t sM[kTileY + 2][kTileX + 2];
   step_sensors(a);
-  (void)stage_tables(a, L);
-  const RT* cT = LDS_COEF ? L.c : a.c;  // LDS or global, never a generic pointer
   const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = nx * ny, nM = a.nM;
-  const int ntx = (nx + kTileX - 1) / kTileX, nty = (ny + kTileY - 1) / kTileY;
-  const int b = blockIdx.x;
-  const int x0 = (b % ntx) * kTileX, y0 = (b / ntx % nty) * kTileY, z0 = b / (ntx * nty) * kZRun;
-  const int tx = threadIdx.x % kTileX, ty = threadIdx.x / kTileX;
-  const int x = x0 + tx, y = y0 + ty;
-  const bool ok = x < nx && y < ny;
-  const int col = ok ? x + y * nx : 0;
-  const int zEnd = min(z0 + kZRun, nz);
-  // halo duty: the tile's edge threads also stage the neighbouring column
-  const int hx = tx == 0 ? x - 1 : (tx == kTileX - 1 ? x + 1 : -1);
-  const int hy = ty == 0 ? y - 1 : (ty == kTileY - 1 ? y + 1 : -1);
-  const bool hxOk = ok && hx >= 0 && hx < nx, hyOk = ok && hy >= 0 && hy < ny;
-  const int hxCol = hxOk ? hx + y * nx : 0, hyCol = hyOk ? x + hy * nx : 0;
-  const int sxh = tx == 0 ? 0 : kTileX + 1, syh = ty == 0 ? 0 : kTileY + 1;
+  const int npb = (nxy + kHeatTPB - 1) / kHeatTPB, blk = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int zi = blk / npb;
+  const int p0 = (blk - zi * npb) * kHeatTPB + threadIdx.x, z0 = zi * zRun, zEnd = min(z0 + zRun, nz);
+  const bool ok = p0 < nxy;
+  const int p = ok ? p0 : nxy - 1, x = p % nx, y = p / nx;
+  const bool sideFrozen = a.sinked && (x == 0 || x == nx - 1 || y == 0 || y == ny - 1);
+  const bool first = __lane_id() == 0, last = __lane_id() == 63;
+  // Neighbours outside the grid are the voxel itself (difference 0).
+  const bool noL = x == 0, noR = x == nx - 1;
+  const OFF oP = (OFF)p, oYm = (OFF)(y > 0 ? p - nx : p), oYp = (OFF)(y < ny - 1 ? p + nx : p);
+  const OFF oE = (OFF)(first ? max(p - 1, 0) : min(p + 1, nxy - 1));
+  auto ldT = [&](int z, OFF o) { return *(const RT*)((const char*)(a.T1 + (int64_t)z * nxy) + (OFF)(o * (OFF)sizeof(RT))); };
+  auto ldM = [&](int z, OFF o) { return (unsigned)*(const uint8_t*)((const char*)(a.M + (int64_t)z * nxy) + o); };
+  struct Side {  // a plane's neighbours within the plane and its source
+    RT ym, yp, e;
+    unsigned mym, myp, me;
+    float q;
+  };
+  auto load_side = [&](int z) {
+    Side s;
+    z = min(z, nz - 1);
+    s.ym = ldT(z, oYm);
+    s.yp = ldT(z, oYp);
+    s.mym = ldM(z, oYm);
+    s.myp = ldM(z, oYp);
+    s.e = 0;
+    s.me = 0;
+    if (first || last) {
+      s.e = ldT(z, oE);
+      s.me = ldM(z, oE);
+    }
+    s.q = a.lightsOn ? *(const float*)((const char*)(a.Q + (int64_t)z * nxy) + (OFF)(oP * (OFF)4)) : 0.f;
+    return s;
+  };
+  auto clampz = [&](int z) { return min(max(z, 0), nz - 1); };
+  RT tBelow = ldT(clampz(z0 - 1), oP), tHere = ldT(z0, oP), tAbove = ldT(clampz(z0 + 1), oP);
+  unsigned mBelow = ldM(clampz(z0 - 1), oP), mHere = ldM(z0, oP), mAbove = ldM(clampz(z0 + 1), oP);
+  Side here = load_side(z0);
+  (void)stage_tables(a, L);
+  const char* cT = (const char*)(LDS_COEF ? L.c : a.c);  // LDS or global, never a generic pointer
+  const unsigned pitch = (unsigned)(nM * sizeof(RT)), axis = pitch * (unsigned)nM;
   const RT dt = a.dt;
   MaxRun run;
-  RT tBelow = 0, tHere = 0;
-  int mBelow = 0, mHere = 0;
-  if (ok) {
-    tBelow = z0 > 0 ? a.T1[col + (z0 - 1) * nxy] : (RT)0;
-    mBelow = z0 > 0 ? (int)a.M[col + (z0 - 1) * nxy] : 0;
-    tHere = a.T1[col + z0 * nxy];
-    mHere = a.M[col + z0 * nxy];
-  }
   for (int z = z0; z < zEnd; ++z) {
-    const int i = col + z * nxy;
-    // this thread's loads for the step, all issued before the LDS stores
-    RT tAbove = 0, hxT = 0, hyT = 0;
-    int mAbove = 0, hxM = 0, hyM = 0;
-    if (ok && z != nz - 1) {
-      tAbove = a.T1[i + nxy];
-      mAbove = a.M[i + nxy];
-    }
-    if (hxOk) {
-      hxT = a.T1[hxCol + z * nxy];
-      hxM = a.M[hxCol + z * nxy];
-    }
-    if (hyOk) {
-      hyT = a.T1[hyCol + z * nxy];
-      hyM = a.M[hyCol + z * nxy];
-    }
-    const RT q = ok && a.lightsOn ? (RT)a.Q[i] : (RT)0;
-    __syncthreads();  // the previous plane's readers are done
-    sT[ty + 1][tx + 1] = tHere;
-    sM[ty + 1][tx + 1] = (uint8_t)mHere;
-    if (hxOk) {
-      sT[ty + 1][sxh] = hxT;
-      sM[ty + 1][sxh] = (uint8_t)hxM;
-    }
-    if (hyOk) {
-      sT[syh][tx + 1] = hyT;
-      sM[syh][tx + 1] = (uint8_t)hyM;
-    }
-    __syncthreads();
+    const Side next = load_side(z + 1);
+    const RT tNext = ldT(min(z + 2, nz - 1), oP);
+    const unsigned mNext = ldM(min(z + 2, nz - 1), oP);
+    RT tl = lane_before(tHere), tr = lane_after(tHere);
+    unsigned ml = lane_before(mHere), mr = lane_after(mHere);
+    if (first) tl = here.e, ml = here.me;
+    if (last) tr = here.e, mr = here.me;
+    if (noL) tl = tHere;
+    if (noR) tr = tHere;
+    const unsigned row0 = mHere * (unsigned)sizeof(RT), row1 = row0 + axis, row2 = row1 + axis;
+    auto cf = [&](unsigned row, unsigned m) { return *(const RT*)(cT + (__umul24(m, pitch) + row)); };
+    const RT cl = cf(row0, ml), cr = cf(row0, mr), cym = cf(row1, here.mym), cyp = cf(row1, here.myp), czm = cf(row2, mBelow), czp = cf(row2, mAbove);
+    RT dTdt = (RT)here.q;
+    dTdt += (tl - tHere) * cl;
+    dTdt += (tr - tHere) * cr;
+    dTdt += (here.ym - tHere) * cym;
+    dTdt += (here.yp - tHere) * cyp;
+    dTdt += (tBelow - tHere) * czm;
+    dTdt += (tAbove - tHere) * czp;
+    if (sideFrozen || (a.sinked && (z == 0 || z == nz - 1))) dTdt = 0;
+    const RT t = tHere + dt * dTdt;
     if (ok) {
-      RT dTdt = 0;
-      if (!frozen(a, x, y, z)) {
-        dTdt = a.lightsOn ? q : (RT)0;
-        if (x != 0) dTdt += (sT[ty + 1][tx] - tHere) * coef(cT, nM, mHere, (int)sM[ty + 1][tx], 0);
-        if (x != nx - 1) dTdt += (sT[ty + 1][tx + 2] - tHere) * coef(cT, nM, mHere, (int)sM[ty + 1][tx + 2], 0);
-        if (y != 0) dTdt += (sT[ty][tx + 1] - tHere) * coef(cT, nM, mHere, (int)sM[ty][tx + 1], 1);
-        if (y != ny - 1) dTdt += (sT[ty + 2][tx + 1] - tHere) * coef(cT, nM, mHere, (int)sM[ty + 2][tx + 1], 1);
-        if (z != 0) dTdt += (tBelow - tHere) * coef(cT, nM, mHere, mBelow, 2);
-        if (z != nz - 1) dTdt += (tAbove - tHere) * coef(cT, nM, mHere, mAbove, 2);
-      }
-      const RT t = tHere + dt * dTdt;
-      a.T2[i] = t;
+      *(RT*)((char*)(a.T2 + (int64_t)z * nxy) + (OFF)(oP * (OFF)sizeof(RT))) = t;
       if (a.calcDamage && L.E[mHere] != 0)
-        a.Om[i] += dt * (RT)exp(L.logA[mHere] - L.E[mHere] / (a.Rgas * ((t + tHere) / 2 + a.czero)));
-      run.add(mHere, (double)t, L.maxKey);
+        a.Om[(int64_t)z * nxy + p] += dt * (RT)exp(L.logA[mHere] - L.E[mHere] / (a.Rgas * ((t + tHere) / 2 + a.czero)));
+      run.add((int)mHere, (double)t, L.maxKey);
     }
     tBelow = tHere;
     mBelow = mHere;
     tHere = tAbove;
     mHere = mAbove;
+    tAbove = tNext;
+    mAbove = mNext;
+    here = next;
   }
-  run.flush(L.maxKey);
   fold_lds_max(L.maxKey, a.maxKey, a.nM);
 }
 
@@ -1476,9 +1485,15 @@ int halloc(HeatBuf& b, size_t bytes) {
 
 template <typename RT>
 void launch_explicit(mcm_heat_plan* P, const HeatArgs<RT>& a, int zr) {
-  const unsigned ge = (unsigned)(((P->nx + kTileX - 1) / kTileX) * ((P->ny + kTileY - 1) / kTileY) * ((P->nz + zr - 1) / zr));
-  if (P->nM * P->nM * 3 <= kLdsCoef) hipLaunchKernelGGL((heat_explicit_tile<RT, true>), dim3(ge), dim3(kTileX * kTileY), 0, P->stream, a, zr);
-  else hipLaunchKernelGGL((heat_explicit_tile<RT, false>), dim3(ge), dim3(kTileX * kTileY), 0, P->stream, a, zr);
+  const int64_t nxy = (int64_t)P->nx * P->ny;
+  const unsigned ge = (unsigned)((nxy + kHeatTPB - 1) / kHeatTPB * ((P->nz + zr - 1) / zr));
+  auto go = [&](auto off) {
+    using OFF = decltype(off);
+    if (P->nM * P->nM * 3 <= kLdsCoef) hipLaunchKernelGGL((heat_explicit_march<RT, true, OFF>), dim3(ge), dim3(kHeatTPB), 0, P->stream, a, zr);
+    else hipLaunchKernelGGL((heat_explicit_march<RT, false, OFF>), dim3(ge), dim3(kHeatTPB), 0, P->stream, a, zr);
+  };
+  if (nxy < ((int64_t)1 << 28)) go(uint32_t());
+  else go(uint64_t());
 }
 
 template <typename RT>
@@ -1508,10 +1523,11 @@ HeatArgs<RT> make_args(mcm_heat_plan* P, double dt, int lightsOn) {
 }
 
 // The explicit stencil's best run of z planes per workgroup depends on how
-// the workgroup count fills the GPU (measured, ms/step at 100^3 / 160^3 /
-// 200^3 / 256^3: 8 planes 0.0189 / 0.0446 / 0.0792 / 0.1272, 16 planes
-// 0.0232 / 0.0375 / 0.0628 / 0.1095, 32 planes 0.0409 / 0.0501 / 0.0561 /
-// 0.1175), so each explicit plan times a few candidate runs once at
+// the workgroup count fills the GPU (measured, us/step at 100^3 / 200^3 /
+// 225x190x171 / 256x256x120: 8 planes 11.7 / 43.8 / 40.7 / 41.3, 12 planes
+// 13.7 / 43.1 / 37.6 / 39.7, 16 planes 16.6 / 41.1 / 40.5 / 41.3, 24 planes
+// 21.2 / 50.1 / 48.8 / 37.6, 32 planes 27.8 / 42.8 / 39.2 / 38.7), so each
+// explicit plan times a few candidate runs once at
 // creation.  The trial steps read the initial state and write only the
 // other state buffer (overwritten by the first real step), a scratch damage
 // field (the DG-ADI work buffer, unused by this scheme) and scratch maxima;
