@@ -15,7 +15,8 @@
 // chunks of a line; along x a wavefront holds contiguous voxels, along y and z
 // a workgroup holds 16 neighbouring lines in registers.  FP32 (the reference's
 // arithmetic) and longer lines: one lane per line running the Thomas
-// recurrence over blocks of loaded elements.
+// recurrence over blocks of loaded elements; FP32 lines of up to 420 voxels run
+// it on lines staged in LDS.
 // The explicit (forward Euler) scheme is one kernel per step.
 //
 // Arithmetic follows the reference's expressions (built without FMA
@@ -72,6 +73,7 @@ struct HeatArgs {
   const RT* T1;          // temperature at the start of the step
   RT* T2;                // result (and intermediate) of the step
   RT* B;                 // Thomas scratch: forward-eliminated diagonal
+  float* fac[3];         // FP32: eliminated diagonals of the x, y and z lines for this dt
   RT* Om;                // damage integral (calcDamage)
   unsigned long long* maxKey;  // [nM] order_key of the running maximum
   // sensor record of T1 (the state before the step), written by the first
@@ -143,6 +145,14 @@ __device__ inline void fold_lds_max(unsigned long long* s, unsigned long long* g
   __syncthreads();
   for (int k = threadIdx.x; k < nM; k += blockDim.x)
     if (s[k] > g[k]) atomicMax(&g[k], s[k]);
+}
+
+// Workgroup b of n, renumbered so that each of the 8 XCDs (which take
+// workgroups in turn) works on consecutive ones and finds its neighbours'
+// data in its own L2.
+__device__ inline int xcd_contiguous(int b, int n) {
+  const int q = n >> 3, r = n & 7, x = b & 7;
+  return x * q + min(x, r) + (b >> 3);
 }
 
 enum : int { SWEEP_X = 0, SWEEP_Y = 1, SWEEP_Z = 2 };
@@ -319,6 +329,272 @@ __device__ void sweep_line(const HeatArgs<RT>& a, const RT* cT, const HeatLds<RT
 }
 
 constexpr int kSweepU = 8;
+
+// FP32 sweeps of lines of up to 420 voxels.  The reference's recurrence is
+// sequential along a line and is kept operation for operation, so its length
+// cannot be cut; what a lane per line loses is the latency of its loads and
+// the few lanes (100^3: 157 wavefronts for 256 CUs).  Here a workgroup takes TL
+// lines: all its threads compute the right-hand sides and the rows'
+// coefficients voxel by voxel (coalesced) into LDS, TL lanes run the recurrence
+// there, and all threads write the lines back with the damage and maxima.
+// 100^3: 53 us a step (three sweeps; 390 with a lane per line), of which 30
+// remain without the recurrences.  Rows are read a group ahead of the recurrence
+// (70 us when each group waited for its own reads).
+// TL: as many lines (32, 16, 8) as fit four numbers per voxel into 54 KB.
+constexpr int kLine32Floats = 54 * 1024 / 16;
+inline int line32_lines(int n) {
+  const int pitch = n | 1;
+  return 32 * pitch <= kLine32Floats ? 32 : 16 * pitch <= kLine32Floats ? 16 : 8 * pitch <= kLine32Floats ? 8 : 0;
+}
+
+// The eliminated diagonal depends on the media and dt only: LINES_BUILD computes
+// it into a.fac, LINES_FACTORED reads it, which leaves a multiply and a
+// subtraction per row in the downward recurrence (LINES_PLAIN computes it on
+// the way, a division and five more operations per row).
+enum : int { LINES_PLAIN = 0, LINES_FACTORED = 1, LINES_BUILD = 2 };
+constexpr int kLine32TPB = 512;
+
+// Runs visit(k, load(k)) for k = from, from + step, ... up to and without `end`
+// (step 1 or -1), loading a group of rows while the group before is visited: the
+// LDS latency stays off the recurrence's chain.
+template <class Load, class Visit>
+__device__ inline void row_groups(int from, int end, int step, Load&& load, Visit&& visit) {
+  constexpr int V = 8;
+  const int count = (end - from) * step;
+  int k = from, left = count;
+  if (left >= V) {
+    decltype(load(0)) cur[V], next[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) cur[v] = load(k + v * step);
+    for (; left >= V; left -= V, k += V * step) {
+      const int ahead = left >= 2 * V ? k + V * step : k;  // the last whole group reloads itself
+#pragma unroll
+      for (int v = 0; v < V; ++v) next[v] = load(ahead + v * step);
+#pragma unroll
+      for (int v = 0; v < V; ++v) visit(k + v * step, cur[v]);
+#pragma unroll
+      for (int v = 0; v < V; ++v) cur[v] = next[v];
+    }
+  }
+  for (; left > 0; --left, k += step) visit(k, load(k));
+}
+
+template <int KIND, int TL, int MODE, bool LDS_COEF>
+__global__ void __launch_bounds__(kLine32TPB) heat_sweep_lines32(HeatArgs<float> a) {
+  extern __shared__ float sLine[];
+  __shared__ HeatLds<float> L;
+  constexpr bool X = KIND == SWEEP_X, Z = KIND == SWEEP_Z;
+  constexpr bool FACTORED = MODE == LINES_FACTORED, BUILD = MODE == LINES_BUILD;
+  constexpr int d = KIND;
+  if (X && !BUILD) step_sensors(a);
+  (void)stage_tables(a, L);
+  const float* cT = LDS_COEF ? L.c : a.c;  // LDS or global, never a generic pointer
+  const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = nx * ny, nM = a.nM;
+  const int n = X ? nx : KIND == SWEEP_Y ? ny : nz, st = X ? 1 : KIND == SWEEP_Y ? nx : nxy;
+  const int pitch = n | 1;  // odd: the recurrence's lanes fall into different banks
+  float* const sR = sLine;                    // right-hand side, then the solution
+  float* const sB = sLine + TL * pitch;       // eliminated diagonal (not FACTORED: dt/2 c(m, before) first)
+  float* const sP = sLine + 2 * TL * pitch;   // dt/2 c(m, after)
+  float* const sS = sLine + 3 * TL * pitch;   // c(before, m); FACTORED: the row's multiplier
+  const int blk = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int tiles = (nx + TL - 1) / TL;  // y and z sweeps: TL consecutive x at one z (y)
+  const int o = X ? 0 : blk / tiles, c0 = X ? blk * TL : (blk - o * tiles) * TL;
+  const int cols = min(TL, (X ? ny * nz : nx) - c0);
+  const float dt = a.dt;
+  const bool sk = a.sinked;
+  float* __restrict__ fac = a.fac[KIND];
+  auto line_frozen = [&](int c) {
+    if (!sk) return false;
+    if (X) {
+      const int y = (c0 + c) % ny, z = (c0 + c) / ny;
+      return y == 0 || y == ny - 1 || z == 0 || z == nz - 1;
+    }
+    const int x = c0 + c, nOther = KIND == SWEEP_Y ? nz : ny;
+    return x == 0 || x == nx - 1 || o == 0 || o == nOther - 1;
+  };
+  // G threads a line, each G voxels apart (a thread stays on its line, so its
+  // coordinates are worked out once); consecutive threads hold consecutive x
+  constexpr int G = kLine32TPB / TL;
+  const int cRaw = X ? (int)threadIdx.x / G : (int)threadIdx.x % TL, kk = X ? (int)threadIdx.x % G : (int)threadIdx.x / TL;
+  const bool mine = cRaw < cols;
+  const int c = mine ? cRaw : cols - 1;
+  const int i0 = X ? (c0 + c) * nx : KIND == SWEEP_Y ? c0 + c + o * nxy : c0 + c + o * nx;
+  const bool lf = line_frozen(c);
+  const int yLine = X ? (c0 + c) % ny : 0, zLine = X ? (c0 + c) / ny : 0;
+  const int oym = yLine > 0 ? -nx : 0, oyp = yLine < ny - 1 ? nx : 0, ozm = zLine > 0 ? -nxy : 0, ozp = zLine < nz - 1 ? nxy : 0;
+  // all lookups and loads are done (clamped) and unwanted terms dropped by
+  // selects, so that the loads of an unrolled group are in flight together
+  constexpr int U = 4;
+  for (int k0 = kk; k0 < n; k0 += U * G) {
+    float T[U], Tl[U], Tr[U], R0[U], Ta[U], Tb[U], Tc[U], Td[U], Q[U], F[U], Fl[U];
+    int M[U], Ml[U], Mr[U], Ma[U], Mb[U], Mc[U], Md[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(k0 + u * G, n - 1), i = i0 + k * st, il = k > 0 ? i - st : i, ir = k < n - 1 ? i + st : i;
+      M[u] = a.M[i], Ml[u] = a.M[il], Mr[u] = a.M[ir];
+      if (FACTORED) F[u] = fac[i], Fl[u] = fac[il];
+      if (BUILD) continue;
+      T[u] = a.T1[i], Tl[u] = a.T1[il], Tr[u] = a.T1[ir];
+      if (X) {
+        Ta[u] = a.T1[i + oym], Tb[u] = a.T1[i + oyp], Tc[u] = a.T1[i + ozm], Td[u] = a.T1[i + ozp];
+        Ma[u] = a.M[i + oym], Mb[u] = a.M[i + oyp], Mc[u] = a.M[i + ozm], Md[u] = a.M[i + ozp];
+        Q[u] = a.Q[i];
+      } else {
+        R0[u] = a.T2[i];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u * G;
+      if (!mine || k >= n) break;
+      const int m = M[u], q = c * pitch + k;
+      const float cl = coef(cT, nM, m, Ml[u], d), cr = coef(cT, nM, m, Mr[u], d);
+      sP[q] = dt / 2 * cr;
+      if (FACTORED) {
+        sB[q] = F[u];
+        sS[q] = -(dt / 2 * cl) / Fl[u];
+      } else {
+        sB[q] = dt / 2 * cl;
+        sS[q] = coef(cT, nM, Ml[u], m, d);
+      }
+      if (BUILD) continue;
+      const bool fz = lf || (sk && (k == 0 || k == n - 1));
+      if (X) {
+        float dTdt = a.lightsOn ? Q[u] : 0.f;
+        if (k != 0) dTdt += (Tl[u] - T[u]) * cl / 2;
+        if (k != n - 1) dTdt += (Tr[u] - T[u]) * cr / 2;
+        if (yLine != 0) dTdt += (Ta[u] - T[u]) * coef(cT, nM, m, Ma[u], 1);
+        if (yLine != ny - 1) dTdt += (Tb[u] - T[u]) * coef(cT, nM, m, Mb[u], 1);
+        if (zLine != 0) dTdt += (Tc[u] - T[u]) * coef(cT, nM, m, Mc[u], 2);
+        if (zLine != nz - 1) dTdt += (Td[u] - T[u]) * coef(cT, nM, m, Md[u], 2);
+        sR[q] = T[u] + dt * (fz ? 0.f : dTdt);
+      } else {
+        float dTdt = 0;
+        if (k != 0) dTdt -= (Tl[u] - T[u]) * cl / 2;
+        if (k != n - 1) dTdt -= (Tr[u] - T[u]) * cr / 2;
+        sR[q] = fz ? R0[u] : R0[u] + dt * dTdt;
+      }
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < cols && !line_frozen(threadIdx.x)) {
+    float* const r = sR + threadIdx.x * pitch;
+    float* const b = sB + threadIdx.x * pitch;
+    const float* const p = sP + threadIdx.x * pitch;
+    const float* const q = sS + threadIdx.x * pitch;
+    const int n1 = sk ? n - 1 : n;  // rows 1 .. n1-1 are eliminated; with frozen ends the last row stands
+    float tprev = BUILD ? 0.f : r[0], bprev = 1;
+    if (!FACTORED) {
+      if (!sk && n > 1) bprev += p[0];
+      b[0] = bprev;
+    }
+    struct Row {
+      float r, b, p, q;
+    };
+    auto row_at = [&](int k) {
+      Row w{};
+      w.q = q[k];
+      if (!BUILD) w.r = r[k];
+      if (!FACTORED) w.b = b[k], w.p = p[k];
+      return w;
+    };
+    auto eliminate = [&](int k, const Row& row) {
+      float w = row.q;
+      if (!FACTORED) {
+        float bb = 1;
+        if (k < n - 1) bb += row.p;
+        bb += row.b;
+        w = -row.b / bprev;
+        if (k > 1 || !sk) bb += w * dt / 2 * row.q;
+        bprev = bb;
+        b[k] = bprev;
+      }
+      if (!BUILD) {
+        tprev = row.r - w * tprev;
+        r[k] = tprev;
+      }
+    };
+    row_groups(1, n1, 1, row_at, eliminate);
+  }
+  // Back substitution divides by the eliminated diagonal b in every row, and a
+  // correctly rounded division is the longest part of the recurrence's chain.
+  // With y = 1 / b rounded to nearest, computed here by all threads, the chain
+  // is q = a y and two corrections q += (a - b q) y with fused multiply-adds,
+  // which round to the same bits as a / b (Markstein, "Computation of elementary
+  // functions on the IBM RISC System/6000 processor", 1990) as long as nothing
+  // leaves the normal range.  The rows keep the range of |a| on the way; a line
+  // that left it is repeated with divisions.
+  const bool divides = (int)threadIdx.x < cols && !line_frozen(threadIdx.x);
+  if (!BUILD) {
+    __syncthreads();
+    for (int k = kk; k < n; k += G) sS[c * pitch + k] = 1.0f / sB[c * pitch + k];
+    __syncthreads();
+  }
+  if (!BUILD && divides) {
+    const float* const r = sR + threadIdx.x * pitch;
+    const float* const b = sB + threadIdx.x * pitch;
+    const float* const p = sP + threadIdx.x * pitch;
+    float* const x = sS + threadIdx.x * pitch;  // y, then the solution
+    // the last row (no term from beyond; frozen: stands), then the others that
+    // are not frozen
+    const int kEnd = sk ? 1 : 0;
+    float lo = 1.f, hi = 1.f, bhi = 1.f;
+    float xnext = sk ? r[n - 1] : (r[n - 1] + 0.f) / b[n - 1];
+    x[n - 1] = xnext;
+    struct Row {
+      float r, b, p, y;
+    };
+    auto row_at = [&](int k) { return Row{r[k], b[k], p[k], x[k]}; };
+    auto substitute = [&](int k, const Row& row) {
+      const float t = row.r + row.p * xnext;
+      float v = t * row.y;
+      v = fmaf(fmaf(-row.b, v, t), row.y, v);
+      v = fmaf(fmaf(-row.b, v, t), row.y, v);
+      xnext = v;
+      x[k] = v;
+      lo = fminf(lo, t == 0.f ? 1.f : fabsf(t));
+      hi = fmaxf(hi, fabsf(t));
+      bhi = fmaxf(bhi, row.b);
+    };
+    row_groups(n - 2, kEnd - 1, -1, row_at, substitute);
+    if (!(lo >= 0x1p-100f && hi <= 0x1p100f && bhi <= 0x1p20f)) {
+      xnext = x[n - 1];
+      for (int k = n - 2; k >= kEnd; --k) {
+        xnext = (r[k] + p[k] * xnext) / b[k];
+        x[k] = xnext;
+      }
+    }
+    if (sk) x[0] = r[0];
+  }
+  __syncthreads();
+  MaxRun run;
+  for (int k0 = kk; k0 < n; k0 += U * G) {
+    int m[U];
+    float t0[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + min(k0 + u * G, n - 1) * st;
+      if (Z && !BUILD) m[u] = a.M[i], t0[u] = a.T1[i];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u * G, i = i0 + k * st, q = c * pitch + k;
+      if (!mine || k >= n) break;
+      if (BUILD) {
+        fac[i] = sB[q];
+        continue;
+      }
+      const float t = lf ? sR[q] : sS[q];
+      a.T2[i] = t;
+      if (Z) {
+        if (a.calcDamage && L.E[m[u]] != 0)
+          a.Om[i] += dt * (float)exp(L.logA[m[u]] - L.E[m[u]] / (a.Rgas * ((t + t0[u]) / 2 + a.czero)));
+        run.add(m[u], (double)t, L.maxKey);
+      }
+    }
+  }
+  if (Z && !BUILD) fold_lds_max(L.maxKey, a.maxKey, nM);
+}
 
 // substeps 1a + 1b (finiteElementHeatPropagator.c:288-312, :352-389): lane per (y, z) x-line
 template <typename RT, bool LDS_COEF>
@@ -515,14 +791,6 @@ __device__ inline void line_solve(const double (&a)[S], const double (&b)[S], co
 // = T1 - u, and likewise along z).  The y and z sweeps then need neither u's
 // stencil nor u itself before the end, and rounding enters relative to the
 // increment.  Frozen voxels have increment 0.
-
-// Workgroup b of n, renumbered so that each of the 8 XCDs (which take
-// workgroups in turn) works on consecutive ones and finds its neighbours'
-// data in its own L2.
-__device__ inline int xcd_contiguous(int b, int n) {
-  const int q = n >> 3, r = n & 7, x = b & 7;
-  return x * q + min(x, r) + (b >> 3);
-}
 
 // substeps 1a + 1b in FP64, a (y, z) x-line per W lanes: lane l holds voxels
 // x = l*S .. l*S+S-1, so every load of the wavefront is contiguous.  Bound by
@@ -1417,6 +1685,7 @@ struct HeatGraph {
   double dt = 0;
   int lightsOn = 0;
   const void *T1 = nullptr, *sensors = nullptr;
+  bool factored = false;  // the captured FP32 sweeps read the line factors
 };
 
 struct mcm_heat_plan {
@@ -1434,6 +1703,10 @@ struct mcm_heat_plan {
   bool interrupted = false;
   int (*interrupt)(void) = nullptr;
   HeatBuf M, Q, c, logA, E, T1, T2, B, Om, maxKey, sIdx, sW, sensors, stage32, stage64, stepDev;
+  HeatBuf fac[3];             // FP32 line factors (ensure_factors) for facDt
+  bool facReady = false;
+  double facDt = 0;
+  bool factored(double dt) const { return facReady && facDt == dt; }
   double constR = 0, constC = 0;
   int64_t graphSteps = 32;    // steps per captured graph (0: launch every step)
   std::vector<HeatGraph> graphs;
@@ -1461,6 +1734,7 @@ struct mcm_heat_group {
     std::vector<double> dt;
     std::vector<int> lightsOn;
     std::vector<const void*> T1, sensors;
+    std::vector<bool> factored;
   };
   std::vector<Graph> graphs;
   void drop_graphs() {
@@ -1519,6 +1793,8 @@ HeatArgs<RT> make_args(mcm_heat_plan* P, double dt, int lightsOn) {
   a.B = (RT*)P->B.p;
   a.Om = (RT*)P->Om.p;
   a.maxKey = (unsigned long long*)P->maxKey.p;
+  if (P->factored(dt))
+    for (int d = 0; d < 3; ++d) a.fac[d] = (float*)P->fac[d].p;
   return a;
 }
 
@@ -1619,6 +1895,55 @@ int record_sensors(mcm_heat_plan* P, int64_t col) {
   return MCM_OK;
 }
 
+// FP32 sweep along axis KIND through LDS (build: its factors); false when the
+// line is too long.
+template <int KIND>
+bool launch_lines32(mcm_heat_plan* P, const HeatArgs<float>& a, bool build = false) {
+  const int n = KIND == SWEEP_X ? P->nx : KIND == SWEEP_Y ? P->ny : P->nz, tl = line32_lines(n);
+  if (!tl) return false;
+  const size_t lds = (size_t)tl * (n | 1) * 16;
+  auto go = [&](auto TL) {
+    constexpr int T = decltype(TL)::value;
+    const dim3 g(KIND == SWEEP_X ? (unsigned)((P->ny * P->nz + T - 1) / T)
+                                 : (unsigned)(((P->nx + T - 1) / T) * (KIND == SWEEP_Y ? P->nz : P->ny)));
+    const dim3 b(kLine32TPB);
+    if (build) hipLaunchKernelGGL((heat_sweep_lines32<KIND, T, LINES_BUILD, true>), g, b, lds, P->stream, a);
+    else if (a.fac[KIND]) hipLaunchKernelGGL((heat_sweep_lines32<KIND, T, LINES_FACTORED, true>), g, b, lds, P->stream, a);
+    else if (P->nM * P->nM * 3 <= kLdsCoef) hipLaunchKernelGGL((heat_sweep_lines32<KIND, T, LINES_PLAIN, true>), g, b, lds, P->stream, a);
+    else hipLaunchKernelGGL((heat_sweep_lines32<KIND, T, LINES_PLAIN, false>), g, b, lds, P->stream, a);
+  };
+  if (tl == 32) go(std::integral_constant<int, 32>());
+  else if (tl == 16) go(std::integral_constant<int, 16>());
+  else go(std::integral_constant<int, 8>());
+  return true;
+}
+
+// The FP32 line factors for dt, built when a run of at least kFactorSteps steps
+// starts with another dt than the last such run's (building them costs about
+// what one step gains three times over).  Runs without them compute them row
+// by row.  Not called while a stream captures: captured steps read the
+// buffers, which every run refills for its own dt before its replays.
+constexpr int64_t kFactorSteps = 4;
+int ensure_factors(mcm_heat_plan* P, int64_t steps, double dt) {
+  if (!P->fp32 || P->explicitScheme) return MCM_OK;
+  if (P->factored(dt)) return MCM_OK;
+  if (steps < kFactorSteps || P->nM * P->nM * 3 > kLdsCoef) {
+    P->facReady = false;
+    return MCM_OK;
+  }
+  const int n[3] = {P->nx, P->ny, P->nz};
+  for (int d = 0; d < 3; ++d)
+    if (line32_lines(n[d]) && !P->fac[d].p) MCM_HIP(hipMalloc(&P->fac[d].p, (size_t)P->L * 4));
+  P->facReady = true;
+  P->facDt = dt;
+  const HeatArgs<float> a = make_args<float>(P, dt, 0);
+  launch_lines32<SWEEP_X>(P, a, true);
+  launch_lines32<SWEEP_Y>(P, a, true);
+  launch_lines32<SWEEP_Z>(P, a, true);
+  MCM_HIP(hipGetLastError());
+  return MCM_OK;
+}
+
 // Lane-per-line y (AXIS 1) or z (AXIS 2) sweep, coefficients in LDS when
 // they fit.
 template <typename RT, int AXIS>
@@ -1650,6 +1975,8 @@ void launch_sweep_x(mcm_heat_plan* P, const HeatArgs<RT>& a, unsigned gx) {
       });
       return;
     }
+  } else if (launch_lines32<SWEEP_X>(P, a)) {
+    return;
   }
   if (P->nM * P->nM * 3 <= kLdsCoef) hipLaunchKernelGGL((heat_sweep_x<RT, true>), dim3(gx), dim3(kHeatTPB), 0, P->stream, a);
   else hipLaunchKernelGGL((heat_sweep_x<RT, false>), dim3(gx), dim3(kHeatTPB), 0, P->stream, a);
@@ -1674,10 +2001,10 @@ void launch_sweep_yz(mcm_heat_plan* P, const HeatArgs<RT>& a, unsigned gy, unsig
     else launch_lane_sweep<RT, 1>(P, a, gy);
     if (wave_line(P->nz)) launch_yz_wave<SWEEP_Z>(P, a, P->nz);
     else launch_lane_sweep<RT, 2>(P, a, gz);
-    return;
+  } else {
+    if (!launch_lines32<SWEEP_Y>(P, a)) launch_lane_sweep<RT, 1>(P, a, gy);
+    if (!launch_lines32<SWEEP_Z>(P, a)) launch_lane_sweep<RT, 2>(P, a, gz);
   }
-  launch_lane_sweep<RT, 1>(P, a, gy);
-  launch_lane_sweep<RT, 2>(P, a, gz);
 }
 
 // The kernels of one time step on the plan's stream; swaps the state buffers.
@@ -1718,7 +2045,7 @@ void enqueue_graph_steps(mcm_heat_plan* P, int64_t K, double dt, int lightsOn) {
 template <typename RT>
 int step_graph(mcm_heat_plan* P, int64_t K, double dt, int lightsOn, hipGraphExec_t* out) {
   for (HeatGraph& g : P->graphs)
-    if (g.steps == K && g.dt == dt && g.lightsOn == lightsOn && g.T1 == P->T1.p && g.sensors == P->sensors.p) {
+    if (g.steps == K && g.dt == dt && g.lightsOn == lightsOn && g.T1 == P->T1.p && g.sensors == P->sensors.p && g.factored == P->factored(dt)) {
       *out = g.exec;
       return MCM_OK;
     }
@@ -1750,6 +2077,7 @@ int step_graph(mcm_heat_plan* P, int64_t K, double dt, int lightsOn, hipGraphExe
   g.lightsOn = lightsOn;
   g.T1 = P->T1.p;
   g.sensors = P->sensors.p;
+  g.factored = P->factored(dt);
   P->graphs.push_back(g);
   *out = exec;
   return MCM_OK;
@@ -1759,6 +2087,7 @@ template <typename RT>
 int advance(mcm_heat_plan* P, int64_t steps, double dt, int lightsOn) {
   int rc = ensure_sensor_capacity(P, P->stepsDone + steps + 1);
   if (rc) return rc;
+  if ((rc = ensure_factors(P, steps, dt))) return rc;
   int64_t n = 0;
   // runs of K steps replay one captured graph (one launch instead of 2-4
   // per step); the interrupt is polled between replays
@@ -2030,6 +2359,7 @@ int mcm_heat_group_advance(mcm_heat_group* G, int64_t steps, const double* dt, c
     int rc = ensure_sensor_capacity(G->plans[i], G->plans[i]->stepsDone + steps + 1);
     if (rc) return rc;
     if (G->plans[i]->nS && !G->plans[i]->stepDev.p) MCM_HIP(hipMalloc(&G->plans[i]->stepDev.p, sizeof(long long)));
+    if ((rc = ensure_factors(G->plans[i], steps, dt[i]))) return rc;
   }
   const int64_t K = stepsPerGraph & ~(int64_t)1;
   int64_t done = 0;
@@ -2038,7 +2368,8 @@ int mcm_heat_group_advance(mcm_heat_group* G, int64_t steps, const double* dt, c
     for (mcm_heat_group::Graph& c : G->graphs) {
       bool same = c.steps == K;
       for (size_t i = 0; same && i < n; ++i)
-        same = c.dt[i] == dt[i] && c.lightsOn[i] == (lightsOn[i] != 0) && c.T1[i] == G->plans[i]->T1.p && c.sensors[i] == G->plans[i]->sensors.p;
+        same = c.dt[i] == dt[i] && c.lightsOn[i] == (lightsOn[i] != 0) && c.T1[i] == G->plans[i]->T1.p && c.sensors[i] == G->plans[i]->sensors.p &&
+               c.factored[i] == G->plans[i]->factored(dt[i]);
       if (same) g = &c;
     }
     if (!g) {
@@ -2081,6 +2412,7 @@ int mcm_heat_group_advance(mcm_heat_group* G, int64_t steps, const double* dt, c
         c.lightsOn.push_back(lightsOn[i] != 0);
         c.T1.push_back(G->plans[i]->T1.p);
         c.sensors.push_back(G->plans[i]->sensors.p);
+        c.factored.push_back(G->plans[i]->factored(dt[i]));
       }
       G->graphs.push_back(std::move(c));
       g = &G->graphs.back();

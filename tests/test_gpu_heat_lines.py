@@ -61,3 +61,48 @@ def test_many_media_read_coefficients_from_memory(api):
     ref = OL.oracle_heat(T0, Om0, P, variant=OL.HEAT_FP64_DGADI)
     assert np.max(np.abs(T64 / ref["T_f64"] - 1)) <= 4e-12
     np.testing.assert_allclose(Om64, ref["Omega_f64"], rtol=1e-9, atol=0)
+
+
+# the FP32 sweeps repeat the reference's operations one by one: same bits as the
+# oracle but for the damage's exp
+@pytest.mark.parametrize("steps", [2, 6])  # without and with the line factors
+@pytest.mark.parametrize("n", [1, 2, 3, 103, 104, 106, 210, 211, 420, 421])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_fp32_line_lengths(api, axis, n, steps):
+    shape = [17, 3, 4]
+    shape[axis] = n
+    if axis != 0:
+        shape[0] = 35  # a full and a partly filled group of 32, 16 or 8 lines
+    T0, Om0, P = line_case(tuple(shape), 0.3, seed=n, steps=steps, sinked=n % 2)
+    print(f"[gpu-heat-lines32] {shape} steps {steps}", flush=True)
+    T, Om, _, mx = api.finiteElementHeatPropagator(T0, Om0, P, precision="fp32")
+    ref = OL.oracle_heat(T0, Om0, P, variant=OL.HEAT_FP32_DGADI)
+    np.testing.assert_array_equal(T, ref["T"])
+    np.testing.assert_array_equal(mx, ref["maxMediaTemps"])
+    np.testing.assert_allclose(Om, ref["Omega"], rtol=1e-5)
+
+
+def test_fp32_factors_follow_the_time_step(api):
+    """Runs of alternating time steps and lengths, replayed graphs and a group:
+    the line factors in memory are always those of the run's own dt."""
+    T0, Om0, P = line_case((35, 21, 18), 0.3, steps=1)
+    runs = [(8, 0.3, 1), (8, 0.1, 0), (8, 0.3, 1), (2, 0.1, 0), (2, 0.3, 1), (8, 0.1, 0)]
+    plain = api.HeatPlan(T0, Om0, P, precision="fp32", graph_steps=0)
+    graphs = api.HeatPlan(T0, Om0, P, precision="fp32", graph_steps=2)
+    grouped = api.HeatPlan(T0, Om0, P, precision="fp32", graph_steps=0)
+    other = api.HeatPlan(T0, Om0, P, precision="fp64", graph_steps=0)
+    group = api.HeatGroup([grouped, other], steps_per_graph=2)
+    T, Om = T0, Om0
+    for steps, dt, on in runs:
+        for _ in range(steps):  # one step a call: never factored
+            plain.advance(1, dt, on)
+        graphs.advance(steps, dt, on)
+        group.advance(steps, [dt, dt], [on, on])
+        Pr = dict(P, steps=steps, dt=dt, lightsOn=bool(on))
+        ref = OL.oracle_heat(T, Om, Pr, variant=OL.HEAT_FP32_DGADI)
+        T, Om = ref["T"], ref["Omega"]
+        for plan in (plain, graphs, grouped):
+            np.testing.assert_array_equal(plan.download(f64=False)["T"], T)
+    group.close()
+    for plan in (plain, graphs, grouped, other):
+        plan.close()
