@@ -202,7 +202,8 @@ int mcm_mc_plan_destroy(mcm_mc_plan *plan);
 /* Launch tuning (no reference counterpart).  The fluence accumulates into 1,
  * 2, 4 or 8 FP64 copies, one per group of the GPU's XCDs, summed before any
  * read: more copies relieve atomic contention on hot voxels (narrow beams),
- * fewer keep the working set small (broad beams).  Times one launch of
+ * fewer keep the working set small (broad beams).  A plan starts with the most
+ * copies that 256 MB hold.  Times one launch of
  * nPackets packets (0: 2^21) of wavelength iL per copy count (within a 2 GiB
  * budget), keeps the fewest copies within 10 % of the fastest trial, then
  * clears the plan's tallies and counters.

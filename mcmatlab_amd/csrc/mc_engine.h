@@ -85,65 +85,62 @@ struct PacketEngine {
     }
   }
 
-  // deposit of the sub-step, then checkEscape + getNewVoxelProperties
-  // (propagatePhoton :1095-1110, MCmatlab.c:254-257).  The deposit (decided
-  // on the state before the escape check, as in the reference) goes to the
-  // sink only after the next voxel's medium index has been requested: a
-  // deposit that flushes the sink's merged value issues an atomic, and loads
-  // and atomics retire in order, so an atomic issued before the load would
-  // make every voxel change wait for the atomic's round trip.
+  // deposit of a sub-step into voxel P.j (decided on the state before the
+  // escape check, as in the reference)
   template <class Sink>
-  MCM_FN void finish_substep(float absorb, const McParams& p, const Medium* med, const uint8_t* cdf, Sink& sink) {
-    bool dep = false;
-    double dv = 0.0;
-    if (P.insideVolume && p.calcNFR) {
-      if (CRITERIA && replay) {
-        dep = true;
-        dv = (double)(replayW * absorb);
-      } else if (!(CRITERIA && p.evalAtEnd) && criteria_met(P, p)) {
-        dep = true;
-        dv = (double)absorb;
-      }
-    }
-    const int jOld = P.j;
-    if (!P.sameVoxel) {
-      const EscapeResult e = check_escape(P, p);
-      if constexpr (Sink::kDeferEscapes) {
-        if ((e.escaped && (p.useLC || p.farFieldRes)) || e.edgeFlux) sink.escape(P, e.escaped, e.edgeFlux, slot);
-      } else if (!replay) {
-        if (e.escaped) {
-          if (p.useLC) {
-            const int b = collector_bin(P, p);
-            if (b >= 0 && criteria_met(P, p)) {
-              sink.image_add(b, (double)P.weight);
-              sink.collected();
-            }
+  MCM_FN void deposit(float absorbed, const McParams& p, Sink& sink) {
+    if (!(P.insideVolume && p.calcNFR)) return;
+    if (CRITERIA && replay) sink.deposit(P.j, replayW * absorbed);
+    else if (!(CRITERIA && p.evalAtEnd) && criteria_met(P, p)) sink.deposit(P.j, absorbed);
+  }
+
+  // checkEscape + getNewVoxelProperties after a boundary was crossed into voxel
+  // jNew of medium mNew (propagatePhoton :1095-1110, MCmatlab.c:254-257)
+  template <class Sink>
+  MCM_FN void enter_voxel(int jNew, int mNew, const McParams& p, const Medium* med, const uint8_t* cdf, Sink& sink) {
+    const float x = P.i[0], y = P.i[1];
+    const EscapeResult e = check_escape(P, p);
+    if constexpr (Sink::kDeferEscapes) {
+      if ((e.escaped && (p.useLC || p.farFieldRes)) || e.edgeFlux) sink.escape(P, e.escaped, e.edgeFlux, slot);
+    } else if (!replay) {
+      if (e.escaped) {
+        if (p.useLC) {
+          const int b = collector_bin(P, p);
+          if (b >= 0 && criteria_met(P, p)) {
+            sink.image_add(b, (double)P.weight);
+            sink.collected();
           }
-          if (p.farFieldRes && criteria_met(P, p)) sink.farField(far_field_bin(P, p), (double)P.weight);
         }
-        if (e.edgeFlux && criteria_met(P, p)) {
-          int face;
-          const int idx = edge_flux_bin(P, p, &face);
-          if (face >= 0) sink.edge(face, idx, (double)P.weight);
-        }
+        if (p.farFieldRes && criteria_met(P, p)) sink.farField(far_field_bin(P, p), (double)P.weight);
       }
-      if (P.alive) {
-        P.j = voxel_of(p, P.i);
-        const int m = p.M[P.j];  // requested before the deposit's atomic
-        if (dep) sink.deposit(jOld, dv);
-        dep = false;
-        const Medium md = med[m];
-        P.mua = md.mua;
-        P.mus = md.mus;
-        P.g = md.g;
-        P.cdf = cdf[m];
+      if (e.edgeFlux && criteria_met(P, p)) {
+        int face;
+        const int idx = edge_flux_bin(P, p, &face);
+        if (face >= 0) sink.edge(face, idx, (double)P.weight);
       }
     }
-    if (dep) sink.deposit(jOld, dv);
+    if (!P.alive) return;
+    if (p.boundaryType == 3 && (P.i[0] != x || P.i[1] != y)) {  // wrapped to the other side
+      jNew = voxel_of(p, P.i);
+      mNew = p.M[jNew];
+    }
+    P.j = jNew;
+    const Medium md = med[mNew];
+    P.mua = md.mua;
+    P.mus = md.mus;
+    P.g = md.g;
+    P.cdf = cdf[mNew];
+  }
+
+  template <class Sink>
+  MCM_FN void next_state(const McParams& p, const Medium* med, const uint8_t* cdf, Sink& sink) {
     if (!P.alive) death(p, med, cdf, sink);
     else state = P.stepLeft > 0.f ? ST_MOVE : ST_SCATTER;
   }
 
+  // One sub-step.  The medium of the voxel entered is requested as soon as the
+  // position is known and used after the absorption and the deposit, whose
+  // arithmetic covers the load.
   template <class Sink>
   MCM_FN void do_move(const McParams& p, const Medium* med, const uint8_t* cdf, Sink& sink) {
     if (P.substeps >= kMaxSubsteps) {
@@ -152,21 +149,35 @@ struct PacketEngine {
       death(p, med, cdf, sink);
       return;
     }
-    const MoveResult mr = move<FRESNEL>(P, p, med);
-    if (FRESNEL && mr.fresnel) {
-      pendAbsorb = mr.absorb;
-      pendJ = mr.jNew;
-      pendM = mr.mNew;
-      state = ST_FRESNEL;
-    } else {
-      finish_substep(mr.absorb, p, med, cdf, sink);
+    const float s = advance(P, p);
+    int jNew = P.j, mNew = 0;
+    if (!P.sameVoxel) {
+      jNew = voxel_of(p, P.i);
+      mNew = p.M[jNew];
     }
+    const float absorbed = absorb(P, s);
+    if constexpr (!CRITERIA) deposit(absorbed, p, sink);
+    if (!P.sameVoxel) {
+      if (FRESNEL && P.ri != med[mNew].ri) {
+        pendAbsorb = absorbed;
+        pendJ = jNew;
+        pendM = mNew;
+        state = ST_FRESNEL;
+        return;
+      }
+      if (CRITERIA && p.criteriaActive) count_transition(P, p, med, mNew);
+    }
+    if constexpr (CRITERIA) deposit(absorbed, p, sink);
+    if (!P.sameVoxel) enter_voxel(jNew, mNew, p, med, cdf, sink);
+    next_state(p, med, cdf, sink);
   }
 
   template <class Sink>
   MCM_FN void do_fresnel(const McParams& p, const Medium* med, const uint8_t* cdf, Sink& sink) {
     fresnel(P, p, med, pendJ, pendM, R);
-    finish_substep(pendAbsorb, p, med, cdf, sink);
+    if constexpr (CRITERIA) deposit(pendAbsorb, p, sink);
+    enter_voxel(pendJ, pendM, p, med, cdf, sink);
+    next_state(p, med, cdf, sink);
   }
 
   template <class Sink>

@@ -20,10 +20,16 @@
 //   served together, which keeps SIMD occupancy high for the expensive
 //   scatter and interface code.
 //
-//   Per-medium optical constants live in LDS.  Deposits accumulate in a
-//   per-lane FP64 register while the packet stays in one voxel and go to the
-//   FP64 fluence grid with a hardware FP64 atomic add when it leaves (or
-//   dies).  Boundary, far-field and detector tallies are FP64 atomics too.
+//   Per-medium optical constants live in LDS.  Deposits are parked in LDS and
+//   added to the FP64 fluence grid, kept in bricks of voxels, with hardware
+//   FP64 atomics that many lanes of one packet share (DeferSink).  Boundary,
+//   far-field and detector tallies are FP64 atomics too.
+//
+//   What bounds it: 4 10^6 packets of a broad beam on 200^3 (1.3 10^9
+//   sub-steps) are 7.4 10^8 line requests of the atomics, which all go to
+//   memory (2.37 10^10/s at most: 31 ms), and 1.27 10^10 vector instructions
+//   (21 ms; the run without fluence takes 21.2 ms); 57.2 ms with one deposit
+//   per lane and instruction into rows of voxels, 35.7 ms now.
 //
 //   Deposition criteria evaluated at end of life (MCmatlab.c:262-264) are
 //   handled by replay instead of per-packet deposit records: when a packet
@@ -64,7 +70,7 @@ constexpr int kPlain = 0, kBatch = 1, kMulti = 2;
 // What the transport reads of a model that differs between the models of a
 // multi-grid launch (copied into the lane's parameters at each fetch).
 struct McGeom {
-  int n[3];
+  int n[3], nbx, nbxy;
   float d[3], inv_d[3];
   float tooOld;
   int boundaryType, calcNFR, needTime, useLC, farFieldRes;
@@ -81,7 +87,9 @@ struct McBatch {
   const Medium* media;            // [nItems * nM]
   const uint8_t* cdfIdx;          // [nItems * nM]
   int64_t L, nImage, nFF, nNI[6];
-  double* NFR;                    // [nItems * L]
+  double* NFR;                    // [nItems * L], L the voxels of the plan's order (McParams::LB)
+  int copies;                     // of the NFR slices, one per group of XCDs, `copyStride` apart
+  int64_t copyStride;
   double* image;                  // [nItems * nImage]
   double* FF;                     // [nItems * nFF]
   double* NI[6];                  // [nItems * nNI[f]]
@@ -130,6 +138,8 @@ __device__ inline __attribute__((always_inline)) void multi_item(const McBatch& 
     q.d[a] = G.d[a];
     q.inv_d[a] = G.inv_d[a];
   }
+  q.nbx = G.nbx;
+  q.nbxy = G.nbxy;
   q.tooOld = G.tooOld;
   q.boundaryType = G.boundaryType;
   q.calcNFR = G.calcNFR;
@@ -144,7 +154,7 @@ __device__ inline __attribute__((always_inline)) void multi_item(const McBatch& 
   E.R.key0 = bt.key[2 * it];
   E.R.key1 = bt.key[2 * it + 1];
   E.R.stream = bt.stream[it];
-  sink.NFR = bt.NFR + bt.off[9 * (size_t)it];
+  sink.NFR = bt.NFR + (xcd() % bt.copies) * bt.copyStride + bt.off[9 * (size_t)it];
   sink.item = it;
 }
 
@@ -166,9 +176,6 @@ __device__ inline unsigned long long bcast64(unsigned long long v, int src) {
 
 __device__ inline void fadd(double* p, double v) { unsafeAtomicAdd(p, v); }
 
-// lanes per transport workgroup: the stride of a lane's deposit ring slots
-constexpr int kRingStride = 256;
-
 // Largest number of packets per transport launch (sizes the launch and
 // escape record buffers: 64 + 48 bytes per packet).
 constexpr uint64_t kMaxLaunchPackets = 1ull << 24;
@@ -187,16 +194,8 @@ struct DeviceSink {
   int accJ;
   unsigned long long nCollected;
   unsigned nRunaway;
-  // the accelerator complex die (XCD) the wavefront runs on; each XCD has
-  // its own L2, so XCD-private fluence copies keep hot voxels from being
-  // contended across XCDs
-  __device__ static int xcd() {
-    unsigned r;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(r));
-    return (int)(r & 7u);
-  }
   __device__ explicit DeviceSink(const McParams& p)
-      : NFR(p.NFR + (size_t)(xcd() % p.nfrReplicas) * p.L), image(p.image), FF(p.FF), ni0(p.NI[0]), ni1(p.NI[1]), ni2(p.NI[2]), ni3(p.NI[3]), ni4(p.NI[4]),
+      : NFR(p.NFR + (size_t)(xcd() % p.nfrReplicas) * p.LB), image(p.image), FF(p.FF), ni0(p.NI[0]), ni1(p.NI[1]), ni2(p.NI[2]), ni3(p.NI[3]), ni4(p.NI[4]),
         ni5(p.NI[5]), acc(0.0), accJ(-1), nCollected(0), nRunaway(0) {}
   __device__ void deposit(int j, double v) {
     if (j == accJ) {
@@ -222,59 +221,61 @@ struct DeviceSink {
   __device__ void runaway() { ++nRunaway; }
 };
 
-// Deposits waiting in LDS per lane (see DeferSink), drained by the whole
-// wavefront together.
-#ifndef MCM_DEPOSIT_RING
-#define MCM_DEPOSIT_RING 8
-#endif
-constexpr int kRing = MCM_DEPOSIT_RING;
+// Deposits a lane parks in LDS (see DeferSink), and the pitch of a lane's slots
+// (odd, so that lanes writing their k-th slot hit different banks).
+constexpr int kRing = 16, kRingPitch = 17;
+struct RingSlots {
+  uint2 d[256 * kRingPitch];  // voxel, absorbed weight (float bits)
+};
 
 // Sink of the transport kernel without deposition criteria: a packet dies
 // once, so its escape is written to the record slot of its own launch index
 // (no shared counter) and tallied by mc_tally_escapes after the launch.
 //
-// Merged deposits do not go to the fluence one at a time: each lane parks
-// (address, value) in its slots of an LDS ring and the wavefront drains the
-// rings together when one of them is nearly full.  Global loads and atomics
-// share one in-order completion counter, so a load issued after an atomic
-// (the next voxel's medium index) waits for the atomic's round trip to the
-// memory side; draining in batches pays that wait once per batch instead of
-// once per voxel crossing.
+// The fluence is bound by the number of 64-byte lines that atomic
+// instructions touch: the memory side takes 2.37e10 of them per second
+// whatever they carry (scattered FP64 adds, 1024 to 2^23 voxels), and lanes
+// of one instruction that hit the same line share one.  Deposits are therefore
+// parked in LDS and issued with 16 lanes per packet: its last 16 voxels are
+// neighbours along its path, and a straight path stays in a sub-brick of
+// 2 x 2 x 2 voxels (one line) for two of them, so 16 deposits take 9.0 requests
+// (measured: 0.565 a deposit, at least 0.5) where one deposit per lane and
+// instruction would take 16.  Rings of 8 take as long.  A parked deposit is the
+// absorbed weight of one sub-step, a float.
 struct DeferSink : DeviceSink {
   static constexpr bool kDeferEscapes = true;
   EscapeRecord* rec;
   int item;
-  unsigned long long* ringA;  // LDS: slot k of this lane at [k * stride]
-  double* ringV;
+  RingSlots* ring;
   int nRing;
-  __device__ DeferSink(const McParams& p, EscapeRecord* r) : DeviceSink(p), rec(r), item(0), ringA(nullptr), ringV(nullptr), nRing(0) {}
-  __device__ void park(double* a, double v) {
-    if (!ringA) {
-      fadd(a, v);
-      return;
-    }
-    ringA[nRing * kRingStride] = (unsigned long long)a;
-    ringV[nRing * kRingStride] = v;
-    if (++nRing == kRing) drain();  // a full ring drains this lane alone
-  }
+  __device__ DeferSink(const McParams& p, EscapeRecord* r) : DeviceSink(p), rec(r), item(0), ring(nullptr), nRing(0) {}
+  // Issues the deposits of the whole wavefront (every lane calls it).
+  // PER_LANE: the lanes' fluence slices differ (batched launches).
+  template <bool PER_LANE>
   __device__ void drain() {
-    for (int k = 0; k < nRing; ++k) fadd((double*)ringA[k * kRingStride], ringV[k * kRingStride]);
+    using GlobalDouble = __attribute__((address_space(1))) double;
+    const int lane = __lane_id(), base = threadIdx.x & ~63;
+#pragma unroll 2
+    for (int r = 0; r < kRing; ++r) {
+      const int src = r * (64 / kRing) + lane / kRing, slot = lane % kRing;
+      const bool full = slot < __shfl(nRing, src, 64);
+      double* nfr = NFR;
+      if constexpr (PER_LANE) {
+        const unsigned lo = __shfl((unsigned)(size_t)NFR, src, 64), hi = __shfl((unsigned)((size_t)NFR >> 32), src, 64);
+        nfr = (double*)(((size_t)hi << 32) | lo);
+      }
+      if (full) {
+        const uint2 d = ring->d[(base + src) * kRingPitch + slot];
+        (void)__builtin_amdgcn_global_atomic_fadd_f64((GlobalDouble*)(nfr + d.x), (double)__uint_as_float(d.y));
+      }
+    }
     nRing = 0;
   }
-  __device__ void deposit(int j, double v) {
-    if (j == accJ) {
-      acc += v;
-    } else {
-      if (accJ >= 0) park(&NFR[accJ], acc);
-      accJ = j;
-      acc = v;
-    }
+  __device__ void deposit(int j, float v) {
+    ring->d[threadIdx.x * kRingPitch + nRing] = make_uint2((unsigned)j, __float_as_uint(v));
+    ++nRing;
   }
-  __device__ void flush() {
-    if (accJ >= 0) park(&NFR[accJ], acc);
-    accJ = -1;
-    acc = 0.0;
-  }
+  __device__ void flush() {}
   __device__ void escape(const Photon& P, bool escaped, bool edgeFlux, uint32_t slot) {
     EscapeRecord E;
     pack_escape(P, escaped, edgeFlux, item, E);
@@ -381,25 +382,22 @@ __global__ void __launch_bounds__(256) mc_tally_escapes(McParams p, McLaunch lp,
 }
 
 template <bool FRESNEL, bool CRITERIA, int BATCH>
-__global__ void __launch_bounds__(256, BATCH == kMulti ? 4 : 1) mc_transport(McParams p, McLaunch lp, McBatch bt, const LaunchRecord* __restrict__ launches,
+__global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p, McLaunch lp, McBatch bt, const LaunchRecord* __restrict__ launches,
                                                     EscapeRecord* __restrict__ escapes) {
   static_assert(!(BATCH != kPlain && CRITERIA), "batched launches run without deposition criteria");
-  constexpr int kMed = BATCH != kPlain ? kBatchMaxMedia : 256;
-  __shared__ Medium sMed[kMed];
-  __shared__ uint8_t sCdf[kMed];
-  __shared__ unsigned long long sCum[BATCH != kPlain ? kBatchMaxItems + 1 : 1];
-  if constexpr (BATCH != kPlain) {
-    for (int k = threadIdx.x; k < bt.nItems * bt.nM; k += blockDim.x) {
-      sMed[k] = bt.media[k];
-      sCdf[k] = bt.cdfIdx[k];
-    }
-    for (int k = threadIdx.x; k <= bt.nItems; k += blockDim.x) sCum[k] = bt.cum[k];
-  } else {
-    for (int k = threadIdx.x; k < 256; k += blockDim.x) {
-      sMed[k] = p.media[k];
-      sCdf[k] = p.cdfIdx[k];
-    }
+  // the media tables of the wavelength, or of every item, behind the items'
+  // packet ranges (dynamic LDS, sized by the launch: table_bytes)
+  extern __shared__ __align__(16) unsigned long long sItems[];
+  const int nEntries = BATCH == kPlain ? p.nM : bt.nItems * bt.nM;
+  unsigned long long* const sCum = sItems;
+  Medium* const sMed = (Medium*)(sItems + (BATCH == kPlain ? 0 : (bt.nItems + 2) & ~1));
+  uint8_t* const sCdf = (uint8_t*)(sMed + nEntries);
+  for (int k = threadIdx.x; k < nEntries; k += blockDim.x) {
+    sMed[k] = BATCH == kPlain ? p.media[k] : bt.media[k];
+    sCdf[k] = BATCH == kPlain ? p.cdfIdx[k] : bt.cdfIdx[k];
   }
+  if constexpr (BATCH != kPlain)
+    for (int k = threadIdx.x; k <= bt.nItems; k += blockDim.x) sCum[k] = bt.cum[k];
   __syncthreads();
 
   const int lane = __lane_id();
@@ -407,21 +405,20 @@ __global__ void __launch_bounds__(256, BATCH == kMulti ? 4 : 1) mc_transport(McP
   E.init(lp.key0, lp.key1, lp.stream);
   using Sink = typename std::conditional<CRITERIA, DeviceSink, DeferSink>::type;
   Sink sink = make_sink<Sink>(p, escapes);
-  // the deposit rings of the plain launch (batched and multi-grid launches
-  // keep every item's tables in LDS and deposit directly)
-  constexpr int RING = (!CRITERIA && BATCH == kPlain) ? kRing : 0;
-  __shared__ unsigned long long sRingA[RING > 0 ? RING * kRingStride : 1];
-  __shared__ double sRingV[RING > 0 ? RING * kRingStride : 1];
-  if constexpr (RING > 0) {
-    sink.ringA = sRingA + threadIdx.x;
-    sink.ringV = sRingV + threadIdx.x;
-  }
+  __shared__ typename std::conditional<CRITERIA, char, RingSlots>::type sRing;
+  if constexpr (!CRITERIA) sink.ring = &sRing;
   // the media tables of the lane's work item (the launch's in a plain launch)
   const Medium* med = sMed;
   const uint8_t* cdf = sCdf;
   unsigned long long nLaunched = 0, nSub = 0, nScat = 0, nIf = 0;
   McParams q;
   const McParams& pr = LaneParams<BATCH>::get(p, q);
+  // Launches of fewer packets than lanes spread them over all wavefronts
+  // (see launch_blocks)
+  {
+    const unsigned long long waves = (unsigned long long)gridDim.x * (blockDim.x / 64);
+    if ((unsigned long long)lane * waves >= lp.nPackets) E.state = ST_DONE;
+  }
   // Multi-grid launches: every lane of a wavefront holds packets of one
   // item (the wavefront's current item), so the item's grid and tables are
   // wavefront-uniform.  Wavefronts start spread over the launch's packets
@@ -439,10 +436,10 @@ __global__ void __launch_bounds__(256, BATCH == kMulti ? 4 : 1) mc_transport(McP
   }
 
   for (;;) {
-    if constexpr (RING > 0) {
-      // a lane parks at most two deposits per iteration (its sub-step's and
-      // its death's): drain every ring once one of them could overflow
-      if (__ballot(sink.nRing >= RING - 2)) sink.drain();
+    if constexpr (!CRITERIA) {
+      // a lane parks at most one deposit per iteration: drain every ring once
+      // one of them is full
+      if (__ballot(sink.nRing == kRing)) sink.template drain<BATCH == kBatch>();
     }
     const int st = E.state;
     const unsigned long long bFetch = __ballot(st == ST_FETCH);
@@ -463,6 +460,7 @@ __global__ void __launch_bounds__(256, BATCH == kMulti ? 4 : 1) mc_transport(McP
             if (__builtin_amdgcn_readfirstlane((unsigned)(v < bt.end[c]))) nxt = c;
           }
           if (nxt >= 0) {
+            sink.template drain<false>();  // parked deposits belong to the old item
             cur = nxt;
             curDone = false;
             multi_item(bt, cur, q, med, cdf, sMed, sCdf, E, sink);
@@ -496,6 +494,8 @@ __global__ void __launch_bounds__(256, BATCH == kMulti ? 4 : 1) mc_transport(McP
         E.do_fresnel(pr, med, cdf, sink);
       }
     } else {
+      // parked deposits belong to the item a lane leaves
+      if constexpr (BATCH == kBatch) sink.template drain<true>();
       // consecutive packet numbers for the waiting lanes, one atomic per wavefront
       const int leader = __ffsll((long long)bFetch) - 1;
       unsigned long long base = 0;
@@ -547,7 +547,7 @@ __global__ void __launch_bounds__(256, BATCH == kMulti ? 4 : 1) mc_transport(McP
             E.R.key0 = bt.key[2 * it];
             E.R.key1 = bt.key[2 * it + 1];
             E.R.stream = bt.stream[it];
-            sink.NFR = bt.NFR + (size_t)it * bt.L;
+            sink.NFR = bt.NFR + (xcd() % bt.copies) * bt.copyStride + (size_t)it * bt.L;
             sink.item = it;
             const LaunchRecord L = launches[k];
             ok = E.start_from(g - sCum[it], L, pr, med, cdf);
@@ -566,7 +566,7 @@ __global__ void __launch_bounds__(256, BATCH == kMulti ? 4 : 1) mc_transport(McP
     }
   }
   sink.flush();
-  if constexpr (RING > 0) sink.drain();
+  if constexpr (!CRITERIA) sink.template drain<BATCH == kBatch>();
   if (nLaunched) atomicAdd(&lp.ctr->launched, nLaunched);
   if (sink.nCollected) atomicAdd(&lp.ctr->collected, sink.nCollected);
   if (nSub) atomicAdd(&lp.ctr->substeps, nSub);
@@ -576,12 +576,25 @@ __global__ void __launch_bounds__(256, BATCH == kMulti ? 4 : 1) mc_transport(McP
 }
 
 // NFR normalisation (normalizeDepositionAndResetO, MCmatlablib.c:1204-1207):
-// out[j] = dep[j] / (V * normfactor * mua[M[j]]) as single; clears dep.
-__global__ void mc_normalize_nfr(double* dep, const uint8_t* M, const double* mua, double scale, float* out, int64_t L) {
+// out[j] = dep[j] / (V * normfactor * mua[M[j]]) as single, dep the sum of its
+// copies, `stride` apart, in the plan's voxel order; clears them.
+__global__ void mc_normalize_nfr(double* dep, int copies, int64_t stride, const uint8_t* M, const double* mua, double scale, float* out,
+                                 VoxelMap map, int64_t L) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= L) return;
-  out[j] = (float)(dep[j] / (scale * mua[M[j]]));
-  dep[j] = 0.0;
+  const int64_t i = map(j);
+  double sum = 0.0;
+  for (int c = 0; c < copies; ++c) {
+    sum += dep[c * stride + i];
+    dep[c * stride + i] = 0.0;
+  }
+  out[j] = (float)(sum / (scale * mua[M[j]]));
+}
+
+// The tally in linear order.
+__global__ void mc_linear_nfr(double* out, const double* dep, VoxelMap map, int64_t L) {
+  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < L) out[j] = dep[map(j)];
 }
 
 // Sum the fluence copies 1..R-1 into copy 0 and clear them.
@@ -702,7 +715,7 @@ int select_wavelength(mcm_mc_plan* pl, int64_t iL) {
   if (T.fresnelPossible) {
     const int tpb = 256;
     const int64_t nb = (T.L + tpb - 1) / tpb;
-    hipLaunchKernelGGL(mc_fill_normal_ri, dim3((unsigned)nb), dim3(tpb), 0, pl->stream, pl->normals.as<float4>(), pl->M.as<uint8_t>(),
+    hipLaunchKernelGGL(mc_fill_normal_ri, dim3((unsigned)nb), dim3(tpb), 0, pl->stream, pl->normals.as<float4>(), pl->Mlin.as<uint8_t>(),
                        p.media, T.L);
     MCM_HIP(hipGetLastError());
   }
@@ -734,9 +747,9 @@ int fold_replicas(mcm_mc_plan* pl) {
   const int R = pl->prm.nfrReplicas;
   if (R <= 1 || !pl->T.calcNFR) return MCM_OK;
   const int tpb = 256;
-  const int64_t nb = (pl->T.L + tpb - 1) / tpb;
+  const int64_t nb = (pl->prm.LB + tpb - 1) / tpb;
   MCM_HIP(hipDeviceSynchronize());  // launches on other streams write the copies
-  hipLaunchKernelGGL(mc_fold_replicas, dim3((unsigned)nb), dim3(tpb), 0, pl->stream, pl->NFR.as<double>(), pl->T.L, R);
+  hipLaunchKernelGGL(mc_fold_replicas, dim3((unsigned)nb), dim3(tpb), 0, pl->stream, pl->NFR.as<double>(), pl->prm.LB, R);
   MCM_HIP(hipGetLastError());
   return MCM_OK;
 }
@@ -748,9 +761,9 @@ int set_replicas(mcm_mc_plan* pl, int R) {
   if (rc) return rc;
   MCM_HIP(hipStreamSynchronize(pl->stream));
   DevBuf nb;
-  MCM_HIP(hipMalloc(&nb.p, (size_t)R * pl->T.L * sizeof(double)));
-  MCM_HIP(hipMemsetAsync(nb.p, 0, (size_t)R * pl->T.L * sizeof(double), pl->stream));
-  MCM_HIP(hipMemcpyAsync(nb.p, pl->NFR.p, (size_t)pl->T.L * sizeof(double), hipMemcpyDeviceToDevice, pl->stream));
+  MCM_HIP(hipMalloc(&nb.p, (size_t)R * pl->prm.LB * sizeof(double)));
+  MCM_HIP(hipMemsetAsync(nb.p, 0, (size_t)R * pl->prm.LB * sizeof(double), pl->stream));
+  MCM_HIP(hipMemcpyAsync(nb.p, pl->NFR.p, (size_t)pl->prm.LB * sizeof(double), hipMemcpyDeviceToDevice, pl->stream));
   MCM_HIP(hipStreamSynchronize(pl->stream));
   std::swap(pl->NFR.p, nb.p);
   pl->prm.nfrReplicas = R;
@@ -776,12 +789,20 @@ int ensure_records(mcm_mc_plan* pl, uint64_t n) {
   return MCM_OK;
 }
 
+// dynamic LDS of a transport launch: the items' packet ranges, media and CDF
+// indices
+size_t table_bytes(int nItems, int nM) {
+  return (size_t)(nItems ? (nItems + 2) & ~1 : 0) * 8 + (size_t)std::max(nItems, 1) * nM * (sizeof(Medium) + 1);
+}
+
+int occupancy_blocks(int device, bool fr, bool cr, int kind, size_t lds);
+
 // One launch of n <= kMaxLaunchPackets packets.  Without deposition
 // criteria: launch kernel -> transport -> escape tallies; with criteria the
 // transport launches and tallies inline.  `bt` (batched launches) maps the
 // global packet indices first .. first+n-1 to work items.
 int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed, uint32_t stream, hipStream_t s,
-                     const McBatch* bt = nullptr, int kind = kPlain, bool fresnel = false, bool tallies = false) {
+                     const McBatch* bt = nullptr, int kind = kPlain, bool fresnel = false, bool tallies = false, int blocks_items = 0) {
   McLaunch lp;
   lp.firstPacket = first;
   lp.nPackets = n;
@@ -795,12 +816,11 @@ int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed,
   McBatch none;
   std::memset(&none, 0, sizeof none);
   const McBatch& B = bt ? *bt : none;
-  const dim3 b(pl->threads);
+  const dim3 b(pl->threads), g(launch_blocks(pl, kind == kPlain ? pl->blocks : blocks_items, n));
   MCM_HIP(hipMemsetAsync(pl->counters.p, 0, sizeof(unsigned long long), s));  // nextPacket
   if (cr) {
-    const dim3 g(pl->blocks);
-    if (fr) hipLaunchKernelGGL((mc_transport<true, true, kPlain>), g, b, 0, s, pl->prm, lp, B, nullptr, nullptr);
-    else hipLaunchKernelGGL((mc_transport<false, true, kPlain>), g, b, 0, s, pl->prm, lp, B, nullptr, nullptr);
+    if (fr) hipLaunchKernelGGL((mc_transport<true, true, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, nullptr, nullptr);
+    else hipLaunchKernelGGL((mc_transport<false, true, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, nullptr, nullptr);
     MCM_HIP(hipGetLastError());
     return MCM_OK;
   }
@@ -813,34 +833,42 @@ int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed,
   for (int f = 0; f < 6; ++f) anyNI = anyNI || T.nNI[f] > 0;
   const bool tally = kind == kMulti ? tallies : (T.base.useLC || T.base.farFieldRes || anyNI);
   if (kind == kMulti) {
-    const dim3 g(pl->blocksMulti);
     hipLaunchKernelGGL(mc_multi_ranges, dim3(1), dim3(256), 0, s, B, (unsigned long long)first, (unsigned long long)n, B.next,
                        const_cast<unsigned long long*>(B.end));
     hipLaunchKernelGGL(mc_launch_packets<kMulti>, g, b, 0, s, pl->prm, lp, B, L, E);
-    if (fr) hipLaunchKernelGGL((mc_transport<true, false, kMulti>), g, b, 0, s, pl->prm, lp, B, L, E);
-    else hipLaunchKernelGGL((mc_transport<false, false, kMulti>), g, b, 0, s, pl->prm, lp, B, L, E);
+    if (fr) hipLaunchKernelGGL((mc_transport<true, false, kMulti>), g, b, table_bytes(B.nItems, B.nM), s, pl->prm, lp, B, L, E);
+    else hipLaunchKernelGGL((mc_transport<false, false, kMulti>), g, b, table_bytes(B.nItems, B.nM), s, pl->prm, lp, B, L, E);
     if (tally) hipLaunchKernelGGL(mc_tally_escapes<kMulti>, g, b, 0, s, pl->prm, lp, B, E);
   } else if (bt) {
-    const dim3 g(pl->blocksBatch);
     hipLaunchKernelGGL(mc_launch_packets<kBatch>, g, b, 0, s, pl->prm, lp, B, L, E);
-    if (fr) hipLaunchKernelGGL((mc_transport<true, false, kBatch>), g, b, 0, s, pl->prm, lp, B, L, E);
-    else hipLaunchKernelGGL((mc_transport<false, false, kBatch>), g, b, 0, s, pl->prm, lp, B, L, E);
+    if (fr) hipLaunchKernelGGL((mc_transport<true, false, kBatch>), g, b, table_bytes(B.nItems, B.nM), s, pl->prm, lp, B, L, E);
+    else hipLaunchKernelGGL((mc_transport<false, false, kBatch>), g, b, table_bytes(B.nItems, B.nM), s, pl->prm, lp, B, L, E);
     if (tally) hipLaunchKernelGGL(mc_tally_escapes<kBatch>, g, b, 0, s, pl->prm, lp, B, E);
   } else {
-    const dim3 g(pl->blocks);
     hipLaunchKernelGGL(mc_launch_packets<kPlain>, g, b, 0, s, pl->prm, lp, B, L, E);
-    if (fr) hipLaunchKernelGGL((mc_transport<true, false, kPlain>), g, b, 0, s, pl->prm, lp, B, L, E);
-    else hipLaunchKernelGGL((mc_transport<false, false, kPlain>), g, b, 0, s, pl->prm, lp, B, L, E);
+    if (fr) hipLaunchKernelGGL((mc_transport<true, false, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, L, E);
+    else hipLaunchKernelGGL((mc_transport<false, false, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, L, E);
     if (tally) hipLaunchKernelGGL(mc_tally_escapes<kPlain>, g, b, 0, s, pl->prm, lp, B, E);
   }
   MCM_HIP(hipGetLastError());
   return MCM_OK;
 }
 
+// Fluence copies of a launch of several items, `voxels` in all and LB in one:
+// those of a plan, within 1 GiB.  The items of a batch run one after another, so
+// one item's copies are in use at a time (8 items of 150^3, 3.3 10^6 packets of a
+// pencil beam: kernel 52.3 ms with one copy, 25.1 ms with eight).
+constexpr int64_t kItemCopiesBytes = (int64_t)2 << 30;
+int item_copies(int64_t LB, int64_t voxels) {
+  int n = start_copies(LB);
+  while (n > 1 && n * voxels * (int64_t)sizeof(double) > kItemCopiesBytes) n /= 2;
+  return n;
+}
+
 // Normalised outputs of one work item from its FP64 tally slices
 // (normalizeDepositionAndResetO, MCmatlablib.c:1186-1250); null slices are
 // skipped.
-int finish_item(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, const double* nfr, const double* img, const double* ff,
+int finish_item(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, double* nfr, int copies, int64_t stride, const double* img, const double* ff,
                 const double* const ni[6], unsigned long long collected, double minutes, int64_t lanes, mcm_mc_output& o) {
   const McTables& T = pl->T;
   hipStream_t s = pl->stream;
@@ -859,8 +887,8 @@ int finish_item(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, const double* nf
     if (!pl->nfrOut.p) MCM_HIP(hipMalloc(&pl->nfrOut.p, (size_t)T.L * sizeof(float)));
     const int tpb = 256;
     const int64_t nb = (T.L + tpb - 1) / tpb;
-    hipLaunchKernelGGL(mc_normalize_nfr, dim3((unsigned)nb), dim3(tpb), 0, s, const_cast<double*>(nfr), pl->M.as<uint8_t>(),
-                       pl->muaNorm.as<double>() + (size_t)iL * T.nM, T.V * normfactor, pl->nfrOut.as<float>(), T.L);
+    hipLaunchKernelGGL(mc_normalize_nfr, dim3((unsigned)nb), dim3(tpb), 0, s, nfr, copies, stride, pl->Mlin.as<uint8_t>(),
+                       pl->muaNorm.as<double>() + (size_t)iL * T.nM, T.V * normfactor, pl->nfrOut.as<float>(), voxel_map(pl), T.L);
     MCM_HIP(hipGetLastError());
     MCM_HIP(hipMemcpyAsync(o.NFR, pl->nfrOut.p, (size_t)T.L * sizeof(float), hipMemcpyDeviceToHost, s));
     MCM_HIP(hipStreamSynchronize(s));
@@ -884,7 +912,7 @@ int finish_item(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, const double* nf
   return MCM_OK;
 }
 
-int occupancy_blocks(int device, bool fr, bool cr, int kind = kPlain) {
+int occupancy_blocks(int device, bool fr, bool cr, int kind, size_t lds) {
   int per = 0;
   const void* k;
   if (kind == kMulti) k = fr ? (const void*)mc_transport<true, false, kMulti> : (const void*)mc_transport<false, false, kMulti>;
@@ -893,7 +921,7 @@ int occupancy_blocks(int device, bool fr, bool cr, int kind = kPlain) {
   else if (fr) k = (const void*)mc_transport<true, false, kPlain>;
   else if (cr) k = (const void*)mc_transport<false, true, kPlain>;
   else k = (const void*)mc_transport<false, false, kPlain>;
-  const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, 256, 0);
+  const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, 256, lds);
   if (e != hipSuccess || per < 1) per = 4;
   return per * cu_count(device);
 }
@@ -938,7 +966,20 @@ int mcm_mc_plan_create(const mcm_mc_input* in, mcm_mc_plan** out) {
   MCM_HIP(hipStreamCreate(&pl->stream));
   McTables& T = pl->T;
   hipStream_t s = pl->stream;
-  if ((rc = upload(pl->M, T.M0.data(), T.M0.size(), s))) return rc;
+  if ((rc = upload(pl->Mlin, T.M0.data(), T.M0.size(), s))) return rc;
+  // bricks unless padding them would cost a lot of memory (grids of one or two
+  // voxels along an axis) or their indices
+  const int nb[3] = {(T.nx + 3) / 4, (T.ny + 3) / 4, (T.nz + 3) / 4};
+  const int64_t padded = (int64_t)nb[0] * nb[1] * nb[2] * 64;
+  const bool bricks = padded <= 2 * T.L && padded < ((int64_t)1 << 31);
+  const VoxelMap map{T.nx, T.ny, bricks ? nb[0] : 0, bricks ? nb[0] * nb[1] : 0};
+  T.base.nbx = map.nbx;
+  T.base.nbxy = map.nbxy;
+  T.base.LB = bricks ? padded : T.L;
+  if ((rc = upload<uint8_t>(pl->M, nullptr, (size_t)T.base.LB, s))) return rc;
+  hipLaunchKernelGGL(mc_to_bricks<uint8_t>, dim3((unsigned)((T.L + 255) / 256)), dim3(256), 0, s, pl->M.as<uint8_t>(), pl->Mlin.as<uint8_t>(),
+                     map, T.L);
+  MCM_HIP(hipGetLastError());
   if (T.fresnelPossible && (rc = upload(pl->normals, T.normals.data(), T.normals.size(), s))) return rc;
   if ((rc = upload(pl->media, T.media.data(), T.media.size(), s))) return rc;
   if ((rc = upload(pl->cdfIdx, T.cdfIdx.data(), T.cdfIdx.size(), s))) return rc;
@@ -950,7 +991,8 @@ int mcm_mc_plan_create(const mcm_mc_input* in, mcm_mc_plan** out) {
   if ((rc = upload(pl->muaNorm, T.muaNorm.data(), T.muaNorm.size(), s))) return rc;
   pl->sourceDistribution = in->sourceDistribution;
   if (in->sourceDistribution && (rc = upload<double>(pl->S, nullptr, (size_t)T.L + 1, s))) return rc;
-  if ((rc = zeros(pl->NFR, (T.calcNFR ? (size_t)T.L : 1) * sizeof(double), s))) return rc;
+  if (T.calcNFR) T.base.nfrReplicas = start_copies(T.base.LB);
+  if ((rc = zero_copies(pl->NFR, T.base.nfrReplicas, T.calcNFR ? T.base.LB : 1, s))) return rc;
   if ((rc = zeros(pl->image, (size_t)std::max<int64_t>(T.nImage, 1) * sizeof(double), s))) return rc;
   if ((rc = zeros(pl->FF, (size_t)std::max<int64_t>(T.nFF, 1) * sizeof(double), s))) return rc;
   for (int f = 0; f < 6; ++f)
@@ -971,11 +1013,9 @@ int mcm_mc_plan_create(const mcm_mc_input* in, mcm_mc_plan** out) {
   p.FF = pl->FF.as<double>();
   for (int f = 0; f < 6; ++f) p.NI[f] = pl->NI[f].as<double>();
   pl->threads = 256;
-  pl->blocks = occupancy_blocks(pl->device, T.fresnelPossible, p.criteriaActive != 0);
-  pl->blocksBatch = occupancy_blocks(pl->device, T.fresnelPossible, false, kBatch);
-  pl->blocksMulti = std::min(occupancy_blocks(pl->device, true, false, kMulti), occupancy_blocks(pl->device, false, false, kMulti));
+  pl->blocks = occupancy_blocks(pl->device, T.fresnelPossible, p.criteriaActive != 0, kPlain, table_bytes(0, T.nM));
   if (const char* e = std::getenv("MCM_MC_MOVE_FRAC")) pl->moveFrac = (float)std::atof(e);
-  if (const char* e = std::getenv("MCM_MC_BLOCKS")) pl->blocks = pl->blocksBatch = pl->blocksMulti = std::max(1, std::atoi(e));
+  if (const char* e = std::getenv("MCM_MC_BLOCKS")) pl->blocks = pl->blocksForced = std::max(1, std::atoi(e));
   if ((rc = select_wavelength(pl.get(), 0))) return rc;
   MCM_HIP(hipStreamSynchronize(s));
   *out = pl.release();
@@ -1009,7 +1049,16 @@ int mcm_mc_plan_tallies(mcm_mc_plan* pl, const double** d_deposit, uint64_t* nPh
   int rc = fold_replicas(pl);
   if (rc) return rc;
   MCM_HIP(hipStreamSynchronize(pl->stream));
-  if (d_deposit) *d_deposit = pl->NFR.as<double>();
+  const double* nfr = pl->NFR.as<double>();
+  if (d_deposit && pl->T.calcNFR && pl->prm.nbx) {
+    if (!pl->nfrLin.p) MCM_HIP(hipMalloc(&pl->nfrLin.p, (size_t)pl->T.L * sizeof(double)));
+    hipLaunchKernelGGL(mc_linear_nfr, dim3((unsigned)((pl->T.L + 255) / 256)), dim3(256), 0, pl->stream, pl->nfrLin.as<double>(), nfr,
+                       voxel_map(pl), pl->T.L);
+    MCM_HIP(hipGetLastError());
+    MCM_HIP(hipStreamSynchronize(pl->stream));
+    nfr = pl->nfrLin.as<double>();
+  }
+  if (d_deposit) *d_deposit = nfr;
   if (nPhotons) *nPhotons = c.launched;
   return MCM_OK;
 }
@@ -1027,14 +1076,12 @@ int mcm_mc_plan_normalize(mcm_mc_plan* pl, int64_t iL, mcm_mc_output* out) {
   double normfactor = (double)c.launched / pl->power;
   if (pl->sourceDistribution) normfactor /= pl->power;
   else if (T.base.beamType == 2 && (T.base.boundaryType == 0 || T.base.boundaryType == 2)) normfactor /= kKillRange * kKillRange;
-  int rc0 = fold_replicas(pl);
-  if (rc0) return rc0;
   if (T.calcNFR && out->NFR) {
     if (!pl->nfrOut.p) MCM_HIP(hipMalloc(&pl->nfrOut.p, (size_t)T.L * sizeof(float)));
     const int tpb = 256;
     const int64_t nb = (T.L + tpb - 1) / tpb;
-    hipLaunchKernelGGL(mc_normalize_nfr, dim3((unsigned)nb), dim3(tpb), 0, s, pl->NFR.as<double>(), pl->M.as<uint8_t>(),
-                       pl->muaNorm.as<double>() + (size_t)iL * T.nM, T.V * normfactor, pl->nfrOut.as<float>(), T.L);
+    hipLaunchKernelGGL(mc_normalize_nfr, dim3((unsigned)nb), dim3(tpb), 0, s, pl->NFR.as<double>(), pl->prm.nfrReplicas, pl->prm.LB, pl->Mlin.as<uint8_t>(),
+                       pl->muaNorm.as<double>() + (size_t)iL * T.nM, T.V * normfactor, pl->nfrOut.as<float>(), voxel_map(pl), T.L);
     MCM_HIP(hipGetLastError());
     MCM_HIP(hipMemcpyAsync(out->NFR + (size_t)iL * T.L, pl->nfrOut.p, (size_t)T.L * sizeof(float), hipMemcpyDeviceToHost, s));
   }
@@ -1083,7 +1130,7 @@ int mcm_mc_plan_autotune(mcm_mc_plan* pl, int64_t iL, uint64_t nPackets, double*
   int rc = MCM_OK;
   for (int c = 0; c < 4 && rc == MCM_OK; ++c) {
     const int R = cand[c];
-    if (R > 1 && (!T.calcNFR || (double)R * T.L * 8 > 2147483648.0)) continue;
+    if (R > 1 && (!T.calcNFR || (double)R * pl->prm.LB * 8 > 2147483648.0)) continue;
     if ((rc = set_replicas(pl, R))) break;
     if ((rc = mcm_mc_plan_simulate(pl, iL, std::min<uint64_t>(nPackets, 1u << 16), 0x7E57ull, 0, nullptr))) break;  // warm-up
     (void)hipEventRecord(e0, pl->stream);
@@ -1106,7 +1153,7 @@ int mcm_mc_plan_autotune(mcm_mc_plan* pl, int64_t iL, uint64_t nPackets, double*
   // discard the trial tallies
   hipStream_t s = pl->stream;
   MCM_HIP(hipDeviceSynchronize());
-  if (T.calcNFR) MCM_HIP(hipMemsetAsync(pl->NFR.p, 0, (size_t)pl->prm.nfrReplicas * T.L * sizeof(double), s));
+  if (T.calcNFR) MCM_HIP(hipMemsetAsync(pl->NFR.p, 0, (size_t)pl->prm.nfrReplicas * pl->prm.LB * sizeof(double), s));
   MCM_HIP(hipMemsetAsync(pl->image.p, 0, (size_t)std::max<int64_t>(T.nImage, 1) * sizeof(double), s));
   MCM_HIP(hipMemsetAsync(pl->FF.p, 0, (size_t)std::max<int64_t>(T.nFF, 1) * sizeof(double), s));
   for (int f = 0; f < 6; ++f) MCM_HIP(hipMemsetAsync(pl->NI[f].p, 0, (size_t)std::max<int64_t>(T.nNI[f], 1) * sizeof(double), s));
@@ -1189,10 +1236,12 @@ int mcm_mc_batch_run(mcm_mc_plan* pl, const mcm_mc_item* items, int64_t nItems, 
   B.stream = dStrm.as<uint32_t>();
   B.media = dMed.as<Medium>();
   B.cdfIdx = dCdf.as<uint8_t>();
-  B.L = T.L;
+  B.L = pl->prm.LB;
   B.nImage = T.nImage;
   B.nFF = T.nFF;
-  if ((rc = zeros(dNFR, (T.calcNFR ? (size_t)nI * T.L : 1) * sizeof(double), s)) ||
+  B.copies = T.calcNFR ? item_copies(pl->prm.LB, nI * pl->prm.LB) : 1;
+  B.copyStride = T.calcNFR ? nI * pl->prm.LB : 1;
+  if ((rc = zero_copies(dNFR, B.copies, B.copyStride, s)) ||
       (rc = zeros(dImg, (size_t)std::max<int64_t>(nI * T.nImage, 1) * sizeof(double), s)) ||
       (rc = zeros(dFF, (size_t)std::max<int64_t>(nI * T.nFF, 1) * sizeof(double), s)) ||
       (rc = zeros(dColl, (size_t)nI * sizeof(unsigned long long), s)))
@@ -1206,12 +1255,13 @@ int mcm_mc_batch_run(mcm_mc_plan* pl, const mcm_mc_item* items, int64_t nItems, 
   B.image = dImg.as<double>();
   B.FF = dFF.as<double>();
   B.collected = dColl.as<unsigned long long>();
+  const int blocks = pl->blocksForced ? pl->blocksForced : occupancy_blocks(pl->device, T.fresnelPossible, false, kBatch, table_bytes(nI, nM));
   MCM_HIP(hipMemsetAsync(pl->counters.p, 0, sizeof(McCounters), s));
   const auto t0 = std::chrono::steady_clock::now();
   const unsigned long long total = cum[nI];
   for (unsigned long long done = 0; done < total;) {
     const uint64_t n = std::min<unsigned long long>(total - done, kMaxLaunchPackets);
-    if ((rc = launch_transport(pl, done, n, 0, 0, s, &B))) return rc;
+    if ((rc = launch_transport(pl, done, n, 0, 0, s, &B, kBatch, false, false, blocks))) return rc;
     done += n;
   }
   MCM_HIP(hipStreamSynchronize(s));
@@ -1226,9 +1276,9 @@ int mcm_mc_batch_run(mcm_mc_plan* pl, const mcm_mc_item* items, int64_t nItems, 
   for (int i = 0; i < nI; ++i) {
     const double* ni[6];
     for (int f = 0; f < 6; ++f) ni[f] = dNI[f].as<double>() + (size_t)i * T.nNI[f];
-    if ((rc = finish_item(pl, items[i].iL, items[i].nPhotons, T.calcNFR ? dNFR.as<double>() + (size_t)i * T.L : nullptr,
-                          dImg.as<double>() + (size_t)i * T.nImage, dFF.as<double>() + (size_t)i * T.nFF, ni, coll[i], minutes,
-                          (int64_t)pl->blocksBatch * pl->threads, outs[i])))
+    if ((rc = finish_item(pl, items[i].iL, items[i].nPhotons, T.calcNFR ? dNFR.as<double>() + (size_t)i * pl->prm.LB : nullptr,
+                          B.copies, B.copyStride, dImg.as<double>() + (size_t)i * T.nImage, dFF.as<double>() + (size_t)i * T.nFF, ni, coll[i], minutes,
+                          (int64_t)blocks * pl->threads, outs[i])))
       return rc;
   }
   return MCM_OK;
@@ -1277,7 +1327,7 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
   bool tallies = false;
   for (int i = 0; i < nI; ++i) {
     const McTables& T = plans[items[i].plan]->T;
-    const int64_t sz[9] = {T.calcNFR ? T.L : 0, T.nImage, T.nFF, T.nNI[0], T.nNI[1], T.nNI[2], T.nNI[3], T.nNI[4], T.nNI[5]};
+    const int64_t sz[9] = {T.calcNFR ? plans[items[i].plan]->prm.LB : 0, T.nImage, T.nFF, T.nNI[0], T.nNI[1], T.nNI[2], T.nNI[3], T.nNI[4], T.nNI[5]};
     for (int k = 0; k < 9; ++k) {
       off[(size_t)i * 9 + k] = tot[k];
       tot[k] += sz[k];
@@ -1286,7 +1336,10 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
     tallies = tallies || T.base.useLC || T.base.farFieldRes;
   }
   DevBuf dTal[9], dColl, dOff, dParams, dGeom;
-  for (int k = 0; k < 9; ++k)
+  int copies = item_copies(tot[0] / nI, tot[0]);
+  const int64_t copyStride = std::max<int64_t>(tot[0], 1);
+  if ((rc = zero_copies(dTal[0], copies, copyStride, s))) return rc;
+  for (int k = 1; k < 9; ++k)
     if ((rc = zeros(dTal[k], (size_t)std::max<int64_t>(tot[k], 1) * sizeof(double), s))) return rc;
   if ((rc = zeros(dColl, (size_t)nI * sizeof(unsigned long long), s)) || (rc = upload(dOff, off.data(), off.size(), s))) return rc;
   std::vector<McParams> params((size_t)nPlans);
@@ -1300,6 +1353,8 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
       g.d[a] = p.d[a];
       g.inv_d[a] = p.inv_d[a];
     }
+    g.nbx = p.nbx;
+    g.nbxy = p.nbxy;
     g.tooOld = p.tooOld;
     g.boundaryType = p.boundaryType;
     g.calcNFR = p.calcNFR;
@@ -1311,6 +1366,7 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
     g.cdfs = p.cdfs;
   }
   if ((rc = upload(dParams, params.data(), params.size(), s)) || (rc = upload(dGeom, geom.data(), geom.size(), s))) return rc;
+  int blocks = pl0->blocksForced;
   MCM_HIP(hipMemsetAsync(pl0->counters.p, 0, sizeof(McCounters), s));
   const auto t0 = std::chrono::steady_clock::now();
   // one sequence of launches per interface class (Fresnel or matched), so
@@ -1358,6 +1414,8 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
     B.media = dMed.as<Medium>();
     B.cdfIdx = dCdf.as<uint8_t>();
     B.NFR = dTal[0].as<double>();
+    B.copies = copies;
+    B.copyStride = copyStride;
     B.image = dTal[1].as<double>();
     B.FF = dTal[2].as<double>();
     for (int f = 0; f < 6; ++f) B.NI[f] = dTal[3 + f].as<double>();
@@ -1368,6 +1426,7 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
     B.off = dOffc.as<int64_t>();
     B.next = dNext.as<unsigned long long>();
     B.end = dEnd.as<unsigned long long>();
+    if (!pl0->blocksForced) blocks = occupancy_blocks(pl0->device, cls == 0, false, kMulti, table_bytes(n, nMmax));
     // launches of whole items where they fit (an item split over two
     // launches pays the tail of its longest-lived packets twice)
     const unsigned long long total = cum[(size_t)n];
@@ -1378,7 +1437,7 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
           stop = cum[(size_t)j] - done >= kMaxLaunchPackets / 4 || cum[(size_t)j] == total ? cum[(size_t)j] : stop;
           break;
         }
-      if ((rc = launch_transport(pl0, done, stop - done, 0, 0, s, &B, kMulti, cls == 0, tallies))) return rc;
+      if ((rc = launch_transport(pl0, done, stop - done, 0, 0, s, &B, kMulti, cls == 0, tallies, blocks))) return rc;
       done = stop;
     }
     std::vector<unsigned long long> cc((size_t)n);
@@ -1400,8 +1459,8 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
     for (int f = 0; f < 6; ++f) ni[f] = dTal[3 + f].as<double>() + o[3 + f];
     const unsigned long long coll = (unsigned long long)outs[i].nPhotonsCollected;
     if ((rc = finish_item(pl, items[i].iL, items[i].nPhotons, pl->T.calcNFR ? dTal[0].as<double>() + o[0] : nullptr,
-                          dTal[1].as<double>() + o[1], dTal[2].as<double>() + o[2], ni, coll, minutes,
-                          (int64_t)pl0->blocksMulti * pl0->threads, outs[i])))
+                          copies, copyStride, dTal[1].as<double>() + o[1], dTal[2].as<double>() + o[2], ni, coll, minutes,
+                          (int64_t)blocks * pl0->threads, outs[i])))
       return rc;
   }
   return MCM_OK;

@@ -52,7 +52,11 @@ struct McParams {
   float inv_d[3];
   int boundaryType;
   int nM;
-  const uint8_t* M;            // 0-based medium per voxel, x fastest
+  // Voxel order of M, the fluence and per-voxel maps (voxel_index): bricks of
+  // 4 x 4 x 4 voxels, nbx a row and nbxy a layer, or x fastest when nbx is 0
+  int nbx, nbxy;
+  int64_t LB;                  // voxels of that order, padding included
+  const uint8_t* M;            // 0-based medium per voxel
   const float4* normalRI;      // unit interface normal (x,y,z) and refractive index per voxel; null if matched
   const Medium* media;         // [nM] (the kernel stages it into LDS)
   const uint8_t* cdfIdx;       // [nM] custom phase-function table per medium
@@ -118,11 +122,29 @@ struct MoveResult {
 
 MCM_FN int clampi(int x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : x); }
 
-MCM_FN int clamp_axis(float i, int n) { return i < 0.f ? 0 : (i >= (float)n ? n - 1 : (int)floorf(i)); }
+// voxel coordinate of position i on an axis of n voxels (no branch; n < 2^24)
+MCM_FN int clamp_axis(float i, int n) { return (int)fminf(fmaxf(floorf(i), 0.f), (float)(n - 1)); }
+
+// Index of voxel (x, y, z) in the order of M and the fluence.  A packet walks
+// from voxel to neighbouring voxel, so both are kept in bricks: 64 bytes of M
+// are one 4 x 4 x 4 brick (a packet stays on the cache line for 4 voxels on
+// average instead of 1 to 2 in rows), and within a brick each 2 x 2 x 2
+// sub-brick is consecutive, so 64 bytes of the fluence are 8 neighbouring
+// voxels and consecutive deposits of a packet share them (DeferSink).
+MCM_FN int brick_index(int x, int y, int z, int nbx, int nbxy) {
+  // bits within the brick: z1 y1 x1 z0 y0 x0; a two-bit number v spreads to
+  // bits 0 and 3 as (5 v) & 9
+  const unsigned s = (((unsigned)x & 3u) | ((unsigned)y & 3u) << 8 | ((unsigned)z & 3u) << 16) * 5u;
+  const unsigned in = (s & 9u) | (s >> 7 & 18u) | (s >> 14 & 36u);
+  return (int)((unsigned)((z >> 2) * nbxy + (y >> 2) * nbx + (x >> 2)) << 6 | in);
+}
+MCM_FN int voxel_index(const McParams& p, int x, int y, int z) {
+  return p.nbx ? brick_index(x, y, z, p.nbx, p.nbxy) : (z * p.n[1] + y) * p.n[0] + x;
+}
 
 // getNewj (MCmatlablib.c:281-285)
 MCM_FN int voxel_of(const McParams& p, const float* i) {
-  return clamp_axis(i[2], p.n[2]) * (p.n[0] * p.n[1]) + clamp_axis(i[1], p.n[1]) * p.n[0] + clamp_axis(i[0], p.n[0]);
+  return voxel_index(p, clamp_axis(i[0], p.n[0]), clamp_axis(i[1], p.n[1]), clamp_axis(i[2], p.n[2]));
 }
 
 // Unique j in [0, N-1] with D[j] < x <= D[j+1] for a nondecreasing table
@@ -159,7 +181,8 @@ MCM_FN void set_crossing_lengths(Photon& P, const McParams& p) {
 }
 
 MCM_FN bool inside_box(const McParams& p, const float* i) {
-  return i[0] < (float)p.n[0] && i[0] >= 0.f && i[1] < (float)p.n[1] && i[1] >= 0.f && i[2] < (float)p.n[2] && i[2] >= 0.f;
+  // (bitwise: six compares without branches)
+  return (i[0] < (float)p.n[0]) & (i[0] >= 0.f) & (i[1] < (float)p.n[1]) & (i[1] >= 0.f) & (i[2] < (float)p.n[2]) & (i[2] >= 0.f);
 }
 
 // Inside the extended region a packet may wander in for boundary types 0 and 2
@@ -482,48 +505,67 @@ MCM_FN void new_voxel_properties(Photon& P, const McParams& p, const Medium* med
   P.cdf = cdfIdx[m];
 }
 
-// Movement half of propagatePhoton (MCmatlablib.c:1022-1047, :1086-1093):
-// step to the next boundary or interaction, absorb continuously.
-template <bool FRESNEL>
-MCM_FN MoveResult move(Photon& P, const McParams& p, const Medium* media) {
-  MoveResult r;
-  P.sameVoxel = true;
+// First part of propagatePhoton's movement (MCmatlablib.c:1022-1040): step to
+// the next boundary or interaction.  Both outcomes of every axis are computed
+// and selected (no branch).  Returns the geometric length of the sub-step [cm].
+MCM_FN float advance(Photon& P, const McParams& p) {
   ++P.substeps;
   const float q = P.stepLeft / P.mus;
   const float s = fminf(q, fminf(P.D[0], fminf(P.D[1], P.D[2])));
   P.stepLeft = s == q ? 0.f : P.stepLeft - s * P.mus;
   if (p.needTime) P.time += s * P.ri / kC;
+  bool crossed = false;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
+    const bool cross = s == P.D[a], up = P.u[a] > 0.f;
     const float fi = floorf(P.i[a]);
-    if (s == P.D[a]) {
-      P.i[a] = P.u[a] > 0.f ? fi + 1.f : fi - kEps * (fabsf(fi) + 1.f);
-      P.D[a] = P.Dfull[a];
-      P.sameVoxel = false;
-    } else {
-      float ni = P.i[a] + s * P.u[a] * p.inv_d[a];
-      if (floorf(ni) != fi) ni = P.u[a] > 0.f ? fi + 1.f - kEps * (fabsf(fi) + 1.f) : fi;
-      P.i[a] = ni;
-      P.D[a] -= s;
-    }
+    // onto the boundary crossed
+    const float below = fi - kEps * (fabsf(fi) + 1.f);
+    const float onto = up ? fi + 1.f : below;
+    // within the voxel
+    const float moved = P.i[a] + s * P.u[a] * p.inv_d[a];
+    const float edge = fi + 1.f - kEps * (fabsf(fi) + 1.f);
+    const float within = floorf(moved) != fi ? (up ? edge : fi) : moved;
+    const float rest = P.D[a] - s;
+    P.i[a] = cross ? onto : within;
+    P.D[a] = cross ? P.Dfull[a] : rest;
+    crossed |= cross;
   }
+  P.sameVoxel = !crossed;
+  return s;
+}
+
+// Continuous absorption over a sub-step of length s (:1086-1093); returns the
+// absorbed weight.
+MCM_FN float absorb(Photon& P, float s) {
+  const float absorbed = -P.weight * expm1f(-P.mua * s);
+  P.weight -= absorbed;
+  return absorbed;
+}
+
+// An interface transition without a change of refractive index, counted for
+// the deposition criteria (:1041-1046).
+MCM_FN void count_transition(Photon& P, const McParams& p, const Medium* media, int mNew) {
+  const int mOld = p.M[P.j];
+  if (mNew != mOld && media[mOld].ri == P.ri && in_count_range(mNew, p)) ++P.transitions;
+}
+
+// Movement half of propagatePhoton: advance, look at the interface crossed,
+// absorb.
+template <bool FRESNEL>
+MCM_FN MoveResult move(Photon& P, const McParams& p, const Medium* media) {
+  MoveResult r;
+  r.s = advance(P, p);
   r.fresnel = false;
   r.jNew = P.j;
   r.mNew = -1;
   if (!P.sameVoxel && (FRESNEL || p.criteriaActive)) {
     r.jNew = voxel_of(p, P.i);
     r.mNew = p.M[r.jNew];
-    const float riNew = media[r.mNew].ri;
-    if (FRESNEL && P.ri != riNew) {
-      r.fresnel = true;
-    } else if (p.criteriaActive) {
-      const int mOld = p.M[P.j];
-      if (r.mNew != mOld && media[mOld].ri == P.ri && in_count_range(r.mNew, p)) ++P.transitions;
-    }
+    if (FRESNEL && P.ri != media[r.mNew].ri) r.fresnel = true;
+    else if (p.criteriaActive) count_transition(P, p, media, r.mNew);
   }
-  r.s = s;
-  r.absorb = -P.weight * expm1f(-P.mua * s);
-  P.weight -= r.absorb;
+  r.absorb = absorb(P, r.s);
   return r;
 }
 
