@@ -20,7 +20,10 @@ namespace mcm {
 
 enum : int { ST_FETCH = 0, ST_MOVE = 1, ST_SCATTER = 2, ST_FRESNEL = 3, ST_DONE = 4 };
 
-template <bool FRESNEL, bool CRITERIA>
+// INLINE_REPLAY: a packet that is to deposit at its end of life is launched
+// again by death(); otherwise it waits in FETCH with `replay` set and the
+// caller starts it again from its launch record.
+template <bool FRESNEL, bool CRITERIA, bool INLINE_REPLAY = true>
 struct PacketEngine {
   Photon P;
   PacketRng R;
@@ -78,7 +81,8 @@ struct PacketEngine {
       // deposit its absorbed weights scaled by the final weight
       replay = true;
       replayW = P.weight;
-      start(packet, p, med, cdf);
+      if constexpr (INLINE_REPLAY) start(packet, p, med, cdf);
+      else state = ST_FETCH;
     } else {
       replay = false;
       state = ST_FETCH;
@@ -140,7 +144,9 @@ struct PacketEngine {
 
   // One sub-step.  The medium of the voxel entered is requested as soon as the
   // position is known and used after the absorption and the deposit, whose
-  // arithmetic covers the load.
+  // arithmetic covers the load.  (Requesting it a sub-step ahead, from the
+  // boundary that the packet is heading for, was no faster: 10^4 packets 0.90 ms
+  // for 0.86.)
   template <class Sink>
   MCM_FN void do_move(const McParams& p, const Medium* med, const uint8_t* cdf, Sink& sink) {
     if (P.substeps >= kMaxSubsteps) {
@@ -182,12 +188,10 @@ struct PacketEngine {
 
   template <class Sink>
   MCM_FN void do_scatter(const McParams& p, const Medium* med, const uint8_t* cdf, Sink& sink) {
-    roulette(P, R);
-    if (!P.alive) {
+    if (!roulette_scatter(P, p, p.cdfs, CRITERIA ? (int)p.M[P.j] : 0, R)) {
       death(p, med, cdf, sink);
       return;
     }
-    scatter(P, p, p.cdfs, CRITERIA ? (int)p.M[P.j] : 0, R);
     state = P.stepLeft > 0.f ? ST_MOVE : ST_SCATTER;
   }
 };

@@ -26,7 +26,7 @@
 // transport's: FETCH (take the next packet number, one atomic per wavefront,
 // or the lane's own packet again for pass 2), MOVE (one voxel sub-step),
 // SCATTER (roulette + deflection), FRESNEL (an interface).  Each iteration the wavefront runs one state for the lanes in
-// it (MOVE while at least half of the live lanes want to move, otherwise the
+// it (MOVE while 30 % of the live lanes want to move, otherwise the
 // state with more waiting lanes), so a wavefront never waits for its
 // longest-lived packet before starting others.
 //
@@ -84,6 +84,10 @@ __device__ inline unsigned long long grad_bcast64(unsigned long long v, int src)
   return ((unsigned long long)hi << 32) | lo;
 }
 
+// Lanes in MOVE that keep the wavefront there, as a share of the live ones
+// (mcm_mc_plan::moveFrac).
+constexpr float kStay = 0.3f;
+
 // Gradient terms that a lane parks in LDS and the wavefront then adds with 8
 // lanes a packet (the transport's DeferSink has the reason); odd pitch against
 // bank conflicts.
@@ -132,7 +136,8 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
   uint64_t k = 0;
   double D = 0.0, tau = 0.0;  // pass 1: box deposit, optical depth; pass 2: box deposits still to come
   uint32_t K = 0;
-  int nTerms = 0, pendJ = 0, pendM = 0;
+  int nTerms = 0, parked = 0;  // terms parked by the lane, by any lane at most
+  int pendJ = 0, pendM = 0;
   bool boxed = false;  // the packet's voxel is in the box (and the packet in the volume)
   double* const grad = g.grad + (size_t)(xcd() % g.copies) * g.LB;
   // spread few packets over the wavefronts (launch_blocks)
@@ -165,9 +170,22 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
     }
     set_voxel(j, m, mua);
   };
+  // the packet goes on with its next state, or its pass ended
+  auto settle = [&]() {
+    st = P.stepLeft > 0.f ? G_MOVE : G_SCATTER;
+    if (!P.alive) {
+      st = G_FETCH;
+      if (!pass2) {
+        const double S = (double)K - tau;
+        sSum[0][t] += D;
+        sSum[1][t] += D * D;
+        sSum[2][t] += D * S;
+        sSum[3][t] += (D * S) * (D * S);
+        again = D > 0.0 && g.replay;
+      }
+    }
+  };
   for (;;) {
-    // a lane parks at most one term per iteration
-    if (__ballot(nTerms == kTerms)) add_terms(grad, sTerms, nTerms);
     const unsigned long long bFetch = __ballot(st == G_FETCH);
     const unsigned long long bMove = __ballot(st == G_MOVE);
     const unsigned long long bScat = __ballot(st == G_SCATTER);
@@ -176,16 +194,16 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
     const int active = cF + cM + cS + cR;
     if (active == 0) break;
     int phase = G_MOVE;
-    if (2 * cM < active) {
+    const int stay = max(1, (int)ceilf(kStay * (float)active));
+    if (cM < stay) {
       int best = cM;
       if (cS > best) { best = cS; phase = G_SCATTER; }
       if (FRESNEL && cR > best) { best = cR; phase = G_FRESNEL; }
       if (cF > best) phase = G_FETCH;
     }
-    bool moved = false;  // the lane's packet goes on with its next state, or ended
-    if (phase == G_MOVE) {
+    if (phase == G_MOVE) do {
       if (st == G_MOVE) {
-        moved = true;
+        bool moved = true;
         if (P.substeps >= kMaxSubsteps) {
           P.alive = false;
         } else {
@@ -221,19 +239,25 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
             }
           }
         }
+        if (moved) settle();
       }
-    } else if (phase == G_SCATTER) {
+      // a lane parks at most one term per sub-step
+      if (++parked >= kTerms && __ballot(nTerms == kTerms)) {
+        add_terms(grad, sTerms, nTerms);
+        parked = 0;
+      }
+    } while (__popcll(__ballot(st == G_MOVE)) >= stay);
+    else if (phase == G_SCATTER) {
       if (st == G_SCATTER) {
-        moved = true;
         ++K;  // the flight ended in an interaction
-        roulette(P, R);
-        if (P.alive) scatter(P, p, p.cdfs, 0, R);
+        roulette_scatter(P, p, p.cdfs, 0, R);
+        settle();
       }
     } else if (FRESNEL && phase == G_FRESNEL) {
       if (st == G_FRESNEL) {
-        moved = true;
         fresnel(P, p, sMed, pendJ, pendM, R);
         enter(pendJ, pendM, g.muaMap ? g.muaMap[pendJ] : 0.f);
+        settle();
       }
     } else {
       const unsigned long long bNew = __ballot(st == G_FETCH && !again);
@@ -264,21 +288,7 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
           set_crossing_lengths(P, p);
           const int j = voxel_of(p, P.i);
           set_voxel(j, p.M[j], g.muaMap ? g.muaMap[j] : 0.f);
-          moved = true;
-        }
-      }
-    }
-    if (moved) {
-      st = P.stepLeft > 0.f ? G_MOVE : G_SCATTER;
-      if (!P.alive) {  // the pass ended
-        st = G_FETCH;
-        if (!pass2) {
-          const double S = (double)K - tau;
-          sSum[0][t] += D;
-          sSum[1][t] += D * D;
-          sSum[2][t] += D * S;
-          sSum[3][t] += (D * S) * (D * S);
-          again = D > 0.0 && g.replay;
+          settle();
         }
       }
     }

@@ -18,7 +18,8 @@
 //   of the live lanes want to move, otherwise whichever state has the most
 //   lanes waiting.  Lanes waiting for a rarer state idle briefly and are then
 //   served together, which keeps SIMD occupancy high for the expensive
-//   scatter and interface code.
+//   scatter and interface code.  While the vote stays with MOVE only its own
+//   lanes are counted again.
 //
 //   Per-medium optical constants live in LDS.  Deposits are parked in LDS and
 //   added to the FP64 fluence grid, kept in bricks of voxels, with hardware
@@ -33,9 +34,11 @@
 //
 //   Deposition criteria evaluated at end of life (MCmatlab.c:262-264) are
 //   handled by replay instead of per-packet deposit records: when a packet
-//   dies meeting the criteria, the lane re-launches the same packet number,
-//   whose stream reproduces the trajectory exactly, and deposits the
-//   absorbed weights scaled by the final weight.
+//   dies meeting the criteria, the lane fetches the same packet's launch record
+//   again, whose stream reproduces the trajectory exactly, and deposits the
+//   absorbed weights scaled by the final weight.  (With launchPhoton inlined
+//   for that, the kernel took 172 registers and 112 bytes of scratch, two
+//   wavefronts a SIMD: 4 10^5 packets 33 ms, now 26.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -242,13 +245,15 @@ struct RingSlots {
 // (measured: 0.565 a deposit, at least 0.5) where one deposit per lane and
 // instruction would take 16.  Rings of 8 take as long.  A parked deposit is the
 // absorbed weight of one sub-step, a float.
+template <bool ESCAPES>
 struct DeferSink : DeviceSink {
-  static constexpr bool kDeferEscapes = true;
+  static constexpr bool kDeferEscapes = ESCAPES;
   EscapeRecord* rec;
   int item;
   RingSlots* ring;
-  int nRing;
-  __device__ DeferSink(const McParams& p, EscapeRecord* r) : DeviceSink(p), rec(r), item(0), ring(nullptr), nRing(0) {}
+  int nRing;   // parked by the lane,
+  int parked;  // by any lane of the wavefront at most
+  __device__ DeferSink(const McParams& p, EscapeRecord* r) : DeviceSink(p), rec(r), item(0), ring(nullptr), nRing(0), parked(0) {}
   // Issues the deposits of the whole wavefront (every lane calls it).
   // PER_LANE: the lanes' fluence slices differ (batched launches).
   template <bool PER_LANE>
@@ -270,6 +275,7 @@ struct DeferSink : DeviceSink {
       }
     }
     nRing = 0;
+    parked = 0;
   }
   __device__ void deposit(int j, float v) {
     ring->d[threadIdx.x * kRingPitch + nRing] = make_uint2((unsigned)j, __float_as_uint(v));
@@ -282,17 +288,6 @@ struct DeferSink : DeviceSink {
     rec[slot] = E;
   }
 };
-
-template <class Sink>
-__device__ inline Sink make_sink(const McParams& p, EscapeRecord* r);
-template <>
-__device__ inline DeviceSink make_sink<DeviceSink>(const McParams& p, EscapeRecord*) {
-  return DeviceSink(p);
-}
-template <>
-__device__ inline DeferSink make_sink<DeferSink>(const McParams& p, EscapeRecord* r) {
-  return DeferSink(p, r);
-}
 
 // launchPhoton for packets firstPacket .. firstPacket + nPackets - 1 into
 // rec[0 .. nPackets-1]; clears the packets' escape record slots.  A launch
@@ -329,7 +324,7 @@ __global__ void __launch_bounds__(256) mc_launch_packets(McParams p, McLaunch lp
     LaunchRecord L;
     pack_launch(P, R, ok, L);
     rec[k] = L;
-    esc[k].c = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (esc) esc[k].c = make_float4(0.f, 0.f, 0.f, 0.f);
     if (!ok) atomicOr(&lp.ctr->aborted, 1u);
   }
 }
@@ -382,7 +377,7 @@ __global__ void __launch_bounds__(256) mc_tally_escapes(McParams p, McLaunch lp,
 }
 
 template <bool FRESNEL, bool CRITERIA, int BATCH>
-__global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p, McLaunch lp, McBatch bt, const LaunchRecord* __restrict__ launches,
+__global__ void __launch_bounds__(256, 4) mc_transport(McParams p, McLaunch lp, McBatch bt, const LaunchRecord* __restrict__ launches,
                                                     EscapeRecord* __restrict__ escapes) {
   static_assert(!(BATCH != kPlain && CRITERIA), "batched launches run without deposition criteria");
   // the media tables of the wavelength, or of every item, behind the items'
@@ -401,12 +396,11 @@ __global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p
   __syncthreads();
 
   const int lane = __lane_id();
-  PacketEngine<FRESNEL, CRITERIA> E;
+  PacketEngine<FRESNEL, CRITERIA, false> E;
   E.init(lp.key0, lp.key1, lp.stream);
-  using Sink = typename std::conditional<CRITERIA, DeviceSink, DeferSink>::type;
-  Sink sink = make_sink<Sink>(p, escapes);
-  __shared__ typename std::conditional<CRITERIA, char, RingSlots>::type sRing;
-  if constexpr (!CRITERIA) sink.ring = &sRing;
+  DeferSink<!CRITERIA> sink(p, escapes);
+  __shared__ RingSlots sRing;
+  sink.ring = &sRing;
   // the media tables of the lane's work item (the launch's in a plain launch)
   const Medium* med = sMed;
   const uint8_t* cdf = sCdf;
@@ -436,11 +430,6 @@ __global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p
   }
 
   for (;;) {
-    if constexpr (!CRITERIA) {
-      // a lane parks at most one deposit per iteration: drain every ring once
-      // one of them is full
-      if (__ballot(sink.nRing == kRing)) sink.template drain<BATCH == kBatch>();
-    }
     const int st = E.state;
     const unsigned long long bFetch = __ballot(st == ST_FETCH);
     const unsigned long long bMove = __ballot(st == ST_MOVE);
@@ -479,10 +468,18 @@ __global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p
       if (cF > best) phase = ST_FETCH;
     }
     if (phase == ST_MOVE) {
-      if (st == ST_MOVE) {
-        ++nSub;
-        E.do_move(pr, med, cdf, sink);
-      }
+      // MOVE stays the choice while `stay` lanes are in it: the others' states
+      // don't change meanwhile
+      const int stay = max(1, (int)ceilf(lp.moveFrac * (float)active));
+      do {
+        if (E.state == ST_MOVE) {
+          ++nSub;
+          E.do_move(pr, med, cdf, sink);
+        }
+        // a lane parks at most one deposit per sub-step: drain every ring once
+        // one of them is full
+        if (++sink.parked >= kRing && __ballot(sink.nRing == kRing)) sink.template drain<BATCH == kBatch>();
+      } while (__popcll(__ballot(E.state == ST_MOVE)) >= stay);
     } else if (phase == ST_SCATTER) {
       if (st == ST_SCATTER) {
         ++nScat;
@@ -493,6 +490,7 @@ __global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p
         ++nIf;
         E.do_fresnel(pr, med, cdf, sink);
       }
+      if (CRITERIA && ++sink.parked >= kRing && __ballot(sink.nRing == kRing)) sink.template drain<BATCH == kBatch>();
     } else {
       // parked deposits belong to the item a lane leaves
       if constexpr (BATCH == kBatch) sink.template drain<true>();
@@ -524,22 +522,27 @@ __global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p
         }
         continue;
       }
-      if (lane == leader) {
-        base = atomicAdd(&lp.ctr->nextPacket, (unsigned long long)cF);
-        if (atomicAdd(&lp.ctr->aborted, 0u)) base = lp.nPackets;  // a failed launch stops the run
+      // (packets to be replayed need no number)
+      const unsigned long long bNew = CRITERIA ? __ballot(st == ST_FETCH && !E.replay) : bFetch;
+      if (!CRITERIA || bNew) {
+        const int first = CRITERIA ? __ffsll((long long)bNew) - 1 : leader;
+        if (lane == first) {
+          base = atomicAdd(&lp.ctr->nextPacket, (unsigned long long)__popcll(bNew));
+          if (atomicAdd(&lp.ctr->aborted, 0u)) base = lp.nPackets;  // a failed launch stops the run
+        }
+        base = bcast64(base, first);
       }
-      base = bcast64(base, leader);
       if (st == ST_FETCH) {
-        const unsigned long long k = base + (unsigned long long)__popcll(bFetch & ((1ull << lane) - 1ull));
+        unsigned long long k = base + (unsigned long long)__popcll(bNew & ((1ull << lane) - 1ull));
+        const bool again = CRITERIA && E.replay;
+        if (again) k = E.slot;
         if (k >= lp.nPackets) {
           E.state = ST_DONE;
         } else {
-          E.replay = false;
           bool ok;
           E.slot = (uint32_t)k;
-          if constexpr (CRITERIA) {
-            ok = E.start(lp.firstPacket + k, pr, med, cdf);
-          } else if constexpr (BATCH != kPlain) {
+          const LaunchRecord L = launches[k];
+          if constexpr (BATCH != kPlain) {
             const unsigned long long g = lp.firstPacket + k;
             const int it = batch_item(g, sCum, bt.nItems);
             med = sMed + it * bt.nM;
@@ -549,12 +552,11 @@ __global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p
             E.R.stream = bt.stream[it];
             sink.NFR = bt.NFR + (xcd() % bt.copies) * bt.copyStride + (size_t)it * bt.L;
             sink.item = it;
-            const LaunchRecord L = launches[k];
             ok = E.start_from(g - sCum[it], L, pr, med, cdf);
           } else {
-            const LaunchRecord L = launches[k];
             ok = E.start_from(lp.firstPacket + k, L, pr, med, cdf);
           }
+          if (again) continue;
           if (ok) {
             ++nLaunched;
           } else {
@@ -565,8 +567,7 @@ __global__ void __launch_bounds__(256, CRITERIA ? 1 : 4) mc_transport(McParams p
       }
     }
   }
-  sink.flush();
-  if constexpr (!CRITERIA) sink.template drain<BATCH == kBatch>();
+  sink.template drain<BATCH == kBatch>();
   if (nLaunched) atomicAdd(&lp.ctr->launched, nLaunched);
   if (sink.nCollected) atomicAdd(&lp.ctr->collected, sink.nCollected);
   if (nSub) atomicAdd(&lp.ctr->substeps, nSub);
@@ -676,11 +677,7 @@ __global__ void mc_example_paths(McParams p, McLaunch lp, int64_t nPaths, double
           if (P.alive) new_voxel_properties(P, p, sMed, sCdf);
         }
       }
-      if (P.alive) roulette(P, R);
-      if (P.alive) {
-        scatter(P, p, p.cdfs, p.M[P.j], R);
-        record(false);
-      }
+      if (P.alive && roulette_scatter(P, p, p.cdfs, p.M[P.j], R)) record(false);
     }
     if (started) {
       if (p.evalAtEnd && !criteria_met(P, p)) {
@@ -818,12 +815,6 @@ int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed,
   const McBatch& B = bt ? *bt : none;
   const dim3 b(pl->threads), g(launch_blocks(pl, kind == kPlain ? pl->blocks : blocks_items, n));
   MCM_HIP(hipMemsetAsync(pl->counters.p, 0, sizeof(unsigned long long), s));  // nextPacket
-  if (cr) {
-    if (fr) hipLaunchKernelGGL((mc_transport<true, true, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, nullptr, nullptr);
-    else hipLaunchKernelGGL((mc_transport<false, true, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, nullptr, nullptr);
-    MCM_HIP(hipGetLastError());
-    return MCM_OK;
-  }
   int rc = ensure_records(pl, n);
   if (rc) return rc;
   LaunchRecord* L = pl->launchRec.as<LaunchRecord>();
@@ -845,10 +836,14 @@ int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed,
     else hipLaunchKernelGGL((mc_transport<false, false, kBatch>), g, b, table_bytes(B.nItems, B.nM), s, pl->prm, lp, B, L, E);
     if (tally) hipLaunchKernelGGL(mc_tally_escapes<kBatch>, g, b, 0, s, pl->prm, lp, B, E);
   } else {
-    hipLaunchKernelGGL(mc_launch_packets<kPlain>, g, b, 0, s, pl->prm, lp, B, L, E);
-    if (fr) hipLaunchKernelGGL((mc_transport<true, false, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, L, E);
+    hipLaunchKernelGGL(mc_launch_packets<kPlain>, g, b, 0, s, pl->prm, lp, B, L, cr ? nullptr : E);
+    if (cr) {
+      // criteria: the transport tallies inline
+      if (fr) hipLaunchKernelGGL((mc_transport<true, true, kPlain>), g, b, table_bytes(0, T.nM), s, pl->prm, lp, B, L, nullptr);
+      else hipLaunchKernelGGL((mc_transport<false, true, kPlain>), g, b, table_bytes(0, T.nM), s, pl->prm, lp, B, L, nullptr);
+    } else if (fr) hipLaunchKernelGGL((mc_transport<true, false, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, L, E);
     else hipLaunchKernelGGL((mc_transport<false, false, kPlain>), g, b, table_bytes(0, pl->T.nM), s, pl->prm, lp, B, L, E);
-    if (tally) hipLaunchKernelGGL(mc_tally_escapes<kPlain>, g, b, 0, s, pl->prm, lp, B, E);
+    if (tally && !cr) hipLaunchKernelGGL(mc_tally_escapes<kPlain>, g, b, 0, s, pl->prm, lp, B, E);
   }
   MCM_HIP(hipGetLastError());
   return MCM_OK;
@@ -971,7 +966,7 @@ int mcm_mc_plan_create(const mcm_mc_input* in, mcm_mc_plan** out) {
   // voxels along an axis) or their indices
   const int nb[3] = {(T.nx + 3) / 4, (T.ny + 3) / 4, (T.nz + 3) / 4};
   const int64_t padded = (int64_t)nb[0] * nb[1] * nb[2] * 64;
-  const bool bricks = padded <= 2 * T.L && padded < ((int64_t)1 << 31);
+  const bool bricks = padded <= 2 * T.L && padded < ((int64_t)1 << 31) && (int64_t)nb[0] * nb[1] < (1 << 24);
   const VoxelMap map{T.nx, T.ny, bricks ? nb[0] : 0, bricks ? nb[0] * nb[1] : 0};
   T.base.nbx = map.nbx;
   T.base.nbxy = map.nbxy;

@@ -125,6 +125,15 @@ MCM_FN int clampi(int x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : x
 // voxel coordinate of position i on an axis of n voxels (no branch; n < 2^24)
 MCM_FN int clamp_axis(float i, int n) { return (int)fminf(fmaxf(floorf(i), 0.f), (float)(n - 1)); }
 
+// product of numbers below 2^24 (full rate; a 32-bit product is a quarter of it)
+MCM_FN unsigned mul24(unsigned a, unsigned b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __umul24(a, b);
+#else
+  return a * b;
+#endif
+}
+
 // Index of voxel (x, y, z) in the order of M and the fluence.  A packet walks
 // from voxel to neighbouring voxel, so both are kept in bricks: 64 bytes of M
 // are one 4 x 4 x 4 brick (a packet stays on the cache line for 4 voxels on
@@ -136,7 +145,8 @@ MCM_FN int brick_index(int x, int y, int z, int nbx, int nbxy) {
   // bits 0 and 3 as (5 v) & 9
   const unsigned s = (((unsigned)x & 3u) | ((unsigned)y & 3u) << 8 | ((unsigned)z & 3u) << 16) * 5u;
   const unsigned in = (s & 9u) | (s >> 7 & 18u) | (s >> 14 & 36u);
-  return (int)((unsigned)((z >> 2) * nbxy + (y >> 2) * nbx + (x >> 2)) << 6 | in);
+  const unsigned brick = mul24((unsigned)z >> 2, (unsigned)nbxy) + mul24((unsigned)y >> 2, (unsigned)nbx) + ((unsigned)x >> 2);
+  return (int)(brick << 6 | in);
 }
 MCM_FN int voxel_index(const McParams& p, int x, int y, int z) {
   return p.nbx ? brick_index(x, y, z, p.nbx, p.nbxy) : (z * p.n[1] + y) * p.n[0] + x;
@@ -749,33 +759,54 @@ MCM_FN EscapeResult check_escape(Photon& P, const McParams& p) {
   return e;
 }
 
-// checkRoulette (MCmatlablib.c:1124-1133)
-MCM_FN void roulette(Photon& P, PacketRng& R) {
-  if (P.weight < kThreshold) {
-    if (R.next() <= kChance) P.weight /= kChance;
-    else P.alive = false;
+// checkRoulette (MCmatlablib.c:1124-1133) and, for a packet that survives it,
+// scatterPhoton (:1138-1184).  Returns whether it did.  The packet's draws, in
+// the stream's order, are taken together (PacketRng::take): one for the
+// roulette of a light packet, none to two for the polar angle, one for the
+// azimuth and one for the step.
+MCM_FN bool roulette_scatter(Photon& P, const McParams& p, const float* cdfs, int mCur, PacketRng& R) {
+  const float g = P.g;
+  const bool table = isnan(g), light = P.weight < kThreshold;
+  const int nPolar = table ? 2 : fabsf(g) == 1.f ? 0 : 1;
+  uint32_t w[4];
+  uint32_t wRoulette;
+  bool pending = light;
+  if (light && table) {  // five draws
+    wRoulette = R.next_word();
+    pending = false;
   }
-}
-
-// scatterPhoton (MCmatlablib.c:1138-1184)
-MCM_FN void scatter(Photon& P, const McParams& p, const float* cdfs, int mCur, PacketRng& R) {
-  float ct;
-  if (isnan(P.g)) {
-    const float* D = cdfs + P.cdf * kCdfSize;
-    const int jt = table_search(R.next(), kCdfSize - 1, D);
-    ct = cosf(((float)jt + R.next()) * kPi / (float)(kCdfSize - 1));
-  } else {
-    const float g = P.g;
-    if (fabsf(g) == 1.f) ct = g;
-    else if (fabsf(g) <= 3.4526698e-04f) ct = 2.f * R.next() - 1.f;  // sqrt(FLT_EPSILON)
+  R.take(w, nPolar + 2 + (pending ? 1 : 0));
+  if (pending) {
+    wRoulette = w[0];
+    w[0] = w[1];
+    w[1] = w[2];
+    w[2] = w[3];
+  }
+  if (light) {
+    if (R.uniform(wRoulette) <= kChance) P.weight /= kChance;
     else {
-      const float t = (1.f - g * g) / (1.f - g + 2.f * g * R.next());
+      P.alive = false;
+      return false;
+    }
+  }
+  float ct;
+  if (table) {
+    const float* D = cdfs + P.cdf * kCdfSize;
+    const int jt = table_search(R.uniform(w[0]), kCdfSize - 1, D);
+    ct = cosf(((float)jt + R.uniform(w[1])) * kPi / (float)(kCdfSize - 1));
+  } else {
+    if (fabsf(g) == 1.f) ct = g;
+    else if (fabsf(g) <= 3.4526698e-04f) ct = 2.f * R.uniform(w[0]) - 1.f;  // sqrt(FLT_EPSILON)
+    else {
+      const float t = (1.f - g * g) / (1.f - g + 2.f * g * R.uniform(w[0]));
       ct = (1.f + g * g - t * t) / (2.f * g);
     }
   }
+  const float azimuth = R.uniform(nPolar == 0 ? w[0] : nPolar == 1 ? w[1] : w[2]);
+  const float step = R.uniform(nPolar == 0 ? w[1] : nPolar == 1 ? w[2] : w[3]);
   const float st = sqrtf(fmaxf(0.f, 1.f - ct * ct));
   float sp, cp;
-  sincosf(2.f * kPi * R.next(), &sp, &cp);
+  sincosf(2.f * kPi * azimuth, &sp, &cp);
   const float rho2 = P.u[0] * P.u[0] + P.u[1] * P.u[1];
   if (fabsf(P.u[2]) < 1.f && rho2 > 0.f) {
     const float rho = sqrtf(rho2);
@@ -792,8 +823,9 @@ MCM_FN void scatter(Photon& P, const McParams& p, const float* cdfs, int mCur, P
   }
   for (int a = 0; a < 3; ++a) P.D[a] = boundary_distance(P.i[a], P.u[a], p.d[a]);
   set_crossing_lengths(P, p);
-  P.stepLeft = -logf(R.next());
+  P.stepLeft = -logf(step);
   if (p.criteriaActive && in_count_range(mCur, p)) ++P.scatterings;
+  return true;
 }
 
 }  // namespace mcm

@@ -66,7 +66,37 @@ struct PacketRng {
     return w;
   }
   // uniform float on (0, 1]
-  MCM_FN float next() { return (float)((next_word() >> 8) + 1u) * (1.0f / 16777216.0f); }
+  MCM_FN static float uniform(uint32_t w) { return (float)((w >> 8) + 1u) * (1.0f / 16777216.0f); }
+  MCM_FN float next() { return uniform(next_word()); }
+  // The next n (0..4) words in w[0..n-1], from at most one new block.  n calls
+  // of next_word() would inline n blocks, and lanes of a wavefront that are at
+  // different words of theirs would run all of them (20 quarter-rate
+  // multiplications each).
+  MCM_FN void take(uint32_t w[4], int n) {
+    const int h = have;
+    w[0] = b0;
+    w[1] = b1;
+    w[2] = b2;
+    w[3] = b3;
+    if (h < n) {
+      uint32_t c[4] = {block++, plo, phi, stream};
+      philox4x32_10(c, key0, key1);
+      w[0] = h > 0 ? w[0] : c[0];
+      w[1] = h > 1 ? w[1] : h == 1 ? c[0] : c[1];
+      w[2] = h > 2 ? w[2] : h == 2 ? c[0] : h == 1 ? c[1] : c[2];
+      w[3] = h == 3 ? c[0] : h == 2 ? c[1] : h == 1 ? c[2] : c[3];
+      const int d = n - h;  // words of the new block taken
+      b0 = d == 1 ? c[1] : d == 2 ? c[2] : c[3];
+      b1 = d == 1 ? c[2] : c[3];
+      b2 = c[3];
+      have = 4 - d;
+    } else {
+      b0 = n == 0 ? b0 : n == 1 ? b1 : n == 2 ? b2 : b3;
+      b1 = n == 0 ? b1 : n == 1 ? b2 : b3;
+      b2 = n == 0 ? b2 : b3;
+      have = h - n;
+    }
+  }
   // uniform double on (0, 1] with 53 random bits (3D-source voxel choice)
   MCM_FN double next53() {
     const uint64_t hi = next_word() >> 5, lo = next_word() >> 6;  // 27 + 26 bits

@@ -70,6 +70,7 @@ def test_fluence_of_a_pure_absorber_by_column(api, shape):
 
 @pytest.mark.parametrize("name,n,cut", [
     ("pencil_bt1", 1, 1), ("pencil_bt1", 65, 64), ("pencil_bt3", 1025, 17), ("fresnel_bt1", 20000, 1030), ("planewave_bt2", 70001, 65536),
+    ("criteria_scatter", 66, 65), ("criteria_collected", 5000, 1023), ("criteria_now", 5000, 64),
     ("pencil_bt1", 300000, 299999)])
 def test_cutting_a_run_changes_nothing(api, name, n, cut):
     """Launches that leave lanes empty, fill one wavefront or one workgroup per
