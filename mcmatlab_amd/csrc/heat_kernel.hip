@@ -1708,6 +1708,7 @@ struct mcm_heat_plan {
   double facDt = 0;
   bool factored(double dt) const { return facReady && facDt == dt; }
   double constR = 0, constC = 0;
+  HostStage hostStage;
   int64_t graphSteps = 32;    // steps per captured graph (0: launch every step)
   std::vector<HeatGraph> graphs;
   void drop_graphs() {
@@ -2150,28 +2151,27 @@ template <typename RT>
 int download(mcm_heat_plan* P, mcm_heat_output* out) {
   const int tpb = 256;
   const unsigned nb = (unsigned)((P->L + tpb - 1) / tpb);
+  int rc = MCM_OK;
   MCM_HIP(hipStreamSynchronize(P->stream));
   if (out->T || out->T_f64) {
     hipLaunchKernelGGL(heat_store<RT>, dim3(nb), dim3(tpb), 0, P->stream, (const RT*)P->T1.p, (float*)P->stage32.p,
                        (double*)(out->T_f64 ? P->stage64.p : nullptr), P->L);
     MCM_HIP(hipGetLastError());
-    if (out->T) MCM_HIP(hipMemcpyAsync(out->T, P->stage32.p, (size_t)P->L * 4, hipMemcpyDeviceToHost, P->stream));
-    if (out->T_f64) MCM_HIP(hipMemcpyAsync(out->T_f64, P->stage64.p, (size_t)P->L * 8, hipMemcpyDeviceToHost, P->stream));
-    MCM_HIP(hipStreamSynchronize(P->stream));
+    if (out->T && (rc = P->hostStage.download(out->T, P->stage32.p, (size_t)P->L * 4, P->device, P->stream))) return rc;
+    if (out->T_f64 && (rc = P->hostStage.download(out->T_f64, P->stage64.p, (size_t)P->L * 8, P->device, P->stream))) return rc;
   }
   if (P->calcDamage && (out->Omega || out->Omega_f64)) {
     hipLaunchKernelGGL(heat_store<RT>, dim3(nb), dim3(tpb), 0, P->stream, (const RT*)P->Om.p, (float*)P->stage32.p,
                        (double*)(out->Omega_f64 ? P->stage64.p : nullptr), P->L);
     MCM_HIP(hipGetLastError());
-    if (out->Omega) MCM_HIP(hipMemcpyAsync(out->Omega, P->stage32.p, (size_t)P->L * 4, hipMemcpyDeviceToHost, P->stream));
-    if (out->Omega_f64) MCM_HIP(hipMemcpyAsync(out->Omega_f64, P->stage64.p, (size_t)P->L * 8, hipMemcpyDeviceToHost, P->stream));
-    MCM_HIP(hipStreamSynchronize(P->stream));
+    if (out->Omega && (rc = P->hostStage.download(out->Omega, P->stage32.p, (size_t)P->L * 4, P->device, P->stream))) return rc;
+    if (out->Omega_f64 && (rc = P->hostStage.download(out->Omega_f64, P->stage64.p, (size_t)P->L * 8, P->device, P->stream))) return rc;
   } else if (!P->calcDamage && out->Omega) {
     out->Omega[0] = NAN;
   }
   if (P->nS && P->sensorsRecorded <= P->stepsDone) {
     // the current state's column (steps record the state they start from)
-    int rc = ensure_sensor_capacity(P, P->stepsDone + 1);
+    rc = ensure_sensor_capacity(P, P->stepsDone + 1);
     if (rc) return rc;
     if ((rc = record_sensors<RT>(P, P->stepsDone))) return rc;
     P->sensorsRecorded = P->stepsDone + 1;

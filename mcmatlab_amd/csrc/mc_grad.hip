@@ -406,7 +406,7 @@ extern "C" int mcm_mc_grad_run(mcm_mc_plan* pl, const mcm_mc_grad_input* in, mcm
   if (out->dJ_dmua) {
     hipLaunchKernelGGL(mc_grad_output, dim3(gL), dim3(256), 0, s, pl->gradLin.as<double>(), pl->gradOut.as<double>(), copies, LB, voxel_map(pl), power, N, T.L);
     MCM_HIP(hipGetLastError());
-    MCM_HIP(hipMemcpyAsync(out->dJ_dmua, pl->gradLin.p, (size_t)T.L * sizeof(double), hipMemcpyDeviceToHost, s));
+    if ((rc = pl->stage.download(out->dJ_dmua, pl->gradLin.p, (size_t)T.L * sizeof(double), pl->device, s))) return rc;
   }
   MCM_HIP(hipStreamSynchronize(s));
   double sums[4];

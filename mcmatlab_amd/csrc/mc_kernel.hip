@@ -610,6 +610,14 @@ __global__ void mc_fold_replicas(double* dep, int64_t L, int R) {
   dep[j] = s;
 }
 
+// Unit interface normals from their polar and azimuthal angles, in FP64.
+__global__ void mc_unit_normals(float4* nri, const float2* angles, int64_t L) {
+  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= L) return;
+  const double th = angles[j].x, ph = angles[j].y;
+  nri[j] = make_float4((float)(sin(th) * cos(ph)), (float)(sin(th) * sin(ph)), (float)cos(th), 1.f);
+}
+
 __global__ void mc_fill_normal_ri(float4* nri, const uint8_t* M, const Medium* media, int64_t L) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= L) return;
@@ -885,8 +893,7 @@ int finish_item(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, double* nfr, int
     hipLaunchKernelGGL(mc_normalize_nfr, dim3((unsigned)nb), dim3(tpb), 0, s, nfr, copies, stride, pl->Mlin.as<uint8_t>(),
                        pl->muaNorm.as<double>() + (size_t)iL * T.nM, T.V * normfactor, pl->nfrOut.as<float>(), voxel_map(pl), T.L);
     MCM_HIP(hipGetLastError());
-    MCM_HIP(hipMemcpyAsync(o.NFR, pl->nfrOut.p, (size_t)T.L * sizeof(float), hipMemcpyDeviceToHost, s));
-    MCM_HIP(hipStreamSynchronize(s));
+    if ((rc = pl->stage.download(o.NFR, pl->nfrOut.p, (size_t)T.L * sizeof(float), pl->device, s))) return rc;
   }
   if (T.base.useLC) {
     const int64_t LLC = (int64_t)T.lcRes0 * T.lcRes0;
@@ -928,7 +935,7 @@ extern "C" {
 int mcm_mc_output_sizes(const mcm_mc_input* in, mcm_mc_sizes* sz) {
   if (!in || !sz) return fail(MCM_ERR_INVALID_ARGUMENT, "null argument");
   McTables T;
-  const std::string err = build_mc_tables(in, T);
+  const std::string err = build_mc_tables(in, T, false);
   if (!err.empty()) return fail(MCM_ERR_INVALID_ARGUMENT, "%s", err.c_str());
   std::memset(sz, 0, sizeof *sz);
   sz->NFR = T.calcNFR ? T.L * T.nL : 0;
@@ -953,7 +960,7 @@ int mcm_mc_plan_create(const mcm_mc_input* in, mcm_mc_plan** out) {
   if (!in || !out) return fail(MCM_ERR_INVALID_ARGUMENT, "null argument");
   *out = nullptr;
   std::unique_ptr<mcm_mc_plan> pl(new mcm_mc_plan());
-  const std::string err = build_mc_tables(in, pl->T);
+  const std::string err = build_mc_tables(in, pl->T, false);
   if (!err.empty()) return fail(MCM_ERR_INVALID_ARGUMENT, "%s", err.c_str());
   int rc = use_device(in->GPUdevice);
   if (rc) return rc;
@@ -975,7 +982,13 @@ int mcm_mc_plan_create(const mcm_mc_input* in, mcm_mc_plan** out) {
   hipLaunchKernelGGL(mc_to_bricks<uint8_t>, dim3((unsigned)((T.L + 255) / 256)), dim3(256), 0, s, pl->M.as<uint8_t>(), pl->Mlin.as<uint8_t>(),
                      map, T.L);
   MCM_HIP(hipGetLastError());
-  if (T.fresnelPossible && (rc = upload(pl->normals, T.normals.data(), T.normals.size(), s))) return rc;
+  DevBuf angles;
+  if (T.fresnelPossible) {
+    if ((rc = upload(angles, (const float2*)in->interfaceNormals, (size_t)T.L, s)) || (rc = upload<float4>(pl->normals, nullptr, (size_t)T.L, s)))
+      return rc;
+    hipLaunchKernelGGL(mc_unit_normals, dim3((unsigned)((T.L + 255) / 256)), dim3(256), 0, s, pl->normals.as<float4>(), angles.as<float2>(), T.L);
+    MCM_HIP(hipGetLastError());
+  }
   if ((rc = upload(pl->media, T.media.data(), T.media.size(), s))) return rc;
   if ((rc = upload(pl->cdfIdx, T.cdfIdx.data(), T.cdfIdx.size(), s))) return rc;
   if ((rc = upload(pl->cdfs, T.cdfs.data(), T.cdfs.size(), s))) return rc;
@@ -1078,7 +1091,7 @@ int mcm_mc_plan_normalize(mcm_mc_plan* pl, int64_t iL, mcm_mc_output* out) {
     hipLaunchKernelGGL(mc_normalize_nfr, dim3((unsigned)nb), dim3(tpb), 0, s, pl->NFR.as<double>(), pl->prm.nfrReplicas, pl->prm.LB, pl->Mlin.as<uint8_t>(),
                        pl->muaNorm.as<double>() + (size_t)iL * T.nM, T.V * normfactor, pl->nfrOut.as<float>(), voxel_map(pl), T.L);
     MCM_HIP(hipGetLastError());
-    MCM_HIP(hipMemcpyAsync(out->NFR + (size_t)iL * T.L, pl->nfrOut.p, (size_t)T.L * sizeof(float), hipMemcpyDeviceToHost, s));
+    if (int rc = pl->stage.download(out->NFR + (size_t)iL * T.L, pl->nfrOut.p, (size_t)T.L * sizeof(float), pl->device, s)) return rc;
   }
   std::vector<double> h;
   auto small = [&](DevBuf& b, int64_t n, float* dst, double div) -> int {

@@ -67,6 +67,7 @@ struct mcm_mc_plan {
   int curL = -1;
   uint64_t lastLaunched = 0, lastCollected = 0;
   mcm::McCounters stats{};
+  mcm::HostStage stage;
   ~mcm_mc_plan() {
     if (stream) (void)hipStreamDestroy(stream);
   }
