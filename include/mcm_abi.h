@@ -332,8 +332,9 @@ int mcm_heat_plan_destroy(mcm_heat_plan *plan);
  *            conductivities enter through; chain rule to TC on the caller's
  *            side) [K s],
  * the exact derivatives of the discrete scheme (up to rounding).  States are
- * checkpointed every checkpointEvery steps (0: 100) and recomputed one
- * segment at a time on the way back.  Needs precision MCM_HEAT_FP64, scheme
+ * all kept where they fit in 4 GiB of device memory, else checkpointed every
+ * checkpointEvery steps (0: 100) and recomputed one segment at a time on the
+ * way back.  Needs precision MCM_HEAT_FP64, scheme
  * MCM_HEAT_DGADI and a damage input (Omega). */
 typedef struct mcm_heat_segment {
   int64_t steps;

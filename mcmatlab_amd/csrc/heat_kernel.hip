@@ -1332,15 +1332,18 @@ __global__ void heat_init_keys(unsigned long long* k, int n) {
 // adds dt A exp(.) E / (R theta^2) / 2 to the adjoints of both u and T3.
 
 // adjoint of the step's damage term for the target voxels
+// dJ/dT of the damage of one step (of length dt, from xa to xb) at either end
+__device__ inline double adj_damage(const HeatArgs<double>& a, double dt, int m, double xa, double xb) {
+  const double E = a.E[m], th = (xa + xb) / 2 + a.czero;
+  return dt * exp(a.logA[m] - E / (a.Rgas * th)) * E / (a.Rgas * th * th) / 2;
+}
+
 __global__ void heat_adj_damage(HeatArgs<double> a, const double* __restrict__ x0, const double* __restrict__ x1,
                                 const uint8_t* __restrict__ target, double* lam, int64_t L) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= L || !target[i]) return;
   const int m = a.M[i];
-  const double E = a.E[m];
-  if (E == 0) return;
-  const double th = (x0[i] + x1[i]) / 2 + a.czero;
-  lam[i] += a.dt * exp(a.logA[m] - E / (a.Rgas * th)) * E / (a.Rgas * th * th) / 2;
+  if (a.E[m] != 0) lam[i] += adj_damage(a, a.dt, m, x0[i], x1[i]);
 }
 
 // A_d^T y = r on every line along axis d: lane per line, Thomas recurrence;
@@ -1517,7 +1520,8 @@ template <bool LDS_COEF>
 __global__ void __launch_bounds__(kHeatTPB) heat_adj_combine(HeatArgs<double> a, const double* __restrict__ mu1, const double* __restrict__ mu2,
                                                             const double* __restrict__ mu3, const double* __restrict__ x0,
                                                             const double* __restrict__ x1, const uint8_t* __restrict__ target,
-                                                            double* lamOut, double* dQ, int lightsOn) {
+                                                            double* lamOut, double* dQ, int lightsOn, const double* __restrict__ xm,
+                                                            double dtm) {
   __shared__ double sC[LDS_COEF ? kLdsCoef : 1];
   if (LDS_COEF) {
     for (int k = threadIdx.x; k < a.nM * a.nM * 3; k += blockDim.x) sC[k] = a.c[k];
@@ -1525,8 +1529,11 @@ __global__ void __launch_bounds__(kHeatTPB) heat_adj_combine(HeatArgs<double> a,
   }
   const double* __restrict__ cT = LDS_COEF ? sC : a.c;
   const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = nx * ny;
-  // one z plane per grid row: 32-bit in-plane index arithmetic
-  const int p = blockIdx.x * blockDim.x + threadIdx.x, z = blockIdx.y;
+  // whole workgroups per z plane, so that index arithmetic is 32-bit; each XCD
+  // takes neighbouring planes and rows.  14.2 us at 96 x 80 x 72 with the damage
+  // of the step before; 15.5 and 4.1 as two kernels in launch order.
+  const int perPlane = (nxy + kHeatTPB - 1) / kHeatTPB, blk = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int z = blk / perPlane, p = (blk - z * perPlane) * kHeatTPB + threadIdx.x;
   if (p >= nxy) return;
   const int x = p % nx, y = p / nx;
   const int64_t i = (int64_t)z * nxy + p;
@@ -1550,9 +1557,9 @@ __global__ void __launch_bounds__(kHeatTPB) heat_adj_combine(HeatArgs<double> a,
   }
   double lam = mu1[i] + dt * (t1[0] / 2 + t1[1] + t1[2]) - dt / 2 * t2 - dt / 2 * t3;
   if (target[i] && a.E[m] != 0) {
-    const double E = a.E[m];
-    const double th = (x0[i] + x1[i]) / 2 + a.czero;
-    lam += dt * exp(a.logA[m] - E / (a.Rgas * th)) * E / (a.Rgas * th * th) / 2;
+    lam += adj_damage(a, dt, m, x0[i], x1[i]);
+    // and what heat_adj_damage would add for the step before, from xm to x0
+    if (xm) lam += adj_damage(a, dtm, m, xm[i], x0[i]);
   }
   lamOut[i] = lam;
   if (lightsOn) dQ[i] += dt * wv(mu1, x, y, z);
@@ -2497,6 +2504,10 @@ int mcm_heat_plan_destroy(mcm_heat_plan* P) {
 }
 
 
+// Most device memory for the states that the adjoint keeps instead of
+// computing them twice.
+static constexpr size_t kAdjointStates = (size_t)4 << 30;
+
 int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segments, int64_t nSegments, const uint8_t* targetMask,
                          int64_t checkpointEvery, mcm_heat_adjoint_output* out) {
   if (!in || !out) return fail(MCM_ERR_INVALID_ARGUMENT, "null argument");
@@ -2516,7 +2527,6 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
     lights.insert(lights.end(), (size_t)segments[k].steps, segments[k].lightsOn != 0);
   }
   const int64_t N = (int64_t)dts.size();
-  const int64_t C = checkpointEvery > 0 ? checkpointEvery : 100;
   mcm_heat_plan* raw = nullptr;
   int rc = mcm_heat_plan_create(in, &raw);
   if (rc) return rc;
@@ -2528,17 +2538,56 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
   // target voxels: the mask, or every voxel whose medium has E != 0
   std::vector<uint8_t> mask((size_t)L);
   for (int64_t i = 0; i < L; ++i) mask[i] = targetMask ? (targetMask[i] != 0) : (in->E[in->M[i]] != 0);
-  const int64_t nChk = std::max<int64_t>(1, (N + C - 1) / C);
-  HeatBuf dMask, chk;
-  if ((rc = halloc(dMask, (size_t)L)) || (rc = halloc(chk, (size_t)nChk * bytes))) return rc;
+  HeatBuf dMask, chk, seg;
+  if ((rc = halloc(dMask, (size_t)L))) return rc;
   MCM_HIP(hipMemcpyAsync(dMask.p, mask.data(), (size_t)L, hipMemcpyHostToDevice, s));
-  auto chkp = [&](int64_t k) { return (double*)chk.p + (size_t)k * L; };
-  // forward pass with checkpoints every C steps
-  for (int64_t n = 0; n < N; ++n) {
-    if (n % C == 0) MCM_HIP(hipMemcpyAsync(chkp(n / C), P->T1.p, bytes, hipMemcpyDeviceToDevice, s));
-    if ((rc = advance<double>(P, 1, dts[(size_t)n], lights[(size_t)n]))) return rc;
+  // The reverse sweep needs the state at every step.  Where all of them fit in
+  // kAdjointStates they are kept (one segment, no checkpoint), else the steps of
+  // one segment at a time are run again from its checkpoint (96 x 80 x 72, 120
+  // steps: 10.7 ms a call kept, 14.8 with three segments of 40 and copies).
+  const bool gradients = out->dJ_dQ || out->dJ_dT0 || out->dJ_dc;
+  bool keep = gradients && (size_t)(N + 1) <= kAdjointStates / bytes;
+  if (keep && hipMalloc(&seg.p, (size_t)(N + 1) * bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    seg.p = nullptr;
+    keep = false;
   }
-  if (N == 0) MCM_HIP(hipMemcpyAsync(chkp(0), P->T1.p, bytes, hipMemcpyDeviceToDevice, s));
+  const int64_t C = keep ? std::max<int64_t>(N, 1) : checkpointEvery > 0 ? checkpointEvery : 100;
+  const int64_t nChk = keep ? 0 : std::max<int64_t>(1, (N + C - 1) / C);
+  if (!keep && (rc = halloc(chk, (size_t)nChk * bytes))) return rc;
+  auto chkp = [&](int64_t k) { return (double*)chk.p + (size_t)k * L; };
+  auto segp = [&](int64_t k) { return (double*)seg.p + (size_t)k * L; };
+  // steps n0 .. n1 - 1 from the state in segp(0) into segp(1), segp(2), ...: each
+  // step reads and writes the segment in place of the plan's state buffers
+  auto run_segment = [&](int64_t n0, int64_t n1) -> int {
+    struct Restore {
+      mcm_heat_plan* P;
+      void *T1, *T2;
+      ~Restore() { P->T1.p = T1, P->T2.p = T2; }
+    } restore{P, P->T1.p, P->T2.p};
+    P->T1.p = segp(0);
+    for (int64_t n = n0; n < n1; ++n) {
+      double* const to = segp(n - n0 + 1);
+      P->T2.p = to;
+      if (int e = advance<double>(P, 1, dts[(size_t)n], lights[(size_t)n])) return e;
+      if (P->T1.p != to) {  // interrupted: the state stays
+        MCM_HIP(hipMemcpyAsync(to, P->T1.p, bytes, hipMemcpyDeviceToDevice, s));
+        P->T1.p = to;
+      }
+    }
+    return MCM_OK;
+  };
+  if (keep) {
+    MCM_HIP(hipMemcpyAsync(segp(0), P->T1.p, bytes, hipMemcpyDeviceToDevice, s));
+    if ((rc = run_segment(0, N))) return rc;
+  } else {
+    // forward pass with checkpoints every C steps
+    for (int64_t n = 0; n < N; ++n) {
+      if (n % C == 0) MCM_HIP(hipMemcpyAsync(chkp(n / C), P->T1.p, bytes, hipMemcpyDeviceToDevice, s));
+      if ((rc = advance<double>(P, 1, dts[(size_t)n], lights[(size_t)n]))) return rc;
+    }
+    if (N == 0) MCM_HIP(hipMemcpyAsync(chkp(0), P->T1.p, bytes, hipMemcpyDeviceToDevice, s));
+  }
   std::vector<double> om((size_t)L);
   MCM_HIP(hipMemcpyAsync(om.data(), P->Om.p, bytes, hipMemcpyDeviceToHost, s));
   MCM_HIP(hipStreamSynchronize(s));
@@ -2547,12 +2596,12 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
     if (mask[i]) J += om[i];
   out->J = J;
   if (out->Omega_f64) std::memcpy(out->Omega_f64, om.data(), bytes);
-  if (!out->dJ_dQ && !out->dJ_dT0 && !out->dJ_dc) return MCM_OK;
+  if (!gradients) return MCM_OK;
   if (P->nz > 65535) return fail(MCM_ERR_UNSUPPORTED, "heat adjoint: nz > 65535 z planes");
   // reverse sweep, one checkpoint segment at a time
-  HeatBuf seg, lam, lamN, mu1, mu2, mu3, dQ, s1, s2, dC;
+  HeatBuf lam, lamN, mu1, mu2, mu3, dQ, s1, s2, dC;
   const int nBins = P->nM * P->nM * 3;
-  if ((rc = halloc(seg, (size_t)(C + 1) * bytes)) || (rc = halloc(lam, bytes)) || (rc = halloc(lamN, bytes)) || (rc = halloc(mu1, bytes)) ||
+  if ((!keep && (rc = halloc(seg, (size_t)(C + 1) * bytes))) || (rc = halloc(lam, bytes)) || (rc = halloc(lamN, bytes)) || (rc = halloc(mu1, bytes)) ||
       (rc = halloc(mu2, bytes)) || (rc = halloc(mu3, bytes)) || (rc = halloc(dQ, bytes)))
     return rc;
   if (out->dJ_dc) {
@@ -2562,7 +2611,6 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
   }
   MCM_HIP(hipMemsetAsync(lam.p, 0, bytes, s));
   MCM_HIP(hipMemsetAsync(dQ.p, 0, bytes, s));
-  auto segp = [&](int64_t k) { return (double*)seg.p + (size_t)k * L; };
   const int tpb = kHeatTPB;
   const unsigned gv = (unsigned)((L + tpb - 1) / tpb);
   const unsigned gx = (unsigned)(((int64_t)P->ny * P->nz + tpb - 1) / tpb);
@@ -2570,28 +2618,30 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
   const unsigned gz = (unsigned)(((int64_t)P->nx * P->ny + tpb - 1) / tpb);
   for (int64_t k = (N + C - 1) / C - 1; k >= 0; --k) {
     const int64_t s0 = k * C, e0 = std::min(N, s0 + C);
-    MCM_HIP(hipMemcpyAsync(P->T1.p, chkp(k), bytes, hipMemcpyDeviceToDevice, s));
-    MCM_HIP(hipMemcpyAsync(segp(0), chkp(k), bytes, hipMemcpyDeviceToDevice, s));
-    for (int64_t n = s0; n < e0; ++n) {
-      if ((rc = advance<double>(P, 1, dts[(size_t)n], lights[(size_t)n]))) return rc;
-      MCM_HIP(hipMemcpyAsync(segp(n - s0 + 1), P->T1.p, bytes, hipMemcpyDeviceToDevice, s));
+    if (!keep) {
+      MCM_HIP(hipMemcpyAsync(segp(0), chkp(k), bytes, hipMemcpyDeviceToDevice, s));
+      if ((rc = run_segment(s0, e0))) return rc;
     }
     for (int64_t n = e0 - 1; n >= s0; --n) {
       HeatArgs<double> a = make_args<double>(P, dts[(size_t)n], lights[(size_t)n]);
       const double* x0 = segp(n - s0);
       const double* x1 = segp(n - s0 + 1);
       double* B = (double*)P->B.p;
-      hipLaunchKernelGGL(heat_adj_damage, dim3(gv), dim3(tpb), 0, s, a, x0, x1, (const uint8_t*)dMask.p, (double*)lam.p, L);
+      // (the others' damage is added by the combine of the step after them)
+      if (n == e0 - 1)
+        hipLaunchKernelGGL(heat_adj_damage, dim3(gv), dim3(tpb), 0, s, a, x0, x1, (const uint8_t*)dMask.p, (double*)lam.p, L);
+      const double* xm = n > s0 ? segp(n - s0 - 1) : nullptr;
+      const double dtm = n > s0 ? dts[(size_t)n - 1] : 0.0;
       adj_solve<2>(P, a, (const double*)lam.p, (double*)mu3.p, B, gz);
       adj_solve<1>(P, a, (const double*)mu3.p, (double*)mu2.p, B, gy);
       adj_solve<0>(P, a, (const double*)mu2.p, (double*)mu1.p, B, gx);
-      const dim3 gc((unsigned)((P->nx * P->ny + tpb - 1) / tpb), (unsigned)P->nz);
+      const dim3 gc((unsigned)((P->nx * P->ny + tpb - 1) / tpb) * (unsigned)P->nz);
       if (P->nM * P->nM * 3 <= kLdsCoef)
         hipLaunchKernelGGL(heat_adj_combine<true>, gc, dim3(tpb), 0, s, a, (const double*)mu1.p, (const double*)mu2.p,
-                           (const double*)mu3.p, x0, x1, (const uint8_t*)dMask.p, (double*)lamN.p, (double*)dQ.p, lights[(size_t)n]);
+                           (const double*)mu3.p, x0, x1, (const uint8_t*)dMask.p, (double*)lamN.p, (double*)dQ.p, lights[(size_t)n], xm, dtm);
       else
         hipLaunchKernelGGL(heat_adj_combine<false>, gc, dim3(tpb), 0, s, a, (const double*)mu1.p, (const double*)mu2.p,
-                           (const double*)mu3.p, x0, x1, (const uint8_t*)dMask.p, (double*)lamN.p, (double*)dQ.p, lights[(size_t)n]);
+                           (const double*)mu3.p, x0, x1, (const uint8_t*)dMask.p, (double*)lamN.p, (double*)dQ.p, lights[(size_t)n], xm, dtm);
       MCM_HIP(hipGetLastError());
       if (out->dJ_dc) {
         const dim3 gp((unsigned)((P->nx * P->ny + tpb - 1) / tpb), (unsigned)P->nz);
