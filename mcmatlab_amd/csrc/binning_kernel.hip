@@ -7,12 +7,14 @@
 // pick the set farthest from all picks so far, and every set is labelled
 // with its nearest pick.  Each pass over the N1 sets is one kernel: a thread
 // updates the running nearest distances and labels of its sets and keeps
-// running maxima, and the workgroups publish theirs; a one-workgroup kernel
-// reduces them and selects the next pick on the device, so the N2 passes
-// run back to back on one stream with no host round trip.  (Selecting in
-// the last workgroup to finish, by an atomic ticket, serialised thousands
-// of same-address atomics per pass: 206 us per pass at 8e6 sets, against
-// 27 us for the pass and the separate selection.)
+// running maxima, and the workgroups publish theirs; every workgroup of the
+// next pass reduces them and selects the pick for itself, so the N2 passes run
+// back to back on one stream with no host round trip.  (Selecting in the last
+// workgroup to finish, by an atomic ticket, serialised thousands of same-address
+// atomics per pass: 206 us per pass at 8e6 sets; in a kernel of one workgroup
+// between two passes it took 23.1 us for the pass and 7.9 for the selection,
+// against 24.4 now.)  A pass is bound by reading the sets, 12 bytes each for two
+// varying rows: 96 MB at 8e6 sets.
 //
 // Selection.  The reference's single-threaded pass scans k = 0..N1-1 and
 // keeps a running maximum whose index m starts at the previous pass's m
@@ -45,16 +47,26 @@ namespace mcm {
 namespace {
 
 constexpr int kBinTPB = 256;
-constexpr int kBinMaxBlocks = 8192;
+// Workgroups of a pass at most: each reads every other's maxima, 16 bytes of
+// each (8e6 sets: a pass takes 36.0, 24.6 and 24.4 us with 8192, 2048 and 1024).
+constexpr int kBinMaxBlocks = 1024;
+
+// The state between passes: scan index and value of the last selection, and the
+// distance of set 0 after the last pass.
+struct BinState {
+  int m;
+  float u, d0;
+  int unused;
+};
 
 struct BinArgs {
   const float* pv;       // [3 * n1] input, interleaved (mua, mus, g)
   float* norm;           // [rows][n1] normalised varying rows
   float* d;              // [n1] squared distance to the nearest pick
   uint8_t* bin;          // [n1] 1-based label of the nearest pick
-  float4* part;          // [blocks] (lo value, lo index, hi value, hi index)
+  float4* part;          // [2][kBinMaxBlocks] (lo value, lo index, hi value, hi index)
   int* picks;            // [n2] picked set of each bin
-  int* st;               // [4]: pick, m0, unused, S (float bits)
+  BinState* st;          // [2]
   int64_t n1;
   int rows;
   int rowOf[3];          // input row -> normalised row (-1: constant)
@@ -98,27 +110,32 @@ __device__ inline void block_best(ArgMax& lo, ArgMax& hi) {
     for (int k = 1; k < TPB / 64; ++k) lo = better(lo, sLo[k]), hi = better(hi, sHi[k]);
 }
 
-constexpr int kSelTPB = 1024;
-
-// Each workgroup publishes its two maxima; bin_select (one workgroup)
-// reduces them and picks the next set.
-__device__ inline void publish(const BinArgs& a, ArgMax lo, ArgMax hi) {
+// Each workgroup publishes its two maxima; the next pass selects from them.
+__device__ inline void publish(float4* part, ArgMax lo, ArgMax hi) {
   block_best(lo, hi);
-  if (threadIdx.x == 0) a.part[blockIdx.x] = make_float4(lo.v, __int_as_float(lo.i), hi.v, __int_as_float(hi.i));
+  if (threadIdx.x == 0) part[blockIdx.x] = make_float4(lo.v, __int_as_float(lo.i), hi.v, __int_as_float(hi.i));
 }
 
-// MODE 0: the first pick, farthest from the mean; 1: the second, farthest
-// from the first; 2: later picks by the reference's scan rule.
-template <int MODE>
-__global__ void __launch_bounds__(kSelTPB) bin_select(BinArgs a, int nParts) {
+// What pass j starts from: the set picked and the scan index, from the maxima
+// that the pass before published (by every workgroup for itself: a kernel of one
+// workgroup between two passes took 7.9 us, 2 in each pass).  Pass 0 picks the
+// set farthest from the mean, pass 1 the farthest from it, later ones follow the
+// reference's scan rule.  Maxima and states alternate between two copies, since
+// workgroups of this pass publish theirs while others still read.
+struct Selection {
+  int pick, m;
+};
+__device__ inline Selection select_set(const BinArgs& a, int j, int nParts) {
+  __shared__ Selection sSel;
+  const float4* part = a.part + (size_t)((j + 1) & 1) * kBinMaxBlocks;
   ArgMax L{-1.f, -1}, H{-1.f, -1};
   // up to 8 partials per thread, all loaded before they are compared
-  for (int b0 = threadIdx.x; b0 < nParts; b0 += 8 * kSelTPB) {
+  for (int b0 = threadIdx.x; b0 < nParts; b0 += 8 * kBinTPB) {
     float4 q[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const int b = b0 + k * kSelTPB;
-      q[k] = b < nParts ? a.part[b] : make_float4(-1.f, __int_as_float(-1), -1.f, __int_as_float(-1));
+      const int b = b0 + k * kBinTPB;
+      q[k] = b < nParts ? part[b] : make_float4(-1.f, __int_as_float(-1), -1.f, __int_as_float(-1));
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -126,23 +143,30 @@ __global__ void __launch_bounds__(kSelTPB) bin_select(BinArgs a, int nParts) {
       H = better(H, ArgMax{q[k].z, __float_as_int(q[k].w)});
     }
   }
-  block_best<kSelTPB>(L, H);
-  if (threadIdx.x != 0) return;
-  if (MODE == 2) {
-    const float S = __int_as_float(a.st[3]);
-    int m = L.i >= 0 && L.v > S ? better(H, L).i : H.i;
-    m = m < 0 ? 0 : m;
-    const float um = m == L.i ? L.v : H.v;
-    a.st[0] = um > a.d[0] ? m : 0;
-    a.st[1] = m;
-    a.st[3] = __float_as_int(um);
-  } else {
-    const int c = H.i < 0 ? 0 : H.i;
-    a.st[0] = c;
-    if (MODE == 0) a.picks[0] = c;
-    a.st[1] = 0;  // the reference's running index starts at 0 (calloc)
-    a.st[3] = 0;
+  block_best(L, H);
+  if (threadIdx.x == 0) {
+    Selection r;
+    float u = 0.f;
+    if (j >= 2) {
+      const BinState S = a.st[(j + 1) & 1];
+      int m = L.i >= 0 && L.v > S.u ? better(H, L).i : H.i;
+      m = m < 0 ? 0 : m;
+      u = m == L.i ? L.v : H.v;
+      r.pick = u > S.d0 ? m : 0;
+      r.m = m;
+    } else {
+      r.pick = H.i < 0 ? 0 : H.i;
+      r.m = 0;  // the reference's running index starts at 0 (calloc)
+    }
+    sSel = r;
+    if (blockIdx.x == 0) {
+      a.picks[j] = r.pick;
+      a.st[j & 1].m = r.m;
+      a.st[j & 1].u = u;
+    }
   }
+  __syncthreads();
+  return sSel;
 }
 
 // pass 0: normalise the varying rows, distances to the mean, first pick
@@ -162,29 +186,32 @@ __global__ void __launch_bounds__(kBinTPB) bin_prepare(BinArgs a) {
     }
     if (s > best.v) best = ArgMax{s, (int)i};
   }
-  publish(a, ArgMax{-1.f, -1}, best);
+  publish(a.part + kBinMaxBlocks, ArgMax{-1.f, -1}, best);
 }
 
 // Passes over the sets for ROWS varying rows: a thread takes kBinPer sets
 // kBinTPB apart and issues all their loads before the arithmetic.
 constexpr int kBinPer = 8;
 
+// The squares are summed in double and rounded to single after each row: the
+// first one alone is a single-precision product, and a later one's product is
+// exact in double, so that one fused operation gives the sum.
 template <int ROWS>
 __device__ inline float sqr_dist_r(const float (&x)[ROWS > 0 ? ROWS : 1], const float (&p)[3]) {
   float s = 0.f;
 #pragma unroll
   for (int q = 0; q < ROWS; ++q) {
     const float t = x[q] - p[q];
-    s = (float)((double)s + (double)t * (double)t);
+    s = q == 0 ? t * t : (float)__builtin_fma((double)t, (double)t, (double)s);
   }
   return s;
 }
 
 // pass 1: distances to the first pick, every label 1, second pick
 template <int ROWS>
-__global__ void __launch_bounds__(kBinTPB) bin_first(BinArgs a) {
+__global__ void __launch_bounds__(kBinTPB) bin_first(BinArgs a, int nParts) {
   float p[3] = {0.f, 0.f, 0.f};
-  const int c = a.picks[0];
+  const int c = select_set(a, 0, nParts).pick;
 #pragma unroll
   for (int q = 0; q < ROWS; ++q) p[q] = a.norm[(int64_t)q * a.n1 + c];
   ArgMax best{-1.f, -1};
@@ -202,19 +229,20 @@ __global__ void __launch_bounds__(kBinTPB) bin_first(BinArgs a) {
       const int64_t i = i0 + k * kBinTPB;
       if (i >= a.n1) break;
       const float s = sqr_dist_r<ROWS>(x[k], p);
+      if (i == 0) a.st[0].d0 = s;
       a.d[i] = s;
       a.bin[i] = 1;
       if (s > best.v) best = ArgMax{s, (int)i};
     }
   }
-  publish(a, ArgMax{-1.f, -1}, best);
+  publish(a.part, ArgMax{-1.f, -1}, best);
 }
 
 // pass j >= 1 of the reference loop: pick j is the current selection
 template <int ROWS>
-__global__ void __launch_bounds__(kBinTPB) bin_step(BinArgs a, int j) {
-  const int c = a.st[0], m0 = a.st[1];
-  if (blockIdx.x == 0 && threadIdx.x == 0) a.picks[j] = c;
+__global__ void __launch_bounds__(kBinTPB) bin_step(BinArgs a, int j, int nParts) {
+  const Selection sel = select_set(a, j, nParts);
+  const int c = sel.pick, m0 = sel.m;
   float p[3] = {0.f, 0.f, 0.f};
 #pragma unroll
   for (int q = 0; q < ROWS; ++q) p[q] = a.norm[(int64_t)q * a.n1 + c];
@@ -242,6 +270,7 @@ __global__ void __launch_bounds__(kBinTPB) bin_step(BinArgs a, int j) {
         a.d[i] = s;
         a.bin[i] = label;
       }
+      if (i == 0) a.st[j & 1].d0 = v;
       if (i < m0) {
         if (v > lo.v) lo = ArgMax{v, (int)i};
       } else if (v > hi.v) {
@@ -249,7 +278,7 @@ __global__ void __launch_bounds__(kBinTPB) bin_step(BinArgs a, int j) {
       }
     }
   }
-  publish(a, lo, hi);
+  publish(a.part + (size_t)(j & 1) * kBinMaxBlocks, lo, hi);
 }
 
 // rescale the picks (:182-186)
@@ -272,16 +301,13 @@ struct DevMem {
   }
 };
 
-__global__ void bin_clear_state(int* st) {
-  if (threadIdx.x < 4) st[threadIdx.x] = 0;
-}
-
 // Device buffers of one call (see BinArgs) and the call's stream.
 struct BinBuffers {
   float *pv, *norm, *d, *out;
   uint8_t* bin;
   float4* part;
-  int *picks, *st;
+  int* picks;
+  BinState* st;
 };
 
 int blocks_for(int64_t n1) { return (int)std::min<int64_t>(kBinMaxBlocks, (n1 + kBinTPB * kBinPer - 1) / (kBinTPB * kBinPer)); }
@@ -330,17 +356,11 @@ int run_passes(const float* paramVals, int64_t n1, int64_t n2, float* downsample
   a.part = B.part;
   a.picks = B.picks;
   a.st = B.st;
-  hipLaunchKernelGGL(bin_clear_state, dim3(1), dim3(64), 0, s, B.st);
   hipLaunchKernelGGL(bin_prepare, dim3(blocksPrep), dim3(kBinTPB), 0, s, a);
-  hipLaunchKernelGGL(bin_select<0>, dim3(1), dim3(kSelTPB), 0, s, a, blocksPrep);
   auto passes = [&](auto rowsTag) {
     constexpr int R = decltype(rowsTag)::value;
-    hipLaunchKernelGGL(bin_first<R>, dim3(blocks), dim3(kBinTPB), 0, s, a);
-    hipLaunchKernelGGL(bin_select<1>, dim3(1), dim3(kSelTPB), 0, s, a, blocks);
-    for (int64_t j = 1; j < n2; ++j) {
-      hipLaunchKernelGGL(bin_step<R>, dim3(blocks), dim3(kBinTPB), 0, s, a, (int)j);
-      hipLaunchKernelGGL(bin_select<2>, dim3(1), dim3(kSelTPB), 0, s, a, blocks);
-    }
+    hipLaunchKernelGGL(bin_first<R>, dim3(blocks), dim3(kBinTPB), 0, s, a, blocksPrep);
+    for (int64_t j = 1; j < n2; ++j) hipLaunchKernelGGL(bin_step<R>, dim3(blocks), dim3(kBinTPB), 0, s, a, (int)j, blocks);
   };
   switch (a.rows) {
     case 0: passes(std::integral_constant<int, 0>()); break;
@@ -364,7 +384,7 @@ constexpr int64_t kScratchSets = 1 << 20;
 constexpr int64_t kScratchBins = 4096;
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t kScratchBytes = align256(kScratchSets * 12) * 2 + align256(kScratchSets * 4) + align256(kScratchSets) +
-                                 align256(kBinMaxBlocks * 16) + align256(kScratchBins * 4) + align256(16) + align256(kScratchBins * 12);
+                                 align256(2 * kBinMaxBlocks * 16) + align256(kScratchBins * 4) + align256(2 * sizeof(BinState)) + align256(kScratchBins * 12);
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 BinBuffers scratch_layout(unsigned char* base, int64_t n1, int64_t n2) {
@@ -379,9 +399,9 @@ BinBuffers scratch_layout(unsigned char* base, int64_t n1, int64_t n2) {
   B.norm = (float*)take((size_t)n1 * 12);
   B.d = (float*)take((size_t)n1 * 4);
   B.bin = take((size_t)n1);
-  B.part = (float4*)take((size_t)kBinMaxBlocks * 16);
+  B.part = (float4*)take((size_t)2 * kBinMaxBlocks * 16);
   B.picks = (int*)take((size_t)n2 * 4);
-  B.st = (int*)take(16);
+  B.st = (BinState*)take(2 * sizeof(BinState));
   B.out = (float*)take((size_t)n2 * 12);
   return B;
 }
@@ -413,15 +433,14 @@ extern "C" int mcm_downsample_params(const float* paramVals, int64_t n1, int64_t
     }
   } rowThreads;
   for (int r = 0; r < 3; ++r) rowThreads.t[r] = std::thread(row_pass, paramVals, n1, r, mx, mn, sum, finite);
-  const int blocks = blocks_for(n1), blocksPrep = prep_blocks_for(n1);
   DevMem pv, norm, d, bin, part, picks, st, out;
   MCM_HIP(hipMalloc(&pv.p, (size_t)n1 * 3 * sizeof(float)));
   MCM_HIP(hipMalloc(&norm.p, (size_t)n1 * 3 * sizeof(float)));
   MCM_HIP(hipMalloc(&d.p, (size_t)n1 * sizeof(float)));
   MCM_HIP(hipMalloc(&bin.p, (size_t)n1));
-  MCM_HIP(hipMalloc(&part.p, (size_t)std::max(blocks, blocksPrep) * sizeof(float4)));
+  MCM_HIP(hipMalloc(&part.p, (size_t)2 * kBinMaxBlocks * sizeof(float4)));
   MCM_HIP(hipMalloc(&picks.p, (size_t)n2 * sizeof(int)));
-  MCM_HIP(hipMalloc(&st.p, 4 * sizeof(int)));
+  MCM_HIP(hipMalloc(&st.p, 2 * sizeof(BinState)));
   MCM_HIP(hipMalloc(&out.p, (size_t)n2 * 3 * sizeof(float)));
   hipStream_t s = nullptr;
   MCM_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
@@ -435,7 +454,7 @@ extern "C" int mcm_downsample_params(const float* paramVals, int64_t n1, int64_t
     (void)hipStreamSynchronize(s);
     return fail(MCM_ERR_INVALID_ARGUMENT, "getDownsampledParamVals: paramVals must be finite");
   }
-  const BinBuffers B{(float*)pv.p, (float*)norm.p, (float*)d.p, (float*)out.p, (uint8_t*)bin.p, (float4*)part.p, (int*)picks.p, (int*)st.p};
+  const BinBuffers B{(float*)pv.p, (float*)norm.p, (float*)d.p, (float*)out.p, (uint8_t*)bin.p, (float4*)part.p, (int*)picks.p, (BinState*)st.p};
   return run_passes(paramVals, n1, n2, downsampled, binidx, B, mx, mn, sum, s);
 }
 
