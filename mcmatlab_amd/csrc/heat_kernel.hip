@@ -1530,7 +1530,7 @@ __global__ void __launch_bounds__(kHeatTPB) heat_adj_combine(HeatArgs<double> a,
   const double* __restrict__ cT = LDS_COEF ? sC : a.c;
   const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = nx * ny;
   // whole workgroups per z plane, so that index arithmetic is 32-bit; each XCD
-  // takes neighbouring planes and rows.  14.2 us at 96 x 80 x 72 with the damage
+  // takes neighbouring planes and rows.  12.3 us at 96 x 80 x 72 with the damage
   // of the step before; 15.5 and 4.1 as two kernels in launch order.
   const int perPlane = (nxy + kHeatTPB - 1) / kHeatTPB, blk = xcd_contiguous(blockIdx.x, gridDim.x);
   const int z = blk / perPlane, p = (blk - z * perPlane) * kHeatTPB + threadIdx.x;
@@ -1539,20 +1539,35 @@ __global__ void __launch_bounds__(kHeatTPB) heat_adj_combine(HeatArgs<double> a,
   const int64_t i = (int64_t)z * nxy + p;
   const int m = a.M[i];
   const double dt = a.dt;
-  // L_d^T (D w) at i for w = mu1, mu2, mu3
-  auto wv = [&](const double* mu, int xx, int yy, int zz) { return heat_frozen(a, xx, yy, zz) ? 0.0 : mu[xx + yy * nx + (int64_t)zz * nxy]; };
+  // L_d^T (D w) at i for w = mu1, mu2, mu3.  Every neighbour is read, one outside
+  // the grid as the voxel itself, and dropped by a select: all loads are under
+  // way at once (14.2 us with a branch per neighbour, 12.3 so).
+  const bool sk = a.sinked;
+  const bool ix = sk && (x == 0 || x == nx - 1), iy = sk && (y == 0 || y == ny - 1), iz = sk && (z == 0 || z == nz - 1);
+  const bool own = !(ix || iy || iz);
+  const double w1 = own ? mu1[i] : 0.0, w2 = own ? mu2[i] : 0.0, w3 = own ? mu3[i] : 0.0;
   double t1[3] = {0, 0, 0}, t2 = 0, t3 = 0;
-  const int xyz[3] = {x, y, z}, ext[3] = {nx, ny, nz};
+  const int xyz[3] = {x, y, z}, ext[3] = {nx, ny, nz}, step[3] = {1, nx, nxy};
+  const bool fz[3] = {iy || iz, ix || iz, ix || iy};  // frozen by the other axes
+#pragma unroll
   for (int d = 0; d < 3; ++d) {
+#pragma unroll
     for (int s = -1; s <= 1; s += 2) {
       const int q = xyz[d] + s;
-      if (q < 0 || q >= ext[d]) continue;
-      const int xx = d == 0 ? q : x, yy = d == 1 ? q : y, zz = d == 2 ? q : z;
-      const int mn = a.M[xx + yy * nx + (int64_t)zz * nxy];
+      const bool in = q >= 0 && q < ext[d], off = fz[d] || (sk && (q == 0 || q == ext[d] - 1));
+      const int64_t j = in ? i + s * step[d] : i;
+      const int mn = a.M[j];
       const double cin = coef(cT, a.nM, mn, m, d), cout = coef(cT, a.nM, m, mn, d);
-      t1[d] += cin * wv(mu1, xx, yy, zz) - cout * wv(mu1, x, y, z);
-      if (d == 1) t2 += cin * wv(mu2, xx, yy, zz) - cout * wv(mu2, x, y, z);
-      if (d == 2) t3 += cin * wv(mu3, xx, yy, zz) - cout * wv(mu3, x, y, z);
+      const double v1 = mu1[j], e1 = cin * (off ? 0.0 : v1) - cout * w1;
+      t1[d] += in ? e1 : 0.0;
+      if (d == 1) {
+        const double v2 = mu2[j], e2 = cin * (off ? 0.0 : v2) - cout * w2;
+        t2 += in ? e2 : 0.0;
+      }
+      if (d == 2) {
+        const double v3 = mu3[j], e3 = cin * (off ? 0.0 : v3) - cout * w3;
+        t3 += in ? e3 : 0.0;
+      }
     }
   }
   double lam = mu1[i] + dt * (t1[0] / 2 + t1[1] + t1[2]) - dt / 2 * t2 - dt / 2 * t3;
@@ -1562,7 +1577,7 @@ __global__ void __launch_bounds__(kHeatTPB) heat_adj_combine(HeatArgs<double> a,
     if (xm) lam += adj_damage(a, dtm, m, xm[i], x0[i]);
   }
   lamOut[i] = lam;
-  if (lightsOn) dQ[i] += dt * wv(mu1, x, y, z);
+  if (lightsOn) dQ[i] += dt * w1;
 }
 
 // Gradient with respect to the conduction coefficients c[a, b, d] (the
