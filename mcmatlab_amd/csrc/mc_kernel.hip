@@ -858,10 +858,12 @@ int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed,
 }
 
 // Fluence copies of a launch of several items, `voxels` in all and LB in one:
-// those of a plan, within 1 GiB.  The items of a batch run one after another, so
-// one item's copies are in use at a time (8 items of 150^3, 3.3 10^6 packets of a
-// pencil beam: kernel 52.3 ms with one copy, 25.1 ms with eight).
-constexpr int64_t kItemCopiesBytes = (int64_t)2 << 30;
+// those of a plan, within 16 GiB (one copy if there is no memory for more).  The
+// items of a batch run one after another, so one item's copies are in use at a
+// time (8 items of 150^3, 3.3 10^6 packets of a pencil beam: kernel 52.3 ms with
+// one copy, 25.1 ms with eight; 64 items, 1.45 10^8 packets: 2.35 s with one,
+// 1.22 s with eight).
+constexpr int64_t kItemCopiesBytes = (int64_t)16 << 30;
 int item_copies(int64_t LB, int64_t voxels) {
   int n = start_copies(LB);
   while (n > 1 && n * voxels * (int64_t)sizeof(double) > kItemCopiesBytes) n /= 2;
