@@ -24,8 +24,8 @@
 //
 // Lanes are persistent and each packet is a small state machine like the
 // transport's: FETCH (take the next packet number, one atomic per wavefront,
-// or the lane's own packet again for pass 2), MOVE (one voxel sub-step),
-// SCATTER (roulette + deflection), FRESNEL (an interface).  Each iteration the wavefront runs one state for the lanes in
+// or the lane's own packet again for pass 2), MOVE (one voxel sub-step, with
+// an interface crossed), SCATTER (roulette + deflection).  Each iteration the wavefront runs one state for the lanes in
 // it (MOVE while 30 % of the live lanes want to move, otherwise the
 // state with more waiting lanes), so a wavefront never waits for its
 // longest-lived packet before starting others.
@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
   const int t = threadIdx.x;
   for (int q = 0; q < 4; ++q) sSum[q][t] = 0.0;
   __syncthreads();
-  constexpr int G_FETCH = 0, G_MOVE = 1, G_SCATTER = 2, G_FRESNEL = 3, G_DONE = 4;
+  constexpr int G_FETCH = 0, G_MOVE = 1, G_SCATTER = 2, G_DONE = 3;
   const int lane = __lane_id();
   PacketRng R;
   R.key0 = g.key0;
@@ -137,7 +137,6 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
   double D = 0.0, tau = 0.0;  // pass 1: box deposit, optical depth; pass 2: box deposits still to come
   uint32_t K = 0;
   int nTerms = 0, parked = 0;  // terms parked by the lane, by any lane at most
-  int pendJ = 0, pendM = 0;
   bool boxed = false;  // the packet's voxel is in the box (and the packet in the volume)
   double* const grad = g.grad + (size_t)(xcd() % g.copies) * g.LB;
   // spread few packets over the wavefronts (launch_blocks)
@@ -189,21 +188,18 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
     const unsigned long long bFetch = __ballot(st == G_FETCH);
     const unsigned long long bMove = __ballot(st == G_MOVE);
     const unsigned long long bScat = __ballot(st == G_SCATTER);
-    const unsigned long long bFres = FRESNEL ? __ballot(st == G_FRESNEL) : 0ull;
-    const int cF = __popcll(bFetch), cM = __popcll(bMove), cS = __popcll(bScat), cR = __popcll(bFres);
-    const int active = cF + cM + cS + cR;
+    const int cF = __popcll(bFetch), cM = __popcll(bMove), cS = __popcll(bScat);
+    const int active = cF + cM + cS;
     if (active == 0) break;
     int phase = G_MOVE;
     const int stay = max(1, (int)ceilf(kStay * (float)active));
     if (cM < stay) {
       int best = cM;
       if (cS > best) { best = cS; phase = G_SCATTER; }
-      if (FRESNEL && cR > best) { best = cR; phase = G_FRESNEL; }
       if (cF > best) phase = G_FETCH;
     }
     if (phase == G_MOVE) do {
       if (st == G_MOVE) {
-        bool moved = true;
         if (P.substeps >= kMaxSubsteps) {
           P.alive = false;
         } else {
@@ -229,17 +225,13 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
             ++nTerms;
           }
           if (!P.sameVoxel) {
-            if (FRESNEL && P.ri != sMed[mNew].ri) {
-              pendJ = jNew;
-              pendM = mNew;
-              st = G_FRESNEL;
-              moved = false;
-            } else {
-              enter(jNew, mNew, muaNew);
-            }
+            // (at once: a packet trapped between two indices meets an interface at
+            // every sub-step, and a state of its own would double its time)
+            if (FRESNEL && P.ri != sMed[mNew].ri) fresnel(P, p, sMed, jNew, mNew, R);
+            enter(jNew, mNew, muaNew);
           }
         }
-        if (moved) settle();
+        settle();
       }
       // a lane parks at most one term per sub-step
       if (++parked >= kTerms && __ballot(nTerms == kTerms)) {
@@ -251,12 +243,6 @@ __global__ void __launch_bounds__(256, 4) mc_grad(McParams p, GradArgs g, const 
       if (st == G_SCATTER) {
         ++K;  // the flight ended in an interaction
         roulette_scatter(P, p, p.cdfs, 0, R);
-        settle();
-      }
-    } else if (FRESNEL && phase == G_FRESNEL) {
-      if (st == G_FRESNEL) {
-        fresnel(P, p, sMed, pendJ, pendM, R);
-        enter(pendJ, pendM, g.muaMap ? g.muaMap[pendJ] : 0.f);
         settle();
       }
     } else {
