@@ -7,8 +7,8 @@
 //   SCATTER  -> roulette + scattering (MCmatlab.c:259-260)
 //   FRESNEL  -> reflection/refraction at a refractive-index change
 // Tally writes go through Sink:
-//   deposit(j, w)   absorbed weight into voxel j (the sink may merge
-//                   consecutive deposits into one voxel), flush() at death
+//   deposit(j, w)   absorbed weight into voxel j (the sink may hold deposits
+//                   back), flush() at death
 //   image_add(bin, w), farField(bin, w), edge(face, idx, w), collected()
 //   or, when Sink::kDeferEscapes, escape(P, escaped, edgeFlux, slot): the packet
 //   is recorded and those tallies are formed later (only without deposition
@@ -196,7 +196,7 @@ struct PacketEngine {
   }
 };
 
-// The tallies of a recorded escape (the inline code of finish_substep with
+// The tallies of a recorded escape (the inline code of enter_voxel with
 // the deposition criteria inactive): light collector image, far field and
 // edge fluxes.
 template <class Sink>

@@ -183,8 +183,7 @@ __device__ inline void fadd(double* p, double v) { unsafeAtomicAdd(p, v); }
 // escape record buffers: 64 + 48 bytes per packet).
 constexpr uint64_t kMaxLaunchPackets = 1ull << 24;
 
-// Tally sink of the GPU kernel: FP64 hardware atomics; consecutive deposits
-// into the same voxel are merged in a register first.  Holds copies of the
+// Tally sink of the GPU kernels: FP64 hardware atomics.  Holds copies of the
 // tally pointers (not a pointer to the launch parameters, whose address must
 // not escape or the parameters are copied to scratch).
 struct DeviceSink {
@@ -193,27 +192,11 @@ struct DeviceSink {
   double* image;
   double* FF;
   double *ni0, *ni1, *ni2, *ni3, *ni4, *ni5;
-  double acc;
-  int accJ;
   unsigned long long nCollected;
   unsigned nRunaway;
   __device__ explicit DeviceSink(const McParams& p)
       : NFR(p.NFR + (size_t)(xcd() % p.nfrReplicas) * p.LB), image(p.image), FF(p.FF), ni0(p.NI[0]), ni1(p.NI[1]), ni2(p.NI[2]), ni3(p.NI[3]), ni4(p.NI[4]),
-        ni5(p.NI[5]), acc(0.0), accJ(-1), nCollected(0), nRunaway(0) {}
-  __device__ void deposit(int j, double v) {
-    if (j == accJ) {
-      acc += v;
-    } else {
-      if (accJ >= 0) fadd(&NFR[accJ], acc);
-      accJ = j;
-      acc = v;
-    }
-  }
-  __device__ void flush() {
-    if (accJ >= 0) fadd(&NFR[accJ], acc);
-    accJ = -1;
-    acc = 0.0;
-  }
+        ni5(p.NI[5]), nCollected(0), nRunaway(0) {}
   __device__ void image_add(int b, double w) { fadd(&image[b], w); }
   __device__ void farField(int b, double w) { fadd(&FF[b], w); }
   __device__ void edge(int f, int i, double w) {
@@ -231,9 +214,10 @@ struct RingSlots {
   uint2 d[256 * kRingPitch];  // voxel, absorbed weight (float bits)
 };
 
-// Sink of the transport kernel without deposition criteria: a packet dies
-// once, so its escape is written to the record slot of its own launch index
-// (no shared counter) and tallied by mc_tally_escapes after the launch.
+// Sink of the transport kernels.  ESCAPES (without deposition criteria): a
+// packet dies once, so its escape is written to the record slot of its own
+// launch index (no shared counter) and tallied by mc_tally_escapes after the
+// launch.
 //
 // The fluence is bound by the number of 64-byte lines that atomic
 // instructions touch: the memory side takes 2.37e10 of them per second
