@@ -94,12 +94,13 @@ def build_test_harnesses(verbose=True):
     project's MEX layer against the mx-API shim (test infrastructure)."""
     out = os.path.join(ROOT, "tests", "_build")
     os.makedirs(out, exist_ok=True)
-    h = os.path.join(ROOT, "tests", "cpu_harness", "mc_host_harness.hip")
-    if os.path.exists(h):
-        _run([HIPCC, "-O2", "-fPIC", "-shared", "-std=c++17", f"--offload-arch={ARCH}", *DEVICE_FLAGS, "-I", INCLUDE, "-I", CSRC,
-              "-x", "hip", h, "-o", os.path.join(out, "libmc_host.so")])
-        if verbose:
-            print("  built tests/_build/libmc_host.so")
+    for src, lib in (("mc_host_harness.hip", "libmc_host.so"), ("rng_harness.hip", "librng_host.so")):
+        h = os.path.join(ROOT, "tests", "cpu_harness", src)
+        if os.path.exists(h):
+            _run([HIPCC, "-O2", "-fPIC", "-shared", "-std=c++17", f"--offload-arch={ARCH}", *DEVICE_FLAGS, "-I", INCLUDE, "-I", CSRC,
+                  "-x", "hip", h, "-o", os.path.join(out, lib)])
+            if verbose:
+                print(f"  built tests/_build/{lib}")
     mexdir = os.path.join(PKG, "mex")
     shim = os.path.join(ROOT, "tests", "mexshim")
     for name in ("MCmatlab_mex.c", "finiteElementHeatPropagator_mex.c", "getDownsampledParamVals_mex.c"):
