@@ -100,9 +100,9 @@ inline std::string build_mc_tables(const mcm_mc_input* in, McTables& T, bool hos
   T.M0.resize((size_t)T.L);
   bool outside = false;
   for (int64_t k = 0; k < T.L; ++k) {
-    const uint8_t m = (uint8_t)(in->M[k] - 1);
-    outside |= m >= T.nM;
-    T.M0[k] = m;
+    const uint8_t m = in->M[k];
+    outside |= (m == 0) | (m > T.nM);  // (of m, not m - 1: 0 - 1 is medium 255 of 256)
+    T.M0[k] = (uint8_t)(m - 1);
   }
   if (outside) return "M holds a medium index outside 1..nM";
   T.timed = std::isnan(in->nPhotonsRequested);
