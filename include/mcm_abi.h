@@ -189,8 +189,9 @@ int mcm_mc_plan_create(const mcm_mc_input *in, mcm_mc_plan **plan);
 int mcm_mc_plan_simulate(mcm_mc_plan *plan, int64_t iL, uint64_t nPhotons, uint64_t seed,
                          uint64_t firstPhoton, void *stream);
 int mcm_mc_plan_normalize(mcm_mc_plan *plan, int64_t iL, mcm_mc_output *out);
-/* Raw FP64 tallies on the device (absorbed weight per voxel, before
- * normalisation), valid until the next plan call. */
+/* Raw FP64 tallies on the device (absorbed weight per voxel, x fastest, before
+ * normalisation) of every run so far, whatever its stream (waits for the
+ * device); valid until the next plan call. */
 int mcm_mc_plan_tallies(mcm_mc_plan *plan, const double **d_deposit, uint64_t *nPhotons);
 /* Event counters accumulated since the last plan_normalize (synchronises):
  * [0] packets launched alive, [1] collected, [2] voxel sub-steps,

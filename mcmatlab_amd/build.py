@@ -101,6 +101,13 @@ def build_test_harnesses(verbose=True):
                   "-x", "hip", h, "-o", os.path.join(out, lib)])
             if verbose:
                 print(f"  built tests/_build/{lib}")
+    # the HIP runtime's stand-in for tests of the host code
+    fake = os.path.join(ROOT, "tests", "fake_hip", "fake_hip.cpp")
+    if os.path.exists(fake):
+        _run(["g++", "-O1", "-fPIC", "-shared", "-std=c++17", "-Wall", "-I", "/opt/rocm/include", fake, "-o",
+              os.path.join(out, "libfake_hip.so"), "-ldl"])
+        if verbose:
+            print("  built tests/_build/libfake_hip.so")
     mexdir = os.path.join(PKG, "mex")
     shim = os.path.join(ROOT, "tests", "mexshim")
     for name in ("MCmatlab_mex.c", "finiteElementHeatPropagator_mex.c", "getDownsampledParamVals_mex.c"):

@@ -1037,7 +1037,8 @@ int mcm_mc_plan_simulate(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, uint64_
 int mcm_mc_plan_tallies(mcm_mc_plan* pl, const double** d_deposit, uint64_t* nPhotons) {
   if (!pl) return fail(MCM_ERR_INVALID_ARGUMENT, "null plan");
   MCM_HIP(hipSetDevice(pl->device));
-  MCM_HIP(hipStreamSynchronize(pl->stream));
+  // runs on a caller's stream count too: what is handed out below is a copy
+  MCM_HIP(hipDeviceSynchronize());
   McCounters c;
   MCM_HIP(hipMemcpy(&c, pl->counters.p, sizeof c, hipMemcpyDeviceToHost));
   int rc = fold_replicas(pl);
