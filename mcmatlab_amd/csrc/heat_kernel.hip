@@ -1694,9 +1694,11 @@ using namespace mcm;
 
 struct HeatBuf {
   void* p = nullptr;
-  ~HeatBuf() {
+  void release() {
     if (p) (void)hipFree(p);
+    p = nullptr;
   }
+  ~HeatBuf() { release(); }
 };
 
 // An instantiated graph of `steps` time steps at one (dt, lights) setting,
@@ -1956,7 +1958,13 @@ int ensure_factors(mcm_heat_plan* P, int64_t steps, double dt) {
   }
   const int n[3] = {P->nx, P->ny, P->nz};
   for (int d = 0; d < 3; ++d)
-    if (line32_lines(n[d]) && !P->fac[d].p) MCM_HIP(hipMalloc(&P->fac[d].p, (size_t)P->L * 4));
+    if (line32_lines(n[d]) && !P->fac[d].p && hipMalloc(&P->fac[d].p, (size_t)P->L * 4) != hipSuccess) {
+      (void)hipGetLastError();
+      P->fac[d].p = nullptr;
+      for (HeatBuf& f : P->fac) f.release();  // (all or none: nothing captured reads them)
+      P->facReady = false;
+      return MCM_OK;
+    }
   P->facReady = true;
   P->facDt = dt;
   const HeatArgs<float> a = make_args<float>(P, dt, 0);

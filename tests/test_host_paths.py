@@ -27,3 +27,38 @@ def test_tallies_wait_for_every_stream(copies):
     device = events.index("sync device")
     assert not any(e.startswith(("launch", "memcpy")) for e in events[:device])
     assert any("mc_linear_nfr" in e for e in events[device:])
+
+
+HEAT = """
+from test_gpu_heat_lines import line_case
+T0, Om0, P = line_case((35, 21, 18), 0.3, steps=6)
+"""
+
+
+def modes(log):
+    """The modes (0 row by row, 1 from factors, 2 building them) of the FP32 line sweeps launched."""
+    names = [ln.split()[1] for ln in log if "heat_sweep_lines32" in ln]
+    return {int(n.split("heat_sweep_lines32")[1].split("ELi")[2].split("EL")[0]) for n in names}
+
+
+@pytest.mark.parametrize("room", [0, 1, 2, 3])  # of the three line factors
+def test_fp32_runs_without_memory_for_line_factors(room):
+    r = fakehip.run(HEAT + f"""
+plan = api.HeatPlan(T0, Om0, P, precision="fp32", graph_steps=2)
+voxels = 35 * 21 * 18
+fake.fake_peak(1)
+before = fake.fake_peak(0)
+fake.fake_set_limit(before + {room} * voxels * 4)
+log()
+plan.advance(6, 0.3, 1)
+first = log()
+fake.fake_peak(1)
+held = fake.fake_peak(0) - before
+fake.fake_set_limit(1 << 40)
+plan.advance(6, 0.3, 1)
+result(first=first, held=held, second=log(), voxels=voxels)
+""")
+    # with too little room: none kept, rows computed on the way; used when there is room again
+    assert modes(r["first"]) == ({1, 2} if room == 3 else {0})
+    assert r["held"] == (12 * r["voxels"] if room == 3 else 0)
+    assert modes(r["second"]) == (set() if room == 3 else {1, 2})  # (a replay of the first run's graph launches no kernel)
