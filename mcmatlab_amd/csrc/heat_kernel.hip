@@ -2561,23 +2561,31 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
   // target voxels: the mask, or every voxel whose medium has E != 0
   std::vector<uint8_t> mask((size_t)L);
   for (int64_t i = 0; i < L; ++i) mask[i] = targetMask ? (targetMask[i] != 0) : (in->E[in->M[i]] != 0);
-  HeatBuf dMask, chk, seg;
+  HeatBuf dMask, chk, seg, lam, lamN, mu1, mu2, mu3, dQ, s1, s2, dC;
   if ((rc = halloc(dMask, (size_t)L))) return rc;
   MCM_HIP(hipMemcpyAsync(dMask.p, mask.data(), (size_t)L, hipMemcpyHostToDevice, s));
   // The reverse sweep needs the state at every step.  Where all of them fit in
   // kAdjointStates they are kept (one segment, no checkpoint), else the steps of
   // one segment at a time are run again from its checkpoint (96 x 80 x 72, 120
   // steps: 10.7 ms a call kept, 14.8 with three segments of 40 and copies).
+  // What the sweep cannot do without is allocated first.
   const bool gradients = out->dJ_dQ || out->dJ_dT0 || out->dJ_dc;
+  const int nBins = P->nM * P->nM * 3;
+  if (gradients && ((rc = halloc(lam, bytes)) || (rc = halloc(lamN, bytes)) || (rc = halloc(mu1, bytes)) || (rc = halloc(mu2, bytes)) ||
+                    (rc = halloc(mu3, bytes)) || (rc = halloc(dQ, bytes))))
+    return rc;
+  // the step's intermediate states and the coefficient sums
+  if (out->dJ_dc && ((rc = halloc(s1, bytes)) || (rc = halloc(s2, bytes)) || (rc = halloc(dC, (size_t)nBins * sizeof(double))))) return rc;
+  int64_t C = std::min<int64_t>(checkpointEvery > 0 ? checkpointEvery : 100, std::max<int64_t>(N, 1));
+  int64_t nChk = std::max<int64_t>(1, (N + C - 1) / C);
   bool keep = gradients && (size_t)(N + 1) <= kAdjointStates / bytes;
   if (keep && hipMalloc(&seg.p, (size_t)(N + 1) * bytes) != hipSuccess) {
     (void)hipGetLastError();
     seg.p = nullptr;
     keep = false;
   }
-  const int64_t C = keep ? std::max<int64_t>(N, 1) : checkpointEvery > 0 ? checkpointEvery : 100;
-  const int64_t nChk = keep ? 0 : std::max<int64_t>(1, (N + C - 1) / C);
-  if (!keep && (rc = halloc(chk, (size_t)nChk * bytes))) return rc;
+  if (keep) C = std::max<int64_t>(N, 1), nChk = 0;
+  else if ((rc = halloc(chk, (size_t)nChk * bytes)) || (gradients && (rc = halloc(seg, (size_t)(C + 1) * bytes)))) return rc;
   auto chkp = [&](int64_t k) { return (double*)chk.p + (size_t)k * L; };
   auto segp = [&](int64_t k) { return (double*)seg.p + (size_t)k * L; };
   // steps n0 .. n1 - 1 from the state in segp(0) into segp(1), segp(2), ...: each
@@ -2622,16 +2630,7 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
   if (!gradients) return MCM_OK;
   if (P->nz > 65535) return fail(MCM_ERR_UNSUPPORTED, "heat adjoint: nz > 65535 z planes");
   // reverse sweep, one checkpoint segment at a time
-  HeatBuf lam, lamN, mu1, mu2, mu3, dQ, s1, s2, dC;
-  const int nBins = P->nM * P->nM * 3;
-  if ((!keep && (rc = halloc(seg, (size_t)(C + 1) * bytes))) || (rc = halloc(lam, bytes)) || (rc = halloc(lamN, bytes)) || (rc = halloc(mu1, bytes)) ||
-      (rc = halloc(mu2, bytes)) || (rc = halloc(mu3, bytes)) || (rc = halloc(dQ, bytes)))
-    return rc;
-  if (out->dJ_dc) {
-    // the step's intermediate states and the coefficient sums
-    if ((rc = halloc(s1, bytes)) || (rc = halloc(s2, bytes)) || (rc = halloc(dC, (size_t)nBins * sizeof(double)))) return rc;
-    MCM_HIP(hipMemsetAsync(dC.p, 0, (size_t)nBins * sizeof(double), s));
-  }
+  if (out->dJ_dc) MCM_HIP(hipMemsetAsync(dC.p, 0, (size_t)nBins * sizeof(double), s));
   MCM_HIP(hipMemsetAsync(lam.p, 0, bytes, s));
   MCM_HIP(hipMemsetAsync(dQ.p, 0, bytes, s));
   const int tpb = kHeatTPB;

@@ -62,3 +62,30 @@ result(first=first, held=held, second=log(), voxels=voxels)
     assert modes(r["first"]) == ({1, 2} if room == 3 else {0})
     assert r["held"] == (12 * r["voxels"] if room == 3 else 0)
     assert modes(r["second"]) == (set() if room == 3 else {1, 2})  # (a replay of the first run's graph launches no kernel)
+
+
+ADJOINT = """
+from test_gpu_heat_lines import line_case
+T0, Om0, P = line_case((16, 16, 16), 0.05, steps=200)
+state = 16 ** 3 * 8
+def peak(**kw):
+    fake.fake_peak(1)
+    r = api.heat_adjoint(T0, Om0, P, **kw)
+    return fake.fake_peak(1)
+"""
+
+
+def test_adjoint_falls_back_to_checkpoints_when_the_kept_states_leave_no_room():
+    """The states that are kept where they fit never take the room of what the
+    reverse sweep cannot do without."""
+    r = fakehip.run(ADJOINT + """
+base = peak(grads=False, checkpointEvery=200) - state  # less its one checkpoint
+peaks = []
+# from room for the checkpointed run (10 checkpoints and 21 states of a segment beside the sweep's 6 fields) to more
+# than the kept one needs
+for states in (40, 100, 200, 203, 206, 207, 208, 300):
+    fake.fake_set_limit(base + states * state)
+    peaks.append((peak(checkpointEvery=20) - base) / state)
+result(peaks=peaks)
+""")
+    assert all(p < 40 for p in r["peaks"][:5]) and all(p > 200 for p in r["peaks"][5:])
