@@ -333,10 +333,16 @@ int mcm_heat_plan_destroy(mcm_heat_plan *plan);
  *            conductivities enter through; chain rule to TC on the caller's
  *            side) [K s],
  * the exact derivatives of the discrete scheme (up to rounding).  States are
- * all kept where they fit in 4 GiB of device memory, else checkpointed every
- * checkpointEvery steps (0: 100) and recomputed one segment at a time on the
- * way back.  Needs precision MCM_HEAT_FP64, scheme
+ * checkpointed every checkpointEvery steps (0: 100) and recomputed one segment
+ * at a time on the way back, or all kept (the same results, half of the forward
+ * work) where they take no more memory than that would, or fit in
+ * MCM_HEAT_ADJOINT_STATES bytes (MCM_HEAT_ADJOINT_STATES_PERIOD when
+ * checkpointEvery is given) and the device has them to spare.
+ * mcm_heat_adjoint_run_within takes that limit from the caller: 0 leaves the
+ * checkpoints alone to bound the memory.  Needs precision MCM_HEAT_FP64, scheme
  * MCM_HEAT_DGADI and a damage input (Omega). */
+#define MCM_HEAT_ADJOINT_STATES ((int64_t)4 << 30)
+#define MCM_HEAT_ADJOINT_STATES_PERIOD ((int64_t)1 << 30)
 typedef struct mcm_heat_segment {
   int64_t steps;
   double dt;
@@ -352,6 +358,9 @@ typedef struct mcm_heat_adjoint_output {
 } mcm_heat_adjoint_output;
 int mcm_heat_adjoint_run(const mcm_heat_input *in, const mcm_heat_segment *segments, int64_t nSegments,
                          const uint8_t *targetMask, int64_t checkpointEvery, mcm_heat_adjoint_output *out);
+int mcm_heat_adjoint_run_within(const mcm_heat_input *in, const mcm_heat_segment *segments, int64_t nSegments,
+                                const uint8_t *targetMask, int64_t checkpointEvery, int64_t maxStateBytes,
+                                mcm_heat_adjoint_output *out);
 
 /* ---- Media binning ------------------------------------------------------
  * [downsampledParamVals, binidx] = getDownsampledParamVals(paramVals, N2)

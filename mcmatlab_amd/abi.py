@@ -22,6 +22,8 @@ MCM_HEAT_FP64 = 0
 MCM_HEAT_FP32 = 1
 MCM_HEAT_DGADI = 0
 MCM_HEAT_EXPLICIT = 1
+MCM_HEAT_ADJOINT_STATES = 4 << 30
+MCM_HEAT_ADJOINT_STATES_PERIOD = 1 << 30
 
 _dp = C.POINTER(C.c_double)
 _fp = C.POINTER(C.c_float)

@@ -352,15 +352,22 @@ def t_dependent_heat(T, Omega, P, M, VHC, TC, d, medium, thermal_of_T, nBins, up
     return state[0], state[1], Ms
 
 
+def _adjoint_states(checkpointEvery):
+    return abi.MCM_HEAT_ADJOINT_STATES_PERIOD if checkpointEvery > 0 else abi.MCM_HEAT_ADJOINT_STATES
+
+
 def heat_adjoint(T, Omega, P, segments=None, targetMask=None, checkpointEvery=0, grads=True, T_f64=None, Omega_f64=None,
-                 coefGrad=False):
-    """mcm_heat_adjoint_run: final damage J summed over the target voxels
+                 coefGrad=False, maxStateBytes=None):
+    """mcm_heat_adjoint_run_within: final damage J summed over the target voxels
     (targetMask, default: media with E != 0) after the schedule `segments`
     = [(steps, dt, lightsOn), ...] (default: P's steps, dt, lightsOn) of FP64
     DG-ADI steps, and its exact discrete gradients with respect to the
     heating rate dTdt_abs and the initial temperature (grads) and to the
     conduction coefficients dTdtperdeltaT (coefGrad; media.conductivity_gradient
-    turns it into dJ/dTC).  Returns a dict J, dJ_dQ, dJ_dT0 ([nx,ny,nz]
+    turns it into dJ/dTC).  States are checkpointed every checkpointEvery
+    steps (0: 100), or all kept where they fit in maxStateBytes (default 4
+    GiB, 1 GiB when checkpointEvery is given; 0 bounds the memory by the
+    checkpoints alone); the results are the same.  Returns a dict J, dJ_dQ, dJ_dT0 ([nx,ny,nz]
     Fortran order, or None), dJ_dc ([nM,nM,3] or None), Omega (final FP64
     damage)."""
     inp = abi.HeatInputs(T, Omega, P, precision=abi.MCM_HEAT_FP64, scheme=abi.MCM_HEAT_DGADI, T_f64=T_f64, Omega_f64=Omega_f64)
@@ -386,9 +393,11 @@ def heat_adjoint(T, Omega, P, segments=None, targetMask=None, checkpointEvery=0,
         nM = int(inp.struct.nM)
         gc = np.zeros(nM * nM * 3)
         out.dJ_dc = gc.ctypes.data_as(C.POINTER(C.c_double))
-    check(lib().mcm_heat_adjoint_run(C.byref(inp.struct), arr, len(segs),
-                                     None if mask is None else mask.ctypes.data_as(C.POINTER(C.c_uint8)),
-                                     int(checkpointEvery), C.byref(out)))
+    if maxStateBytes is None:
+        maxStateBytes = _adjoint_states(checkpointEvery)
+    check(lib().mcm_heat_adjoint_run_within(C.byref(inp.struct), arr, len(segs),
+                                            None if mask is None else mask.ctypes.data_as(C.POINTER(C.c_uint8)),
+                                            int(checkpointEvery), int(maxStateBytes), C.byref(out)))
     f = lambda a: None if a is None else a.reshape(shape, order="F")
     return {"J": out.J, "dJ_dQ": f(gq), "dJ_dT0": f(gt), "Omega": f(om),
             "dJ_dc": None if gc is None else gc.reshape(int(inp.struct.nM), int(inp.struct.nM), 3, order="F")}
@@ -402,8 +411,8 @@ def heat_damage_function():
     per medium [nM]) times the incoming gradient.  `setup` is a dict with the
     heat MEX fields P (M, A, E, sensors, heatBoundaryType; its dTdt_abs and
     dTdtperdeltaT are replaced), VHC [nM], d = (dx, dy, dz), segments
-    [(steps, dt, lightsOn), ...] and optionally targetMask and
-    checkpointEvery.  Usage:
+    [(steps, dt, lightsOn), ...] and optionally targetMask,
+    checkpointEvery and maxStateBytes.  Usage:
         HD = heat_damage_function()
         J = HD.apply(Q, T0, TC, setup)
         J.backward()   # Q.grad, T0.grad, TC.grad
@@ -424,7 +433,8 @@ def heat_damage_function():
             t0 = np.asfortranarray(T0.detach().cpu().numpy().astype(np.float64))
             om0 = np.zeros(t0.shape, np.float32)
             r = heat_adjoint(t0.astype(np.float32), om0, P, segments=setup["segments"], targetMask=setup.get("targetMask"),
-                             checkpointEvery=setup.get("checkpointEvery", 0), T_f64=t0, coefGrad=True)
+                             checkpointEvery=setup.get("checkpointEvery", 0), T_f64=t0, coefGrad=True,
+                             maxStateBytes=setup.get("maxStateBytes"))
             gtc = conductivity_gradient(r["dJ_dc"], VHC, tc, dx, dy, dz)
             dev = Q.device
             ctx.save_for_backward(torch.from_numpy(np.ascontiguousarray(r["dJ_dQ"])).to(dev, Q.dtype),
@@ -445,9 +455,14 @@ def heat_adjoints(cases, workers=4, **kw):
     runs on its own plan and stream from its own host thread (the library
     releases the interpreter lock while it works), so small models overlap
     on the GPU.  cases = [(T, Omega, P, segments), ...]; keyword arguments
-    go to every heat_adjoint call.  Returns the results in order."""
+    go to every heat_adjoint call (maxStateBytes is what the calls that run
+    together may take between them).  Returns the results in order."""
     from concurrent.futures import ThreadPoolExecutor
 
+    cases = list(cases)
+    together = max(1, min(int(workers), len(cases)))
+    total = kw.pop("maxStateBytes", None)
+    kw["maxStateBytes"] = (_adjoint_states(kw.get("checkpointEvery", 0)) if total is None else int(total)) // together
     with ThreadPoolExecutor(max_workers=max(1, int(workers))) as ex:
         futs = [ex.submit(heat_adjoint, T, Om, P, segments=segs, **kw) for T, Om, P, segs in cases]
         return [f.result() for f in futs]

@@ -2527,13 +2527,16 @@ int mcm_heat_plan_destroy(mcm_heat_plan* P) {
 }
 
 
-// Most device memory for the states that the adjoint keeps instead of
-// computing them twice.
-static constexpr size_t kAdjointStates = (size_t)4 << 30;
-
 int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segments, int64_t nSegments, const uint8_t* targetMask,
                          int64_t checkpointEvery, mcm_heat_adjoint_output* out) {
+  return mcm_heat_adjoint_run_within(in, segments, nSegments, targetMask, checkpointEvery,
+                                     checkpointEvery > 0 ? MCM_HEAT_ADJOINT_STATES_PERIOD : MCM_HEAT_ADJOINT_STATES, out);
+}
+
+int mcm_heat_adjoint_run_within(const mcm_heat_input* in, const mcm_heat_segment* segments, int64_t nSegments, const uint8_t* targetMask,
+                                int64_t checkpointEvery, int64_t maxStateBytes, mcm_heat_adjoint_output* out) {
   if (!in || !out) return fail(MCM_ERR_INVALID_ARGUMENT, "null argument");
+  if (maxStateBytes < 0) return fail(MCM_ERR_INVALID_ARGUMENT, "maxStateBytes must be non-negative");
   if (in->precision != MCM_HEAT_FP64 || in->scheme != MCM_HEAT_DGADI)
     return fail(MCM_ERR_UNSUPPORTED, "the adjoint is implemented for the FP64 DG-ADI scheme");
   if (!in->Omega && !in->Omega_f64) return fail(MCM_ERR_INVALID_ARGUMENT, "the objective is the damage integral: Omega is required");
@@ -2565,10 +2568,11 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
   if ((rc = halloc(dMask, (size_t)L))) return rc;
   MCM_HIP(hipMemcpyAsync(dMask.p, mask.data(), (size_t)L, hipMemcpyHostToDevice, s));
   // The reverse sweep needs the state at every step.  Where all of them fit in
-  // kAdjointStates they are kept (one segment, no checkpoint), else the steps of
-  // one segment at a time are run again from its checkpoint (96 x 80 x 72, 120
-  // steps: 10.7 ms a call kept, 14.8 with three segments of 40 and copies).
-  // What the sweep cannot do without is allocated first.
+  // maxStateBytes, or are no more than the checkpoints and a segment, they are
+  // kept (one segment, no checkpoint), else the steps of one segment at a time
+  // are run again from its checkpoint (96 x 80 x 72, 120 steps: 10.7 ms a call
+  // kept, 14.8 with three segments of 40 and copies).  What the sweep cannot do
+  // without is allocated first.
   const bool gradients = out->dJ_dQ || out->dJ_dT0 || out->dJ_dc;
   const int nBins = P->nM * P->nM * 3;
   if (gradients && ((rc = halloc(lam, bytes)) || (rc = halloc(lamN, bytes)) || (rc = halloc(mu1, bytes)) || (rc = halloc(mu2, bytes)) ||
@@ -2578,7 +2582,7 @@ int mcm_heat_adjoint_run(const mcm_heat_input* in, const mcm_heat_segment* segme
   if (out->dJ_dc && ((rc = halloc(s1, bytes)) || (rc = halloc(s2, bytes)) || (rc = halloc(dC, (size_t)nBins * sizeof(double))))) return rc;
   int64_t C = std::min<int64_t>(checkpointEvery > 0 ? checkpointEvery : 100, std::max<int64_t>(N, 1));
   int64_t nChk = std::max<int64_t>(1, (N + C - 1) / C);
-  bool keep = gradients && (size_t)(N + 1) <= kAdjointStates / bytes;
+  bool keep = gradients && ((size_t)(N + 1) <= (size_t)maxStateBytes / bytes || N + 1 <= nChk + C + 1);
   if (keep && hipMalloc(&seg.p, (size_t)(N + 1) * bytes) != hipSuccess) {
     (void)hipGetLastError();
     seg.p = nullptr;

@@ -89,3 +89,46 @@ for states in (40, 100, 200, 203, 206, 207, 208, 300):
 result(peaks=peaks)
 """)
     assert all(p < 40 for p in r["peaks"][:5]) and all(p > 200 for p in r["peaks"][5:])
+
+
+def test_adjoint_memory_is_bounded_by_the_caller():
+    """Kept states take at most 1 GiB beside an explicit checkpoint period (4 GiB
+    without one), what the caller allows, or what the checkpoints would take;
+    calls that run together share the limit."""
+    r = fakehip.run(ADJOINT + """
+base = peak(grads=False, checkpointEvery=200) - state
+sweep = 6 * state
+def states(**kw):
+    return (peak(**kw) - base - sweep) / state
+out = dict(
+    default=states(),
+    period=states(checkpointEvery=20),
+    none=states(checkpointEvery=20, maxStateBytes=0),          # 10 checkpoints, 21 states of a segment
+    short=states(checkpointEvery=20, maxStateBytes=200 * state),
+    enough=states(checkpointEvery=20, maxStateBytes=201 * state),
+    asked=states(checkpointEvery=200, maxStateBytes=0),        # as many as one segment
+    unset=states(maxStateBytes=0),                             # every 100 steps
+)
+limits = []
+def note(*a, **kw):
+    limits.append(kw["maxStateBytes"])
+api.heat_adjoint = note
+one = (T0, Om0, P, None)
+api.heat_adjoints([one] * 8, workers=4, checkpointEvery=20)
+api.heat_adjoints([one] * 2, workers=4)
+api.heat_adjoints(iter([one] * 8), workers=8, maxStateBytes=800)
+result(out=out, limits=sorted(set(limits)))
+""")
+    assert r["out"] == {"default": 201, "period": 201, "none": 31, "short": 31, "enough": 201, "asked": 201, "unset": 103}
+    assert r["limits"] == [100, 1 << 28, 2 << 30]
+
+
+def test_adjoint_refuses_a_negative_memory_limit():
+    r = fakehip.run(ADJOINT + """
+try:
+    peak(maxStateBytes=-1)
+    result(code=0)
+except _lib.MCMError as e:
+    result(code=e.code)
+""")
+    assert r["code"] == -1
