@@ -234,7 +234,10 @@ typedef struct mcm_mc_item {
  * faces sized as mcm_mc_output_sizes reports divided by nL), nPhotons,
  * nPhotonsCollected, nThreads and the batch's simulationTime.  Deposition
  * criteria, 3D sources and wavelength-dependent refractive indices are
- * MCM_ERR_UNSUPPORTED; nItems * nM must not exceed 2048. */
+ * MCM_ERR_UNSUPPORTED; nItems * nM must not exceed 2048.  The call holds the
+ * FP64 tallies of every item in device memory; with many packets (1/256 of the
+ * voxels of a copy each) the fluence in 2, 4 or 8 copies within 16 GiB, or in
+ * one where there is no memory for more. */
 int mcm_mc_batch_run(mcm_mc_plan *plan, const mcm_mc_item *items, int64_t nItems, mcm_mc_output *outs);
 
 /* Work items on different grids (no reference counterpart): item i runs
@@ -247,7 +250,7 @@ int mcm_mc_batch_run(mcm_mc_plan *plan, const mcm_mc_item *items, int64_t nItems
  * device; deposition criteria and 3D sources are MCM_ERR_UNSUPPORTED, the
  * items of one plan need equal refractive indices, nItems is 1..256 and
  * nItems * (largest nM) must not exceed 2048.  Uses plans[0]'s stream,
- * counters and packet records. */
+ * counters and packet records, and memory like mcm_mc_batch_run. */
 typedef struct mcm_mc_multi_item {
   int64_t plan;        /* index into plans */
   int64_t iL;          /* wavelength of that plan */

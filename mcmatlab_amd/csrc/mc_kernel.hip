@@ -842,15 +842,22 @@ int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed,
 }
 
 // Fluence copies of a launch of several items, `voxels` in all and LB in one:
-// those of a plan, within 16 GiB (one copy if there is no memory for more).  The
-// items of a batch run one after another, so one item's copies are in use at a
-// time (8 items of 150^3, 3.3 10^6 packets of a pencil beam: kernel 52.3 ms with
-// one copy, 25.1 ms with eight; 64 items, 1.45 10^8 packets: 2.35 s with one,
-// 1.22 s with eight).
+// at most those of a plan, within 16 GiB (one copy if there is no memory for
+// more).  The items of a batch run one after another, so one item's copies are
+// in use at a time (8 items of 150^3, 3.3 10^6 packets of a pencil beam: kernel
+// 52.3 ms with one copy, 25.1 ms with eight; 64 items, 1.45 10^8 packets: 2.35 s
+// with one, 1.22 s with eight).
+// Copies pay by the packet (narrow beams) and cost by the voxel, which is
+// cleared and summed in each: n copies take n packets in kItemCopyVoxels voxels.
+// Whole calls with 1, 2, 4 and 8 copies, ms, pencil / tophat beam: 64 items of
+// 150^3 and 300 packets 77 80 80 84 / 79 81 203 397, 30000 packets (2.3 copies)
+// 104 97 99 101 / 88 92 95 99; 8 items of 150^3 and 300000 packets (23) 51 36 32
+// 31 / 26 25 26 27.
 constexpr int64_t kItemCopiesBytes = (int64_t)16 << 30;
-int item_copies(int64_t LB, int64_t voxels) {
+constexpr int64_t kItemCopyVoxels = 256;
+int item_copies(int64_t LB, int64_t voxels, uint64_t packets) {
   int n = start_copies(LB);
-  while (n > 1 && n * voxels * (int64_t)sizeof(double) > kItemCopiesBytes) n /= 2;
+  while (n > 1 && (n * voxels * (int64_t)sizeof(double) > kItemCopiesBytes || (double)packets * kItemCopyVoxels < (double)n * voxels)) n /= 2;
   return n;
 }
 
@@ -1234,7 +1241,7 @@ int mcm_mc_batch_run(mcm_mc_plan* pl, const mcm_mc_item* items, int64_t nItems, 
   B.L = pl->prm.LB;
   B.nImage = T.nImage;
   B.nFF = T.nFF;
-  B.copies = T.calcNFR ? item_copies(pl->prm.LB, nI * pl->prm.LB) : 1;
+  B.copies = T.calcNFR ? item_copies(pl->prm.LB, nI * pl->prm.LB, cum[nI]) : 1;
   B.copyStride = T.calcNFR ? nI * pl->prm.LB : 1;
   if ((rc = zero_copies(dNFR, B.copies, B.copyStride, s)) ||
       (rc = zeros(dImg, (size_t)std::max<int64_t>(nI * T.nImage, 1) * sizeof(double), s)) ||
@@ -1331,7 +1338,9 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
     tallies = tallies || T.base.useLC || T.base.farFieldRes;
   }
   DevBuf dTal[9], dColl, dOff, dParams, dGeom;
-  int copies = item_copies(tot[0] / nI, tot[0]);
+  uint64_t packets = 0;
+  for (int i = 0; i < nI; ++i) packets += items[i].nPhotons;
+  int copies = item_copies(tot[0] / nI, tot[0], packets);
   const int64_t copyStride = std::max<int64_t>(tot[0], 1);
   if ((rc = zero_copies(dTal[0], copies, copyStride, s))) return rc;
   for (int k = 1; k < 9; ++k)

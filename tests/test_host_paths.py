@@ -132,3 +132,22 @@ except _lib.MCMError as e:
     result(code=e.code)
 """)
     assert r["code"] == -1
+
+
+@pytest.mark.parametrize("kind", ["batch", "multi"])
+def test_fluence_copies_of_a_batch_follow_its_packets(kind):
+    """Copies pay by the packet and cost by the voxel: n copies from n packets in
+    256 voxels."""
+    r = fakehip.run(f"""
+import models
+plan = api.MCPlan(models.base(n=40))
+out = {{}}
+for packets in (1, 499, 501, 999, 1001, 1999, 2001, 20000):
+    items = [(0, packets, 1, 0)] * 16
+    log()
+    plan.batch(items) if {kind == "batch"} else api.multi_run([plan], [(0, *it) for it in items])
+    slices = [int(l.split()[1]) / (16 * 40 ** 3 * 8) for l in log() if l.startswith("malloc ")]
+    out[packets] = max(slices)
+result(**{{str(k): v for k, v in out.items()}})
+""")
+    assert r == {"1": 1, "499": 1, "501": 2, "999": 2, "1001": 4, "1999": 4, "2001": 8, "20000": 8}
