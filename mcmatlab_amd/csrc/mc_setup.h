@@ -98,11 +98,17 @@ inline std::string build_mc_tables(const mcm_mc_input* in, McTables& T, bool hos
   T.nL = (int)in->nL;
   T.L = in->nx * in->ny * in->nz;
   T.M0.resize((size_t)T.L);
-  bool outside = false;
-  for (int64_t k = 0; k < T.L; ++k) {
-    const uint8_t m = in->M[k];
-    outside |= (m == 0) | (m > T.nM);  // (of m, not m - 1: 0 - 1 is medium 255 of 256)
-    T.M0[k] = (uint8_t)(m - 1);
+  // (locals: a store of a byte may alias anything; m == 0 by itself, since 0 - 1
+  // is medium 255 of 256)
+  const uint8_t* const M = in->M;
+  uint8_t* const M0 = T.M0.data();
+  const int64_t L = T.L;
+  const uint8_t last = (uint8_t)std::min(T.nM, 255);
+  uint8_t outside = 0;
+  for (int64_t k = 0; k < L; ++k) {
+    const uint8_t m = M[k];
+    outside |= (uint8_t)(m == 0) | (uint8_t)(m > last);
+    M0[k] = (uint8_t)(m - 1);
   }
   if (outside) return "M holds a medium index outside 1..nM";
   T.timed = std::isnan(in->nPhotonsRequested);
