@@ -863,8 +863,8 @@ int item_copies(int64_t LB, int64_t voxels, uint64_t packets) {
 
 // Normalised outputs of one work item from its FP64 tally slices
 // (normalizeDepositionAndResetO, MCmatlablib.c:1186-1250); null slices are
-// skipped.
-int finish_item(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, double* nfr, int copies, int64_t stride, const double* img, const double* ff,
+// skipped.  `stage` is the launch's: one pinned block whatever the plans.
+int finish_item(mcm_mc_plan* pl, HostStage& stage, int64_t iL, uint64_t nPhotons, double* nfr, int copies, int64_t stride, const double* img, const double* ff,
                 const double* const ni[6], unsigned long long collected, double minutes, int64_t lanes, mcm_mc_output& o) {
   const McTables& T = pl->T;
   hipStream_t s = pl->stream;
@@ -886,7 +886,7 @@ int finish_item(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, double* nfr, int
     hipLaunchKernelGGL(mc_normalize_nfr, dim3((unsigned)nb), dim3(tpb), 0, s, nfr, copies, stride, pl->Mlin.as<uint8_t>(),
                        pl->muaNorm.as<double>() + (size_t)iL * T.nM, T.V * normfactor, pl->nfrOut.as<float>(), voxel_map(pl), T.L);
     MCM_HIP(hipGetLastError());
-    if ((rc = pl->stage.download(o.NFR, pl->nfrOut.p, (size_t)T.L * sizeof(float), pl->device, s))) return rc;
+    if ((rc = stage.download(o.NFR, pl->nfrOut.p, (size_t)T.L * sizeof(float), pl->device, s))) return rc;
   }
   if (T.base.useLC) {
     const int64_t LLC = (int64_t)T.lcRes0 * T.lcRes0;
@@ -1278,7 +1278,7 @@ int mcm_mc_batch_run(mcm_mc_plan* pl, const mcm_mc_item* items, int64_t nItems, 
   for (int i = 0; i < nI; ++i) {
     const double* ni[6];
     for (int f = 0; f < 6; ++f) ni[f] = dNI[f].as<double>() + (size_t)i * T.nNI[f];
-    if ((rc = finish_item(pl, items[i].iL, items[i].nPhotons, T.calcNFR ? dNFR.as<double>() + (size_t)i * pl->prm.LB : nullptr,
+    if ((rc = finish_item(pl, pl->stage, items[i].iL, items[i].nPhotons, T.calcNFR ? dNFR.as<double>() + (size_t)i * pl->prm.LB : nullptr,
                           B.copies, B.copyStride, dImg.as<double>() + (size_t)i * T.nImage, dFF.as<double>() + (size_t)i * T.nFF, ni, coll[i], minutes,
                           (int64_t)blocks * pl->threads, outs[i])))
       return rc;
@@ -1462,7 +1462,7 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
     const double* ni[6];
     for (int f = 0; f < 6; ++f) ni[f] = dTal[3 + f].as<double>() + o[3 + f];
     const unsigned long long coll = (unsigned long long)outs[i].nPhotonsCollected;
-    if ((rc = finish_item(pl, items[i].iL, items[i].nPhotons, pl->T.calcNFR ? dTal[0].as<double>() + o[0] : nullptr,
+    if ((rc = finish_item(pl, pl0->stage, items[i].iL, items[i].nPhotons, pl->T.calcNFR ? dTal[0].as<double>() + o[0] : nullptr,
                           copies, copyStride, dTal[1].as<double>() + o[1], dTal[2].as<double>() + o[2], ni, coll, minutes,
                           (int64_t)blocks * pl0->threads, outs[i])))
       return rc;

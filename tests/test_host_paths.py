@@ -151,3 +151,15 @@ for packets in (1, 499, 501, 999, 1001, 1999, 2001, 20000):
 result(**{{str(k): v for k, v in out.items()}})
 """)
     assert r == {"1": 1, "499": 1, "501": 2, "999": 2, "1001": 4, "1999": 4, "2001": 8, "20000": 8}
+
+
+def test_a_multi_grid_launch_downloads_through_one_pinned_block():
+    r = fakehip.run("""
+import models
+m = models.base(n=130)
+plans = [api.MCPlan(m) for _ in range(3)]
+log()
+api.multi_run(plans, [(k, 0, 100, 1, 0) for k in range(3)])
+result(pinned=[l for l in log() if l.startswith("pinned")])
+""")
+    assert len(r["pinned"]) == 1
