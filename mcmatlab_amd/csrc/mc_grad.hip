@@ -306,13 +306,18 @@ using namespace mcm;
 // Largest number of packets per launch (64-byte records).
 constexpr uint64_t kGradLaunchPackets = 1ull << 22;
 
-static int ensure_grad_records(mcm_mc_plan* pl, uint64_t n) {
+// Records for n packets, or fewer (then n becomes that) where there is no memory
+// for as many.
+static int ensure_grad_records(mcm_mc_plan* pl, uint64_t& n) {
   if (n <= pl->gradRecCap) return MCM_OK;
   MCM_HIP(hipStreamSynchronize(pl->stream));
-  if (pl->gradRec.p) MCM_HIP(hipFree(pl->gradRec.p));
-  pl->gradRec.p = nullptr;
-  pl->gradRecCap = 0;
-  MCM_HIP(hipMalloc(&pl->gradRec.p, (size_t)n * sizeof(LaunchRecord)));
+  for (;; n = (n + 1) / 2) {
+    free_buf(pl->gradRec);
+    pl->gradRecCap = 0;
+    if (hipMalloc(&pl->gradRec.p, (size_t)n * sizeof(LaunchRecord)) == hipSuccess) break;
+    (void)hipGetLastError();
+    if (n <= kFewestLaunchPackets) return fail(MCM_ERR_OUT_OF_MEMORY, "Error: Out of memory (packet records for %llu packets)", (unsigned long long)n);
+  }
   pl->gradRecCap = n;
   return MCM_OK;
 }
@@ -373,10 +378,13 @@ extern "C" int mcm_mc_grad_run(mcm_mc_plan* pl, const mcm_mc_grad_input* in, mcm
   int per = 0;
   const void* kern = T.fresnelPossible ? (const void*)mc_grad<true> : (const void*)mc_grad<false>;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, 256, 0) != hipSuccess || per < 1) per = 2;
+  uint64_t most = kGradLaunchPackets;
   for (uint64_t done = 0; done < in->nPhotons; done += g.nPackets) {
     g.firstPacket = done;
-    g.nPackets = std::min<uint64_t>(in->nPhotons - done, kGradLaunchPackets);
+    g.nPackets = std::min<uint64_t>(in->nPhotons - done, most);
+    const uint64_t asked = g.nPackets;
     if ((rc = ensure_grad_records(pl, g.nPackets))) return rc;
+    if (g.nPackets < asked) most = g.nPackets;
     if (done) MCM_HIP(hipMemsetAsync(g.next, 0, sizeof *g.next, s));
     LaunchRecord* rec = pl->gradRec.as<LaunchRecord>();
     const dim3 b(256), grid(launch_blocks(pl, per * cu_count(pl->device), g.nPackets));

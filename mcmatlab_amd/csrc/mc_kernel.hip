@@ -760,21 +760,24 @@ int set_replicas(mcm_mc_plan* pl, int R) {
   return MCM_OK;
 }
 
-int ensure_records(mcm_mc_plan* pl, uint64_t n) {
-  if (n <= pl->recCap) return MCM_OK;
+// Record buffers for n packets of a launch (escapes: for their escapes too),
+// kept by the plan.  Where there is no memory for that many, n becomes the number
+// there is memory for, down to kFewestLaunchPackets.
+int ensure_records(mcm_mc_plan* pl, uint64_t& n, bool escapes) {
+  if (n <= pl->recCap && (!escapes || n <= pl->escapeCap)) return MCM_OK;
   MCM_HIP(hipDeviceSynchronize());  // earlier launches may use the old buffers on any stream
-  for (DevBuf* b : {&pl->launchRec, &pl->escapeRec})
-    if (b->p) {
-      MCM_HIP(hipFree(b->p));
-      b->p = nullptr;
-    }
-  if (hipMalloc(&pl->launchRec.p, (size_t)n * sizeof(LaunchRecord)) != hipSuccess ||
-      hipMalloc(&pl->escapeRec.p, (size_t)n * sizeof(EscapeRecord)) != hipSuccess) {
+  for (;; n = (n + 1) / 2) {
+    free_buf(pl->launchRec);
+    free_buf(pl->escapeRec);
+    pl->recCap = pl->escapeCap = 0;
+    if (hipMalloc(&pl->launchRec.p, (size_t)n * sizeof(LaunchRecord)) == hipSuccess &&
+        (!escapes || hipMalloc(&pl->escapeRec.p, (size_t)n * sizeof(EscapeRecord)) == hipSuccess))
+      break;
     (void)hipGetLastError();
-    pl->recCap = 0;
-    return fail(MCM_ERR_OUT_OF_MEMORY, "Error: Out of memory (packet records for %llu packets)", (unsigned long long)n);
+    if (n <= kFewestLaunchPackets) return fail(MCM_ERR_OUT_OF_MEMORY, "Error: Out of memory (packet records for %llu packets)", (unsigned long long)n);
   }
   pl->recCap = n;
+  if (escapes) pl->escapeCap = n;
   return MCM_OK;
 }
 
@@ -786,12 +789,15 @@ size_t table_bytes(int nItems, int nM) {
 
 int occupancy_blocks(int device, bool fr, bool cr, int kind, size_t lds);
 
-// One launch of n <= kMaxLaunchPackets packets.  Without deposition
-// criteria: launch kernel -> transport -> escape tallies; with criteria the
-// transport launches and tallies inline.  `bt` (batched launches) maps the
-// global packet indices first .. first+n-1 to work items.
-int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed, uint32_t stream, hipStream_t s,
+// One launch of n <= kMaxLaunchPackets packets, or of as many as there is
+// memory for records of (n on return).  Launch kernel -> transport -> escape
+// tallies; with deposition criteria the transport tallies inline.  `bt` (batched
+// launches) maps the global packet indices first .. first+n-1 to work items.
+int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t& n, uint64_t seed, uint32_t stream, hipStream_t s,
                      const McBatch* bt = nullptr, int kind = kPlain, bool fresnel = false, bool tallies = false, int blocks_items = 0) {
+  const bool cr = kind == kPlain && pl->prm.criteriaActive != 0;
+  int rc = ensure_records(pl, n, !cr);
+  if (rc) return rc;
   McLaunch lp;
   lp.firstPacket = first;
   lp.nPackets = n;
@@ -801,14 +807,11 @@ int launch_transport(mcm_mc_plan* pl, uint64_t first, uint64_t n, uint64_t seed,
   lp.moveFrac = pl->moveFrac;
   lp.ctr = pl->counters.as<McCounters>();
   const bool fr = kind == kMulti ? fresnel : pl->T.fresnelPossible;
-  const bool cr = kind == kPlain && pl->prm.criteriaActive != 0;
   McBatch none;
   std::memset(&none, 0, sizeof none);
   const McBatch& B = bt ? *bt : none;
   const dim3 b(pl->threads), g(launch_blocks(pl, kind == kPlain ? pl->blocks : blocks_items, n));
   MCM_HIP(hipMemsetAsync(pl->counters.p, 0, sizeof(unsigned long long), s));  // nextPacket
-  int rc = ensure_records(pl, n);
-  if (rc) return rc;
   LaunchRecord* L = pl->launchRec.as<LaunchRecord>();
   EscapeRecord* E = pl->escapeRec.as<EscapeRecord>();
   const McTables& T = pl->T;
@@ -1033,9 +1036,12 @@ int mcm_mc_plan_simulate(mcm_mc_plan* pl, int64_t iL, uint64_t nPhotons, uint64_
   if (rc) return rc;
   if (s != pl->stream) MCM_HIP(hipStreamSynchronize(pl->stream));
   // launched/collected/... accumulate over launches until normalize
+  uint64_t most = kMaxLaunchPackets;
   for (uint64_t done = 0; done < nPhotons;) {
-    const uint64_t n = std::min<uint64_t>(nPhotons - done, kMaxLaunchPackets);
+    uint64_t n = std::min<uint64_t>(nPhotons - done, most);
+    const uint64_t asked = n;
     if ((rc = launch_transport(pl, firstPhoton + done, n, seed, (uint32_t)iL, s))) return rc;
+    if (n < asked) most = n;
     done += n;
   }
   return MCM_OK;
@@ -1261,9 +1267,12 @@ int mcm_mc_batch_run(mcm_mc_plan* pl, const mcm_mc_item* items, int64_t nItems, 
   MCM_HIP(hipMemsetAsync(pl->counters.p, 0, sizeof(McCounters), s));
   const auto t0 = std::chrono::steady_clock::now();
   const unsigned long long total = cum[nI];
+  uint64_t most = kMaxLaunchPackets;
   for (unsigned long long done = 0; done < total;) {
-    const uint64_t n = std::min<unsigned long long>(total - done, kMaxLaunchPackets);
+    uint64_t n = std::min<unsigned long long>(total - done, most);
+    const uint64_t asked = n;
     if ((rc = launch_transport(pl, done, n, 0, 0, s, &B, kBatch, false, false, blocks))) return rc;
+    if (n < asked) most = n;
     done += n;
   }
   MCM_HIP(hipStreamSynchronize(s));
@@ -1371,6 +1380,7 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
   }
   if ((rc = upload(dParams, params.data(), params.size(), s)) || (rc = upload(dGeom, geom.data(), geom.size(), s))) return rc;
   int blocks = pl0->blocksForced;
+  uint64_t most = kMaxLaunchPackets;
   MCM_HIP(hipMemsetAsync(pl0->counters.p, 0, sizeof(McCounters), s));
   const auto t0 = std::chrono::steady_clock::now();
   // one sequence of launches per interface class (Fresnel or matched), so
@@ -1435,14 +1445,16 @@ int mcm_mc_multi_run(mcm_mc_plan* const* plans, int64_t nPlans, const mcm_mc_mul
     // launches pays the tail of its longest-lived packets twice)
     const unsigned long long total = cum[(size_t)n];
     for (unsigned long long done = 0; done < total;) {
-      unsigned long long stop = done + std::min<unsigned long long>(total - done, kMaxLaunchPackets);
+      unsigned long long stop = done + std::min<unsigned long long>(total - done, most);
       for (int j = n; j > 0; --j)
         if (cum[(size_t)j] <= stop && cum[(size_t)j] > done) {
-          stop = cum[(size_t)j] - done >= kMaxLaunchPackets / 4 || cum[(size_t)j] == total ? cum[(size_t)j] : stop;
+          stop = cum[(size_t)j] - done >= most / 4 || cum[(size_t)j] == total ? cum[(size_t)j] : stop;
           break;
         }
-      if ((rc = launch_transport(pl0, done, stop - done, 0, 0, s, &B, kMulti, cls == 0, tallies, blocks))) return rc;
-      done = stop;
+      uint64_t launched = stop - done;
+      if ((rc = launch_transport(pl0, done, launched, 0, 0, s, &B, kMulti, cls == 0, tallies, blocks))) return rc;
+      if (launched < stop - done) most = launched;
+      done += launched;
     }
     std::vector<unsigned long long> cc((size_t)n);
     MCM_HIP(hipMemcpyAsync(cc.data(), dCollc.p, cc.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));

@@ -56,11 +56,11 @@ struct mcm_mc_plan {
   DevBuf M, Mlin, normals, media, cdfIdx, cdfs, fpid1, aid1, fpid2, aid2, S, muaNorm;
   DevBuf nfrLin;   // linear copy of the fluence tally for mcm_mc_plan_tallies
   DevBuf NFR, image, FF, NI[6], counters, nfrOut;
-  DevBuf launchRec, escapeRec;  // per-launch packet records (no deposition criteria)
+  DevBuf launchRec, escapeRec;  // per-launch packet records (of escapes: without deposition criteria)
   DevBuf gradMap, gradLin, gradOut, gradSmall;  // gradient runs: mua map, its linear form, dJ/dmua, sums/flags/counter
   int gradCopies = 1;
   DevBuf gradRec;  // launch records of a gradient run
-  uint64_t recCap = 0, gradRecCap = 0;
+  uint64_t recCap = 0, escapeCap = 0, gradRecCap = 0;
   std::vector<double> Shost;   // cumulative 3D source table of the current wavelength
   const float* sourceDistribution = nullptr;
   double power = 0;            // current wavelength's source power
@@ -95,6 +95,15 @@ inline int zeros(DevBuf& b, size_t bytes, hipStream_t s) {
   MCM_HIP(hipMemsetAsync(b.p, 0, std::max<size_t>(bytes, 8), s));
   return MCM_OK;
 }
+
+inline void free_buf(DevBuf& b) {
+  if (b.p) (void)hipFree(b.p);
+  b.p = nullptr;
+}
+
+// A run is cut into launches whose packet records there is memory for, of at
+// least this many packets.
+constexpr uint64_t kFewestLaunchPackets = 1ull << 12;
 
 // Voxel order of a plan for kernels that walk the grid in its linear (x
 // fastest) order.

@@ -163,3 +163,62 @@ api.multi_run(plans, [(k, 0, 100, 1, 0) for k in range(3)])
 result(pinned=[l for l in log() if l.startswith("pinned")])
 """)
     assert len(r["pinned"]) == 1
+
+
+def covered(log, kernel):
+    """Workgroups of each launch of a kernel."""
+    return [int(ln.split()[2]) for ln in log if ln.startswith("launch ") and kernel in ln]
+
+
+@pytest.mark.parametrize("kind", ["criteria", "plain", "batch", "multi", "grad"])
+def test_runs_take_smaller_launches_where_packet_records_do_not_fit(kind):
+    """A launch's records (64 bytes a packet, 112 with escapes) are the only
+    memory a run needs by the packet: with room for an eighth of them the run is
+    cut into eight launches, with no room for 4096 packets it is refused."""
+    r = fakehip.run(f"""
+import models
+kind = {kind!r}
+m = models.cases()["criteria_scatter" if kind == "criteria" else "pencil_bt1"]()
+plan = api.MCPlan(m)
+N = 1 << 20
+size = 64 if kind in ("criteria", "grad") else 112
+def go():
+    if kind == "batch":
+        plan.batch([(0, N, 1, 0)])
+    elif kind == "multi":
+        api.multi_run([plan], [(0, 0, N, 1, 0)])
+    elif kind == "grad":
+        plan.absorbed_power(((0, 1), (0, 1), (0, 1)), N)
+    else:
+        plan.simulate(N)
+# what the call needs beside the records
+other = api.MCPlan(m)
+plan, kept = other, plan
+fake.fake_peak(1)
+before = fake.fake_peak(0)
+go()
+rest = fake.fake_peak(1) - before - size * N
+other.close()
+plan = kept
+fake.fake_peak(1)
+before = fake.fake_peak(1)
+log()
+fake.fake_set_limit(before + rest + size * N // 8)
+go()
+cut = log()
+used = fake.fake_peak(1) - before - rest
+plan.close()
+plan = api.MCPlan(m)
+fake.fake_peak(1)
+fake.fake_set_limit(fake.fake_peak(1) + rest + size * 4000)
+try:
+    go()
+    code = 0
+except _lib.MCMError as e:
+    code = e.code
+result(cut=cut, used=used, whole=size * N // 8, code=code)
+""")
+    kernel = "mc_gradI" if kind == "grad" else "mc_transport"
+    assert len(covered(r["cut"], kernel)) == 8
+    assert r["used"] == r["whole"]
+    assert r["code"] == -2
