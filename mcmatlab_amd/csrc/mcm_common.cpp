@@ -2,7 +2,6 @@
 #include "mcm_common.h"
 
 #include <algorithm>
-#include <system_error>
 #include <thread>
 
 #include <cstdlib>
@@ -103,7 +102,7 @@ int HostStage::download(void* dst, const void* src, size_t bytes, int device, hi
   for (int t = 1; t < kThreads; ++t) {
     try {
       th[t] = std::thread(run, t);
-    } catch (const std::system_error&) {  // no thread to be had: its stripe here
+    } catch (...) {  // no thread to be had (or no memory to start one): its stripe here
       run(t);
     }
   }

@@ -222,3 +222,21 @@ result(cut=cut, used=used, whole=size * N // 8, code=code)
     assert len(covered(r["cut"], kernel)) == 8
     assert r["used"] == r["whole"]
     assert r["code"] == -2
+
+
+BIG = """
+from test_gpu_heat_lines import line_case
+T0, Om0, P = line_case((128, 128, 129), 0.05, steps=0)
+plan = api.HeatPlan(T0, Om0, P)
+log()
+"""
+
+
+def test_large_downloads_do_without_threads():
+    """A thread that cannot be started, for whatever reason, leaves its stripe to the caller's."""
+    r = fakehip.run(BIG + """
+fake.fake_fail_threads(1)
+plan.download(f64=False)
+result(bytes=sum(int(l.split()[1]) for l in log() if l.startswith("download ")), L=int(T0.size))
+""")
+    assert r["bytes"] >= 8 * r["L"]  # T and Omega
