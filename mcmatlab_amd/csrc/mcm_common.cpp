@@ -109,7 +109,12 @@ int HostStage::download(void* dst, const void* src, size_t bytes, int device, hi
   run(0);
   for (auto& t : th)
     if (t.joinable()) t.join();
-  for (hipError_t e : err) MCM_HIP(e);
+  for (hipError_t e : err)
+    if (e != hipSuccess) {
+      // copies of the other stripes, or this one's other block, may be under way
+      (void)hipStreamSynchronize(s);
+      MCM_HIP(e);
+    }
   return MCM_OK;
 }
 

@@ -240,3 +240,20 @@ plan.download(f64=False)
 result(bytes=sum(int(l.split()[1]) for l in log() if l.startswith("download ")), L=int(T0.size))
 """)
     assert r["bytes"] >= 8 * r["L"]  # T and Omega
+
+
+@pytest.mark.parametrize("nth", [1, 3, 5])
+def test_a_failed_download_leaves_nothing_under_way(nth):
+    """The other stripes' copies into the pinned block have ended before the error
+    is returned: the block is used again, or freed, by what comes next."""
+    r = fakehip.run(BIG + f"""
+fake.fake_fail_downloads({nth})
+try:
+    plan.download(f64=False)
+    code = 0
+except _lib.MCMError as e:
+    code = e.code
+result(code=code, log=log())
+""")
+    assert r["code"] == -3
+    assert r["log"][-1] == "sync stream"
