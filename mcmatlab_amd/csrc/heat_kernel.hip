@@ -1037,7 +1037,10 @@ struct BurnQueue {
 };
 __device__ inline void burn(const HeatArgs<double>& a, const BurnQueue& B, int e, const double* sLogA, const double* sE) {
   const int m = B.m[e], i = B.i[e];
-  a.Om[i] += a.dt * exp(fma(-sE[m], prcp(a.Rgas * B.th[e]), sLogA[m]));
+  const double rt = a.Rgas * B.th[e];
+  double r = prcp(rt);
+  if (!__builtin_isfinite(r)) r = __builtin_amdgcn_rcp(rt);  // 0 and infinities, where the refinement has no value
+  a.Om[i] += a.dt * exp(fma(-sE[m], r, sLogA[m]));
 }
 
 // substeps 2a + 2b (KIND Y) and 3a + 3b with the Arrhenius update and the
