@@ -2153,6 +2153,26 @@ int advance(mcm_heat_plan* P, int64_t steps, double dt, int lightsOn) {
   return MCM_OK;
 }
 
+// The conduction coefficients.  Those of media that never meet along an axis
+// (none do along an axis of one voxel) may have any value, but some kernels read
+// one for a neighbour outside the grid, as a factor of a zero difference: where
+// such a coefficient is infinite or no number it is 0 here.
+std::vector<float> used_coefficients(const mcm_heat_input* in) {
+  const int64_t nM = in->nM, n[3] = {in->nx, in->ny, in->nz}, st[3] = {1, in->nx, in->nx * in->ny}, L = n[0] * n[1] * n[2];
+  std::vector<float> c(in->dTdtperdeltaT, in->dTdtperdeltaT + nM * nM * 3);
+  if (std::all_of(c.begin(), c.end(), [](float v) { return std::isfinite(v); })) return c;
+  std::vector<uint8_t> meet(c.size(), 0);
+  for (int d = 0; d < 3; ++d)
+    for (int64_t i = 0; i < L; ++i) {
+      if (i / st[d] % n[d] == n[d] - 1) continue;
+      const int64_t a = in->M[i], b = in->M[i + st[d]];
+      meet[a + b * nM + d * nM * nM] = meet[b + a * nM + d * nM * nM] = 1;
+    }
+  for (size_t k = 0; k < c.size(); ++k)
+    if (!meet[k] && !std::isfinite(c[k])) c[k] = 0.f;
+  return c;
+}
+
 template <typename RT>
 int upload_state(mcm_heat_plan* P, const mcm_heat_input* in) {
   const int tpb = 256;
@@ -2314,9 +2334,10 @@ int mcm_heat_plan_create(const mcm_heat_input* in, mcm_heat_plan** out) {
   const int nM = P->nM;
   std::vector<double> c64((size_t)nM * nM * 3), la64(nM), e64(nM), w64((size_t)std::max<int64_t>(P->nS, 1) * 3);
   std::vector<float> c32(c64.size()), la32(nM), e32(nM), w32(w64.size());
+  const std::vector<float> coefs = used_coefficients(in);
   for (size_t k = 0; k < c64.size(); ++k) {
-    c64[k] = (double)in->dTdtperdeltaT[k];
-    c32[k] = in->dTdtperdeltaT[k];
+    c64[k] = (double)coefs[k];
+    c32[k] = coefs[k];
   }
   for (int m = 0; m < nM; ++m) {
     la64[m] = std::log(in->A[m]);

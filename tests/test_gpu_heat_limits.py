@@ -34,3 +34,35 @@ def test_damage_at_infinite_and_zero_absolute_temperature(scheme, shape):
         np.testing.assert_allclose(Om64[at], 3 * 0.05 * rate, rtol=1e-14)
         rest[at] = False
     assert np.all(np.isfinite(T64[rest])) and np.all(np.isfinite(Om64[rest])) and np.all(Om64[rest] > 0)
+
+
+@pytest.mark.parametrize("precision,scheme", [("fp64", "dgadi"), ("fp64", "explicit"), ("fp32", "dgadi"), ("fp32", "explicit")])
+@pytest.mark.parametrize("shape", [(70, 1, 9), (1, 20, 9), (9, 20, 1), (1, 1, 33), (66, 7, 6)])
+def test_coefficients_of_pairs_that_never_meet_are_not_used(precision, scheme, shape):
+    """An axis of one voxel has no neighbours, and media laid in layers of one
+    voxel never meet themselves: whatever their coefficients are, 0, infinite or
+    no number, the state is the same."""
+    from mcmatlab_amd import api
+
+    print(f"[heat-limits] {precision} {scheme} {shape}", flush=True)
+    T0, Om0, P = line_case(shape, 0.05, nM=4, steps=6, sinked=0)
+    M = np.zeros(shape, np.uint8)
+    M[:] = (np.arange(shape[2]) % 3)[None, None, :]  # medium 3 nowhere
+    if shape[0] > 2:
+        M[-1] = 0  # more pairs along x and z
+    P["M"] = np.asfortranarray(M)
+    met = np.zeros((4, 4, 3), bool)
+    for d in range(3):
+        lo, hi = (np.moveaxis(M, d, 0)[s].ravel() for s in (slice(None, -1), slice(1, None)))
+        met[lo, hi, d] = met[hi, lo, d] = True
+    assert not met.all()
+    r = []
+    for value in (0.0, np.inf, np.nan):
+        c = np.array(P["dTdtperdeltaT"], copy=True)
+        c[~met] = value
+        T, Om, _, mx = api.finiteElementHeatPropagator(T0, Om0, dict(P, dTdtperdeltaT=c), precision=precision, scheme=scheme)
+        assert np.all(np.isfinite(T)) and np.all(np.isfinite(Om))
+        r.append((T, Om, mx))
+    for other in r[1:]:
+        for a, b in zip(r[0], other):
+            assert np.array_equal(a, b)
