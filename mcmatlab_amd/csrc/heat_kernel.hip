@@ -15,8 +15,8 @@
 // chunks of a line; along x a wavefront holds contiguous voxels, along y and z
 // a workgroup holds 16 neighbouring lines in registers.  FP32 (the reference's
 // arithmetic) and longer lines: one lane per line running the Thomas
-// recurrence over blocks of loaded elements; FP32 lines of up to 420 voxels run
-// it on lines staged in LDS.
+// recurrence over blocks of loaded elements; FP32 lines of up to 431 voxels
+// (line32_lines) run it on lines staged in LDS.
 // The explicit (forward Euler) scheme is one kernel per step.
 //
 // Arithmetic follows the reference's expressions (built without FMA
@@ -330,7 +330,7 @@ __device__ void sweep_line(const HeatArgs<RT>& a, const RT* cT, const HeatLds<RT
 
 constexpr int kSweepU = 8;
 
-// FP32 sweeps of lines of up to 420 voxels.  The reference's recurrence is
+// FP32 sweeps of lines that fit in LDS (line32_lines).  The reference's recurrence is
 // sequential along a line and is kept operation for operation, so its length
 // cannot be cut; what a lane per line loses is the latency of its loads and
 // the few lanes (100^3: 157 wavefronts for 256 CUs).  Here a workgroup takes TL
@@ -340,7 +340,8 @@ constexpr int kSweepU = 8;
 // 100^3: 53 us a step (three sweeps; 390 with a lane per line), of which 30
 // remain without the recurrences.  Rows are read a group ahead of the recurrence
 // (70 us when each group waited for its own reads).
-// TL: as many lines (32, 16, 8) as fit four numbers per voxel into 54 KB.
+// TL: as many lines (32, 16, 8) as fit four numbers per voxel into 54 KB: lines
+// of up to 107, 215 and 431 voxels.
 constexpr int kLine32Floats = 54 * 1024 / 16;
 inline int line32_lines(int n) {
   const int pitch = n | 1;
