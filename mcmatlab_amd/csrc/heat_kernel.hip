@@ -1128,10 +1128,13 @@ __global__ void __launch_bounds__(NC * 16) heat_sweep_yz(HeatArgs<double> a) {
       queued += __popcll(bal);
       if (queued >= 64) {
         queued -= 64;
+        wave_lds_fence();
         burn(a, B, queued + lane, sLogA, sE);
+        wave_lds_fence();
       }
     }
   }
+  wave_lds_fence();
   if (lane < queued) burn(a, B, lane, sLogA, sE);
   fold_lds_max(sMax, a.maxKey, nM);
 }

@@ -100,6 +100,7 @@ struct GradTerms {
 __device__ inline void add_terms(double* grad, const GradTerms& t, int& n) {
   using GlobalDouble = __attribute__((address_space(1))) double;
   const int lane = __lane_id(), base = threadIdx.x & ~63;
+  wave_lds_fence();
 #pragma unroll 2
   for (int r = 0; r < kTerms; ++r) {
     const int src = r * (64 / kTerms) + lane / kTerms, slot = lane % kTerms;
@@ -108,6 +109,7 @@ __device__ inline void add_terms(double* grad, const GradTerms& t, int& n) {
       (void)__builtin_amdgcn_global_atomic_fadd_f64((GlobalDouble*)(grad + t.j[k]), t.v[k]);
     }
   }
+  wave_lds_fence();
   n = 0;
 }
 

@@ -244,6 +244,7 @@ struct DeferSink : DeviceSink {
   __device__ void drain() {
     using GlobalDouble = __attribute__((address_space(1))) double;
     const int lane = __lane_id(), base = threadIdx.x & ~63;
+    wave_lds_fence();
 #pragma unroll 2
     for (int r = 0; r < kRing; ++r) {
       const int src = r * (64 / kRing) + lane / kRing, slot = lane % kRing;
@@ -258,6 +259,7 @@ struct DeferSink : DeviceSink {
         (void)__builtin_amdgcn_global_atomic_fadd_f64((GlobalDouble*)(nfr + d.x), (double)__uint_as_float(d.y));
       }
     }
+    wave_lds_fence();
     nRing = 0;
     parked = 0;
   }

@@ -29,6 +29,16 @@ int fail(int code, const char* fmt, ...);
 int use_device(int device);
 int cu_count(int device);
 
+#ifdef __HIP__
+// Between stores to LDS by some lanes of a wavefront and loads of them by others,
+// and back.  A wavefront's LDS operations execute in their order, so no
+// instruction is needed; it keeps the compiler from moving them.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+#endif
+
 // Downloads of large arrays through pinned memory that a plan keeps (16 MB,
 // allocated by its first large download and freed with it).  The runtime's own
 // copy into pageable memory pins and faults in the pages from one thread:
