@@ -325,6 +325,9 @@ int check_args(const float* paramVals, int64_t n1, int64_t n2, float* downsample
 void row_pass(const float* paramVals, int64_t n1, int r, float* mx, float* mn, float* sum, bool* finite) {
   float hi = paramVals[r], lo = hi, sm = hi;
   bool ok = std::isfinite(hi);
+  // (8e6 sets: 4.1 ms, wherever the loop lies; one set at a time 4.1 or 4.9 by the
+  // address that the linker gives it)
+#pragma clang loop unroll_count(2)
   for (int64_t i = 1; i < n1; ++i) {
     const float v = paramVals[3 * i + r];
     ok = ok && std::isfinite(v);
