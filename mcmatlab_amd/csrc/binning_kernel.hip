@@ -51,12 +51,10 @@ constexpr int kBinTPB = 256;
 // each (8e6 sets: a pass takes 36.0, 24.6 and 24.4 us with 8192, 2048 and 1024).
 constexpr int kBinMaxBlocks = 1024;
 
-// The state between passes: scan index and value of the last selection, and the
-// distance of set 0 after the last pass.
+// The state between passes: value of the last selection, and the distance of set 0
+// after the last pass.
 struct BinState {
-  int m;
   float u, d0;
-  int unused;
 };
 
 struct BinArgs {
@@ -161,7 +159,6 @@ __device__ inline Selection select_set(const BinArgs& a, int j, int nParts) {
     sSel = r;
     if (blockIdx.x == 0) {
       a.picks[j] = r.pick;
-      a.st[j & 1].m = r.m;
       a.st[j & 1].u = u;
     }
   }

@@ -646,7 +646,7 @@ __global__ void __launch_bounds__(kHeatTPB) heat_sweep_z(HeatArgs<RT> a) {
 // Wavefront-parallel tridiagonal solve (FP64 sweeps)
 //
 // A system  a[r] x[r-1] + b[r] x[r] + c[r] x[r+1] = d[r]  of up to W*S rows
-// is spread over a segment of W lanes (W = 64, 32 or 16; a wavefront solves
+// is spread over a segment of W lanes (W = 64 or 32; a wavefront solves
 // 64 / W systems side by side), S consecutive rows per lane (row
 // r = lane * S + s, lane counted within the segment); unused rows are
 // a = c = 0, b = 1, d = 0.  The matrices of the heat step are strictly
@@ -669,34 +669,11 @@ __global__ void __launch_bounds__(kHeatTPB) heat_sweep_z(HeatArgs<RT> a) {
 __device__ inline double lane_shfl(double v, int src) { return __shfl(v, src < 0 ? 0 : (src > 63 ? 63 : src), 64); }
 __device__ inline int lane_shfl(int v, int src) { return __shfl(v, src < 0 ? 0 : (src > 63 ? 63 : src), 64); }
 
-// DPP move within rows of 16 lanes (CTRL 0x100 + h: row_shl:h, lane p gets
-// lane p + h; 0x110 + h: row_shr:h, lane p gets lane p - h; 0 where the
-// source lies outside the row)
-template <int CTRL>
-__device__ inline int dpp_move(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
-template <int CTRL>
-__device__ inline double dpp_move(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = dpp_move<CTRL>((int)b), hi = dpp_move<CTRL>((int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 // v of lane wl + h (UP) or wl - h of the same W-lane segment; a lane whose
 // source lies outside its segment gets an unspecified value, which callers
-// mask.  16-lane segments are the DPP unit's rows, so their shifts are VALU
-// row moves rather than LDS-routed permutes.
+// mask.
 template <int W, bool UP, typename V>
 __device__ inline V seg_shift(V v, int h) {
-  if constexpr (W == 16) {
-    constexpr int base = UP ? 0x100 : 0x110;
-    switch (h) {
-      case 1: return dpp_move<base + 1>(v);
-      case 2: return dpp_move<base + 2>(v);
-      case 4: return dpp_move<base + 4>(v);
-      case 8: return dpp_move<base + 8>(v);
-      default: break;
-    }
-  }
   const int wl = __lane_id();
   return lane_shfl(v, UP ? wl + h : wl - h);
 }
@@ -717,7 +694,7 @@ constexpr double kDecoupled = 0x1p-30;
 template <int S, int W = 64>
 __device__ inline void line_solve(const double (&a)[S], const double (&b)[S], const double (&c)[S], const double (&d)[S], double (&x)[S]) {
   // a line per W-lane segment of the wavefront; lane is the index within it
-  static_assert(W == 16 || W == 32 || W == 64, "segments of 16, 32 or 64 lanes");
+  static_assert(W == 32 || W == 64, "segments of 32 or 64 lanes");
   const int lane = __lane_id() & (W - 1);
   // 1: x[s] = p[s] - q[s] UL - g[s] x[s+1]
   double g[S], p[S], q[S];
@@ -743,10 +720,9 @@ __device__ inline void line_solve(const double (&a)[S], const double (&b)[S], co
     R = -g[s] * R;
   }
   // shuffles run in every lane (a lane reading from a lane that is inactive
-  // at the shuffle gets 0), then lanes without the neighbour are masked; DPP
-  // moves deliver 0 there by themselves
+  // at the shuffle gets 0), then lanes without the neighbour are masked
   double Pn = seg_shift<W, true>(P, 1), Qn = seg_shift<W, true>(Q, 1), Rn = seg_shift<W, true>(R, 1);
-  if (W != 16 && lane == W - 1) Pn = Qn = Rn = 0.0;
+  if (lane == W - 1) Pn = Qn = Rn = 0.0;
   const double e = g[S - 1], ib = prcp(fma(-e, Qn, 1.0));
   double pa = q[S - 1] * ib, pc = e * Rn * ib, pd = fma(-e, Pn, p[S - 1]) * ib;
   // 3: U + pa U(lane - h) + pc U(lane + h) = pd
@@ -754,22 +730,18 @@ __device__ inline void line_solve(const double (&a)[S], const double (&b)[S], co
 #pragma unroll
   for (int h = 1; h < W; h <<= 1) {
     double dm = seg_shift<W, false>(pd, h), dp = seg_shift<W, true>(pd, h);
-    if (W != 16) {
-      dm = lane >= h ? dm : 0.0;
-      dp = lane + h < W ? dp : 0.0;
-    }
+    dm = lane >= h ? dm : 0.0;
+    dp = lane + h < W ? dp : 0.0;
     if (__all(fmax(fabs(pa), fabs(pc)) <= kDecoupled)) {
       pd = fma(-pc, dp, fma(-pa, dm, pd));
       break;
     }
     double am = seg_shift<W, false>(pa, h), cm = seg_shift<W, false>(pc, h);
     double ap = seg_shift<W, true>(pa, h), cp = seg_shift<W, true>(pc, h);
-    if (W != 16) {
-      am = lane >= h ? am : 0.0;
-      cm = lane >= h ? cm : 0.0;
-      ap = lane + h < W ? ap : 0.0;
-      cp = lane + h < W ? cp : 0.0;
-    }
+    am = lane >= h ? am : 0.0;
+    cm = lane >= h ? cm : 0.0;
+    ap = lane + h < W ? ap : 0.0;
+    cp = lane + h < W ? cp : 0.0;
     const double r = prcp(fma(-pc, ap, fma(-pa, cm, 1.0)));
     pd = fma(-pc, dp, fma(-pa, dm, pd)) * r;
     pa = -pa * am * r;
@@ -778,7 +750,7 @@ __device__ inline void line_solve(const double (&a)[S], const double (&b)[S], co
   U = pd;
   // 4
   double UL = seg_shift<W, false>(U, 1);
-  if (W != 16 && lane == 0) UL = 0.0;
+  if (lane == 0) UL = 0.0;
   x[S - 1] = U;
 #pragma unroll
   for (int s = S - 2; s >= 0; --s) x[s] = fma(-g[s], x[s + 1], fma(-q[s], UL, p[s]));
