@@ -197,7 +197,7 @@ int mcm_mc_plan_tallies(mcm_mc_plan *plan, const double **d_deposit, uint64_t *n
  * [0] packets launched alive, [1] collected, [2] voxel sub-steps,
  * [3] scatterings, [4] interface (Fresnel) events, [5] packets retired at the
  * sub-step cap, [6] aborted (1 = a packet failed 10^6 launch attempts),
- * [7] lanes per launch. */
+ * [7] lanes of a launch that fills the device (few packets take fewer). */
 int mcm_mc_plan_counters(mcm_mc_plan *plan, double counters[8]);
 int mcm_mc_plan_destroy(mcm_mc_plan *plan);
 /* Launch tuning (no reference counterpart).  The fluence accumulates into 1,

@@ -32,7 +32,7 @@
 //
 // 10^6 packets on 128^3 (pass 1 alone 5.7 ms): 16.6 ms with one
 // term per lane added when a packet leaves a voxel, 11.0 ms with the terms
-// parked (GradTerms) and a copy of the gradient per XCD (10^7: 0.185 and 0.134 s).
+// parked (GradTerms) and a copy of the gradient per XCD (10^7: 0.185 and 0.107 to 0.160 s).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
