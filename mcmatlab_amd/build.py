@@ -104,7 +104,7 @@ def build_test_harnesses(verbose=True):
     # the HIP runtime's stand-in for tests of the host code
     fake = os.path.join(ROOT, "tests", "fake_hip", "fake_hip.cpp")
     if os.path.exists(fake):
-        _run(["g++", "-O1", "-fPIC", "-shared", "-std=c++17", "-Wall", "-I", "/opt/rocm/include", fake, "-o",
+        _run(["g++", "-O1", "-fPIC", "-shared", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include", fake, "-o",
               os.path.join(out, "libfake_hip.so"), "-ldl"])
         if verbose:
             print("  built tests/_build/libfake_hip.so")

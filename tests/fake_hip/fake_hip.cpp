@@ -3,9 +3,6 @@
 // tests see what the host code allocates, launches and waits for, and can limit
 // the device's memory or let a call fail.  Device memory is host memory (zeros);
 // every event is a line of a log.
-#ifndef __HIP_PLATFORM_AMD__
-#define __HIP_PLATFORM_AMD__
-#endif
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 
